@@ -24,6 +24,7 @@
 #include "ifs_engine.h"
 #include "ifs_fmm.h"
 #include "ifs_internal.h"
+#include "ifs_pair.h"
 
 using namespace ifs;
 
@@ -414,7 +415,7 @@ int class_batch_finalize(ifs_ctx *c, ClassBatch &B) {
 // Chunks, runs, segments and reduction lists for nrhs right-hand sides per call.
 // Gauss-Legendre nodes and weights on [-1, 1] by Newton's iteration on P_Q in long
 // double (Golub-Welsch would do as well; Q <= a few thousand here).
-static void gauss_legendre(int Q, std::vector<double> &x, std::vector<double> &w) {
+void gauss_legendre(int Q, std::vector<double> &x, std::vector<double> &w) {
     x.assign(Q, 0.0);
     w.assign(Q, 0.0);
     const long double pi = 3.14159265358979323846264338327950288L;
@@ -1108,9 +1109,15 @@ static int create_impl(ifs_ctx **out, const ifs_cluster *cl, const ifs_params *p
                     make_task(dv, p->k, p->z_selector, c->Leff[l], c->Leff[j], c->off[l], c->off[j]));
             }
         }
-        if ((rc = batch_finalize(c, B, std::min<size_t>(c->ws_budget, (size_t)8 << 30), true)) != IFS_OK)
-            return fail(rc);
         batch_cost(B, c->flops_mv, c->bytes_mv);
+        if (pair_takes(B.tasks)) {
+            c->pair = new (std::nothrow) PairBatch();
+            if (!c->pair) return fail(IFS_E_NOMEM);
+            rc = pair_finalize(c, *c->pair, B.tasks, "direct");
+        } else {
+            rc = batch_finalize(c, B, std::min<size_t>(c->ws_budget, (size_t)8 << 30), true);
+        }
+        if (rc != IFS_OK) return fail(rc);
     } else {
         if ((rc = fmm::build(c, &c->fmm)) != IFS_OK) return fail(rc);
     }
@@ -1126,6 +1133,7 @@ int ifs_destroy(ifs_ctx *c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     graphs_clear(c);
     if (c->fmm) fmm::destroy(c->fmm);
+    delete c->pair;
     if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
     delete c;
     return IFS_OK;
@@ -1172,6 +1180,8 @@ int matvec_impl(ifs_ctx *c, const double2 *x, double2 *b, int normalised, int nr
     }
     if (c->fmm) {
         rc = fmm::run(c, c->fmm, c->d_xh.as<double2>(), c->d_acc.as<double2>(), nrhs, nc, prec);
+    } else if (c->pair) {
+        rc = pair_run(c, *c->pair, c->d_xh.as<double2>(), c->d_acc.as<double2>(), nrhs, nc, nc);
     } else {
         rc = batch_run(c, c->direct, c->d_xh.as<double2>(), c->d_acc.as<double2>(), nrhs, nc, nc);
     }
@@ -1194,6 +1204,7 @@ static uint64_t matvec_sig(ifs_ctx *c) {
                             &c->direct.own_ax, &c->direct.own_y, &c->direct.own_z, &c->d_snm, &c->d_an, &c->d_bn})
         mix((uint64_t)(uintptr_t)d->p);
     for (auto &kv : c->gq_nodes) mix((uint64_t)(uintptr_t)kv.second.p);
+    if (c->pair) mix(pair_sig(*c->pair));
     if (c->fmm) mix(fmm::buffers_sig(c->fmm));
     return h;
 }

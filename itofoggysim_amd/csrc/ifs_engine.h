@@ -15,6 +15,7 @@ namespace ifs {
 namespace fmm {
 struct Fmm;
 }
+struct PairBatch;
 struct DevBuf {
     void *p = nullptr;
     size_t bytes = 0;
@@ -147,7 +148,8 @@ struct ifs_ctx {
     size_t cache_budget = 0;        // tables kept across matvecs
     size_t ws_cached = 0;           // bytes held by cached batches
 
-    ifs::Batch direct;              // sphere -> sphere (direct all pairs)
+    ifs::Batch direct;              // sphere -> sphere (direct all pairs) where the pair kernels do not apply
+    ifs::PairBatch *pair = nullptr; // sphere -> sphere (direct all pairs)
     ifs::fmm::Fmm *fmm = nullptr;
 
     // Krylov workspace
@@ -238,6 +240,8 @@ int matvec_graph(ifs_ctx *c, const double2 *x, double2 *b, int normalised, int n
                  int prec = 0);
 void graphs_clear(ifs_ctx *c);
 int class_batch_finalize(ifs_ctx *c, ClassBatch &B);
+// Gauss-Legendre nodes and weights on [-1, 1] (host).
+void gauss_legendre(int Q, std::vector<double> &x, std::vector<double> &w);
 // Device Gauss-Legendre rule of Q nodes (cached per context): mu, then w.
 int gq_rule(ifs_ctx *c, int Q, const double **mu, const double **w);
 int class_batch_plan(ifs_ctx *c, ClassBatch &B, int nrhs);

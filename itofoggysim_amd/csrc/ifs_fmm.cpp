@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "ifs_engine.h"
+#include "ifs_pair.h"
 #include "ifs_tree.h"
 
 namespace ifs {
@@ -48,6 +49,7 @@ struct Fmm {
     DevBuf C, D;                                // multipole / local pools
     int64_t nC = 0;
     Batch p2m, l2p, p2p;
+    PairBatch pair;                             // near field, unless the pair kernels do not apply (p2p)
     std::vector<ClassBatch> m2m, m2l, l2l;      // indexed by level
     int64_t counts[6] = {0, 0, 0, 0, 0, 0};
 };
@@ -313,7 +315,12 @@ int build(ifs_ctx *c, Fmm **out) {
     }
     if ((rc = fin(f->p2m, "p2m"))) goto fail;
     if ((rc = fin(f->l2p, "l2p"))) goto fail;
-    if ((rc = fin(f->p2p, "p2p"))) goto fail;
+    if (pair_takes(f->p2p.tasks)) {
+        batch_cost(f->p2p, c->flops_mv, c->bytes_mv);
+        if ((rc = pair_finalize(c, f->pair, f->p2p.tasks, "p2p"))) goto fail;
+    } else if ((rc = fin(f->p2p, "p2p"))) {
+        goto fail;
+    }
     *out = f;
     return IFS_OK;
 fail:
@@ -339,6 +346,7 @@ int run(ifs_ctx *c, Fmm *f, const double2 *xh, double2 *acc, int nrhs, int64_t l
         if (l > f->l_min && (rc = class_batch_run(c, f->l2l[l], D, D, nrhs, prec))) return rc;
     }
     if ((rc = batch_run(c, f->l2p, D, acc, nrhs, st, ld))) return rc;
+    if (f->pair.active()) return pair_run(c, f->pair, xh, acc, nrhs, ld, ld);
     if ((rc = batch_run(c, f->p2p, xh, acc, nrhs, ld, ld))) return rc;
     return IFS_OK;
 }
@@ -352,6 +360,7 @@ uint64_t buffers_sig(Fmm *f) {
     for (const Batch *B : {&f->p2m, &f->l2p, &f->p2p})
         for (const DevBuf *d : {&B->d_tasks, &B->d_segs, &B->own_d, &B->own_s, &B->own_ax, &B->own_y, &B->own_z})
             buf(*d);
+    mix(pair_sig(f->pair));
     for (const auto *v : {&f->m2m, &f->m2l, &f->l2l})
         for (const ClassBatch &B : *v) {
             mix((uint64_t)B.plan_nrhs);

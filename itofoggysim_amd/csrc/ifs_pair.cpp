@@ -1,0 +1,335 @@
+// Plan and launch order of the sphere-pair translations (kernels: ifs_pair.hip).
+#include "ifs_pair.h"
+
+#include <algorithm>
+#include <cmath>
+#include <map>
+
+namespace ifs {
+
+namespace {
+
+// Chunk of rotated and shifted columns held at once.
+constexpr size_t kPairChunk = (size_t)1 << 30;
+
+// Largest growth of |h1_p(t)| up to the last order P = Ls + Lt that the quadrature may
+// carry: |h1_P| / |h1_0| follows exp(2/3 z^{3/2}) in z = (P - t) / (t/2)^{1/3}; at z = 2.5
+// it is 16 to 27 for every P from 3 to 126 (evaluated), so the quadrature rounds within
+// a few 1e-15 of the largest entry.  Closer pairs take tables from the degree recurrence.
+bool is_close(const Task &T) {
+    const double P = (double)(T.Ls + T.Lt);
+    return P - T.t > 2.5 * std::cbrt(0.5 * T.t);
+}
+
+// Doubles of one node set's two operand-ordered matrices.
+size_t quad_size(int L, int Q) {
+    const size_t QT = Q / 16, S1 = (L + 3) / 4, UT = (L + 15) / 16;
+    return (size_t)(L + 1) * 2 * QT * 64 * (S1 + 4 * UT);
+}
+
+int upload(DevBuf &d, const void *h, size_t bytes) {
+    int rc = d.alloc(std::max<size_t>(bytes, 16));
+    if (rc) return rc;
+    if (bytes && hipMemcpy(d.p, h, bytes, hipMemcpyHostToDevice) != hipSuccess) return IFS_E_HIP;
+    return IFS_OK;
+}
+
+// Tiles of at most four translations of one target (sources by order, close pairs apart).
+void build_tiles(PairBatch &B, std::map<int, int64_t> &quads) {
+    std::vector<Task> far, close;
+    for (size_t i = 0; i < B.tasks.size();) {
+        size_t j = i;
+        far.clear();
+        close.clear();
+        for (; j < B.tasks.size() && B.tasks[j].dst == B.tasks[i].dst; ++j)
+            (is_close(B.tasks[j]) ? close : far).push_back(B.tasks[j]);
+        for (auto *v : {&far, &close}) {
+            std::stable_sort(v->begin(), v->end(), [](const Task &a, const Task &b) { return a.Ls < b.Ls; });
+            for (size_t a = 0; a < v->size(); a += 4) {
+                const size_t n = std::min<size_t>(4, v->size() - a);
+                PairTile T{};
+                T.Ls = (*v)[a + n - 1].Ls;
+                T.Lt = (*v)[a].Lt;
+                T.K = std::min(T.Ls, T.Lt);
+                T.NL = std::max(T.Ls, T.Lt);
+                T.Q = v == &far ? (T.Ls + T.Lt + 1 + 15) / 16 * 16 : 0;
+                T.tabw = 2 * (T.NL + 1) + T.Q;
+                if (T.Q) quads[T.Q] = 0;
+                for (size_t s = 0; s < 4; ++s) {
+                    const Task &K = (*v)[a + std::min(s, n - 1)];
+                    PairSlot S{};
+                    S.src = s < n ? K.src : -1;
+                    S.t = K.t;
+                    S.cth = K.cth;
+                    S.phi = K.phi;
+                    S.Ls = K.Ls;
+                    S.K = K.K;
+                    B.slots.push_back(S);
+                }
+                B.tiles.push_back(T);
+            }
+        }
+        i = j;
+    }
+}
+
+// Chunks, segments and per-chunk target lists; workspace offsets.
+int pair_plan(ifs_ctx *c, PairBatch &B, int nrhs) {
+    B.chunks.clear();
+    B.segs.clear();
+    B.targets.clear();
+    B.close.clear();
+    const size_t budget = std::max<size_t>(std::min(c->ws_budget, kPairChunk), 1);
+    // first tile of every target
+    std::vector<size_t> first;
+    std::vector<int64_t> dst;
+    {
+        size_t tile = 0;
+        for (size_t i = 0; i < B.tasks.size();) {
+            size_t j = i, nf = 0, nc = 0;
+            for (; j < B.tasks.size() && B.tasks[j].dst == B.tasks[i].dst; ++j) ++(is_close(B.tasks[j]) ? nc : nf);
+            first.push_back(tile);
+            dst.push_back(B.tasks[i].dst);
+            tile += (nf + 3) / 4 + (nc + 3) / 4;
+            i = j;
+        }
+        first.push_back(tile);
+    }
+    PairBatch::Chunk cur;
+    size_t used = 0;
+    int64_t tab = 0, ax = 0;  // running table offsets when the tables are kept
+    auto close_chunk = [&]() {
+        cur.t1 = (int)(B.segs.empty() ? 0 : B.segs.back().t_end);
+        cur.s1 = (int)B.segs.size();
+        cur.g1 = (int)B.targets.size();
+        cur.c1 = (int)B.close.size();
+        B.chunks.push_back(cur);
+        PairBatch::Chunk n;
+        n.t0 = cur.t1;
+        n.s0 = cur.s1;
+        n.g0 = cur.g1;
+        n.c0 = cur.c1;
+        cur = n;
+        used = 0;
+    };
+    for (size_t g = 0; g + 1 < first.size(); ++g) {
+        const int nt = (int)(first[g + 1] - first[g]);
+        // tiles one wave sums: eight partial sums per target at most eight tiles long.  A
+        // target's sum then does not depend on what else the plan holds.
+        const int G = std::min(8, (nt + 7) / 8);
+        bool open = false;
+        for (size_t a = first[g]; a < first[g + 1]; a += G) {
+            const size_t b = std::min(first[g + 1], a + G);
+            size_t bytes = 0;
+            for (size_t t = a; t < b; ++t) {
+                const PairTile &T = B.tiles[t];
+                bytes += 128 * (size_t)(rows_size(T.Ls, T.K) + rows_size(T.Lt, T.K)) * nrhs;
+                if (!B.kept) {
+                    bytes += 64 * (size_t)T.tabw;
+                    for (int s = 0; s < 4 && T.Q == 0; ++s)
+                        bytes += 16 * (size_t)(ax_size(T.Lt, B.slots[4 * t + s].Ls, B.slots[4 * t + s].K) +
+                                               sect_size(B.slots[4 * t + s].K, T.Lt + B.slots[4 * t + s].Ls + 2));
+                }
+            }
+            bytes += 32 * (size_t)B.tiles[a].Lt * (B.tiles[a].Lt + 2) * nrhs;
+            if (used && used + bytes > budget) {
+                close_chunk();
+                open = false;
+            }
+            used += bytes;
+            const int Lt = B.tiles[a].Lt;
+            if (!open) {
+                B.targets.push_back({dst[g], Lt, (int)B.segs.size(), 0, 0});
+                open = true;
+            }
+            B.segs.push_back({cur.n_w, Lt, (int)a, (int)b, 0});
+            B.targets.back().s_end = (int)B.segs.size();
+            cur.n_w += 2LL * Lt * (Lt + 2);
+            for (size_t t = a; t < b; ++t) {
+                PairTile &T = B.tiles[t];
+                T.off_y = cur.n_y;
+                T.off_z = cur.n_z;
+                cur.n_y += 16 * rows_size(T.Ls, T.K);
+                cur.n_z += 16 * rows_size(T.Lt, T.K);
+                int64_t &nt_ = B.kept ? tab : cur.n_tab, &na_ = B.kept ? ax : cur.n_ax;
+                T.off_tab = nt_;
+                nt_ += 4LL * T.tabw;
+                cur.max_Ls = std::max(cur.max_Ls, T.Ls);
+                cur.max_Lt = std::max(cur.max_Lt, T.Lt);
+                cur.max_K = std::max(cur.max_K, T.K);
+                cur.max_P = std::max(cur.max_P, T.Ls + T.Lt);
+                for (int s = 0; s < 4; ++s) {
+                    PairSlot &S = B.slots[4 * t + s];
+                    if (S.src < 0) continue;
+                    for (int n = 1; n <= S.Ls; ++n) {
+                        const double kk = std::min(n, S.K);
+                        cur.f_fwd += 8.0 * ((kk + 1.0) * (n + 1.0) + kk * n);
+                    }
+                    for (int n = 1; n <= T.Lt; ++n) {
+                        const double kk = std::min(n, S.K);
+                        cur.f_back += 8.0 * ((kk + 1.0) * (n + 1.0) + kk * n);
+                    }
+                    cur.f_ax += 16.0 * (double)ax_size(T.Lt, S.Ls, S.K) / 2.0;
+                    if (T.Q) continue;
+                    Task K{};
+                    K.t = S.t;
+                    K.Ls = S.Ls;
+                    K.Lt = T.Lt;
+                    K.K = S.K;
+                    K.kind = IFS_ZSEL_HANKEL1;
+                    S.off_ax = K.off_ax = na_;
+                    K.off_s = cur.n_s;
+                    na_ += ax_size(T.Lt, S.Ls, S.K);
+                    cur.n_s += sect_size(S.K, T.Lt + S.Ls + 2);
+                    cur.maxK_close = std::max(cur.maxK_close, S.K);
+                    cur.max_nmax = std::max(cur.max_nmax, T.Lt + S.Ls + 2);
+                    B.close.push_back(K);
+                }
+            }
+        }
+    }
+    if (cur.t0 < (int)B.tiles.size()) close_chunk();
+    int64_t my = 0, mz = 0, mw = 0, mt = 0, ma = 0, ms = 0;
+    for (auto &ch : B.chunks) {
+        my = std::max(my, ch.n_y);
+        mz = std::max(mz, ch.n_z);
+        mw = std::max(mw, ch.n_w);
+        mt = std::max(mt, ch.n_tab);
+        ma = std::max(ma, ch.n_ax);
+        ms = std::max(ms, ch.n_s);
+    }
+    int rc;
+    auto grow = [](DevBuf &d, size_t b) { return d.alloc(std::max(d.bytes, std::max<size_t>(b, 16))); };
+    if ((rc = grow(c->ws_y, 8 * (size_t)my * nrhs)) || (rc = grow(c->ws_z, 8 * (size_t)mz * nrhs)) ||
+        (rc = grow(c->ws_s, 16 * std::max<size_t>((size_t)mw * nrhs, (size_t)ms))))
+        return rc;
+    if (!B.kept && ((rc = grow(c->ws_d, 16 * (size_t)mt)) || (rc = grow(c->ws_ax, 16 * (size_t)ma)))) return rc;
+    if ((rc = upload(B.d_tiles, B.tiles.data(), sizeof(PairTile) * B.tiles.size())) ||
+        (rc = upload(B.d_slots, B.slots.data(), sizeof(PairSlot) * B.slots.size())) ||
+        (rc = upload(B.d_segs, B.segs.data(), sizeof(PairSeg) * B.segs.size())) ||
+        (rc = upload(B.d_targets, B.targets.data(), sizeof(PairTarget) * B.targets.size())) ||
+        (rc = upload(B.d_close, B.close.data(), sizeof(Task) * B.close.size())))
+        return rc;
+    B.plan_nrhs = nrhs;
+    return IFS_OK;
+}
+
+}  // namespace
+
+bool pair_takes(const std::vector<Task> &tasks) {
+    for (auto &T : tasks)
+        if (T.kind != IFS_ZSEL_HANKEL1 || T.Ls > kPairMaxL || T.Lt > kPairMaxL || !(T.t > 0.0)) return false;
+    return !tasks.empty();
+}
+
+int pair_finalize(ifs_ctx *c, PairBatch &B, std::vector<Task> &tasks, const char *name) {
+    static const char *p2p[4] = {"p2p_gen_tables", "p2p_rot_fwd", "p2p_axial", "p2p_rot_back"};
+    if (std::string(name) == "p2p")
+        for (int i = 0; i < 4; ++i) B.pn[i] = p2p[i];
+    B.tasks.swap(tasks);
+    for (auto &T : B.tasks) B.NL = std::max(B.NL, std::max(T.Ls, T.Lt));
+    std::map<int, int64_t> quads;
+    build_tiles(B, quads);
+    // nodes and weights of every set first, then the matrices
+    std::map<int, int64_t> at;
+    std::vector<double> nodes, mu, w;
+    for (auto &q : quads) {
+        at[q.first] = (int64_t)nodes.size();
+        gauss_legendre(q.first, mu, w);
+        nodes.insert(nodes.end(), mu.begin(), mu.end());
+        nodes.insert(nodes.end(), w.begin(), w.end());
+    }
+    int64_t nq = (int64_t)nodes.size();
+    for (auto &q : quads) {
+        q.second = nq;
+        nq += (int64_t)quad_size(B.NL, q.first);
+    }
+    int64_t tab = 0, ax = 0;
+    for (size_t t = 0; t < B.tiles.size(); ++t) {
+        PairTile &T = B.tiles[t];
+        if (T.Q) {
+            T.off_q = quads[T.Q];
+            T.off_mu = at[T.Q];
+        }
+        tab += 4LL * T.tabw;
+        for (int s = 0; s < 4 && !T.Q; ++s)
+            if (B.slots[4 * t + s].src >= 0) ax += ax_size(T.Lt, B.slots[4 * t + s].Ls, B.slots[4 * t + s].K);
+    }
+    int rc;
+    const size_t nd = (size_t)pair_delta_off_host(B.NL + 1);
+    if ((rc = B.d_quad.alloc(8 * (size_t)std::max<int64_t>(nq, 2))) || (rc = B.d_delta.alloc(8 * nd))) return rc;
+    if (!nodes.empty() && hipMemcpy(B.d_quad.p, nodes.data(), 8 * nodes.size(), hipMemcpyHostToDevice) != hipSuccess)
+        return IFS_E_HIP;
+    launch_pair_delta(B.NL, B.d_delta.as<double>(), nd, c->stream);
+    for (auto &q : quads)
+        launch_pair_quad(B.NL, q.first, B.d_quad.as<double>() + at[q.first], B.d_quad.as<double>() + q.second,
+                         quad_size(B.NL, q.first), c->stream);
+    if (hipPeekAtLastError() != hipSuccess) return IFS_E_HIP;
+    const size_t need = 16 * (size_t)(tab + ax);
+    B.kept = need + c->ws_cached <= c->cache_budget;
+    if (B.kept) {
+        if ((rc = B.own_tab.alloc(16 * (size_t)tab)) || (rc = B.own_ax.alloc(16 * (size_t)std::max<int64_t>(ax, 1))))
+            return rc;
+        c->ws_cached += need;
+    }
+    return pair_plan(c, B, 1);
+}
+
+int pair_run(ifs_ctx *c, PairBatch &B, const double2 *src_pool, double2 *dst_pool, int nrhs, int64_t src_stride,
+             int64_t dst_stride) {
+    if (B.plan_nrhs != nrhs) {
+        if (hipStreamSynchronize(c->stream) != hipSuccess) return IFS_E_HIP;
+        int rc = pair_plan(c, B, nrhs);
+        if (rc) return rc;
+    }
+    const PairTile *tiles = B.d_tiles.as<PairTile>();
+    const PairSlot *slots = B.d_slots.as<PairSlot>();
+    const PairSeg *segs = B.d_segs.as<PairSeg>();
+    const double *quad = B.d_quad.as<double>(), *delta = B.d_delta.as<double>();
+    double2 *tab = B.kept ? B.own_tab.as<double2>() : c->ws_d.as<double2>();
+    double2 *wax = B.kept ? B.own_ax.as<double2>() : c->ws_ax.as<double2>();
+    double *Y = c->ws_y.as<double>(), *Z = c->ws_z.as<double>();
+    double2 *W = c->ws_s.as<double2>();
+    for (auto &ch : B.chunks) {
+        const int nt = ch.t1 - ch.t0;
+        if (!(B.kept && B.ready)) {
+            Scope s(c, B.pn[0]);
+            launch_pair_tables(tiles, slots, ch.t0, nt, ch.max_P, quad, tab, c->stream);
+            if (ch.c1 > ch.c0) {
+                const Task *tk = B.d_close.as<Task>() + ch.c0;
+                launch_gen_sect(tk, ch.c1 - ch.c0, ch.max_nmax, c->ws_s.as<double2>(), c->stream);
+                launch_gen_axial(tk, ch.c1 - ch.c0, ch.maxK_close, ch.max_nmax, c->ws_s.as<double2>(), wax, c->stream);
+            }
+        }
+        {
+            Scope s(c, B.pn[1], ch.f_fwd * nrhs);
+            launch_pair_fwd(tiles, slots, ch.t0, nt, ch.max_Ls, delta, tab, src_pool, src_stride, Y, ch.n_y, nrhs,
+                            c->stream);
+        }
+        {
+            Scope s(c, B.pn[2], ch.f_ax * nrhs);
+            launch_pair_axial(tiles, slots, ch.t0, nt, ch.max_K, ch.max_Lt, B.NL, quad, tab, wax, Y, ch.n_y, Z,
+                              ch.n_z, nrhs, c->stream);
+        }
+        {
+            Scope s(c, B.pn[3], ch.f_back * nrhs);
+            launch_pair_back(tiles, segs, ch.s0, ch.s1 - ch.s0, ch.max_Lt, delta, tab, Z, ch.n_z, W, ch.n_w, nrhs,
+                             c->stream);
+            launch_pair_reduce(B.d_targets.as<PairTarget>(), segs, ch.g0, ch.g1 - ch.g0, ch.max_Lt, W, ch.n_w,
+                               dst_pool, dst_stride, nrhs, c->stream);
+        }
+    }
+    if (hipPeekAtLastError() != hipSuccess) return IFS_E_HIP;
+    if (B.kept) B.ready = true;
+    return IFS_OK;
+}
+
+uint64_t pair_sig(const PairBatch &B) {
+    uint64_t h = (uint64_t)B.plan_nrhs;
+    for (const DevBuf *d : {&B.d_tiles, &B.d_slots, &B.d_segs, &B.d_targets, &B.d_close, &B.d_delta, &B.d_quad,
+                            &B.own_tab, &B.own_ax})
+        h ^= (uint64_t)(uintptr_t)d->p + 0x9e3779b97f4a7c15ull + (h << 6) + (h >> 2);
+    return h;
+}
+
+}  // namespace ifs
