@@ -336,16 +336,19 @@ int batch_run(ifs_ctx *c, Batch &B, const double2 *src_pool, double2 *dst_pool, 
 
 // Per-column algorithmic flops of the three products (folded rotations, decoupled
 // coaxial shift): forward rotation, coaxial shift, back rotation.
-static void class_col_flops(const Task &T, double &ffwd, double &fax, double &fback) {
+static void class_col_flops(const Task &T, int n0, double &ffwd, double &fax, double &fback) {
     ffwd = fax = fback = 0.0;
     // folded rotation: E (kk+1)x(n+1) and O kk x n (its zero row and column excluded)
     auto rot = [&](int n) {
         double kk = std::min(n, T.K);
         return 8.0 * ((kk + 1.0) * (n + 1.0) + kk * n);
     };
-    for (int n = 1; n <= T.Ls; ++n) ffwd += rot(n);
-    for (int n = 1; n <= T.Lt; ++n) fback += rot(n);
-    for (int k = -T.K; k <= T.K; ++k) fax += 16.0 * (double)ax_block(k, T.Lt, T.Ls);
+    for (int n = n0; n <= T.Ls; ++n) ffwd += rot(n);
+    for (int n = n0; n <= T.Lt; ++n) fback += rot(n);
+    if (n0 > 1)
+        fax = 8.0 * (double)ax0_size(T.Lt, n0);
+    else
+        for (int k = -T.K; k <= T.K; ++k) fax += 16.0 * (double)ax_block(k, T.Lt, T.Ls);
 }
 
 static bool same_d(const Task &a, const Task &b) { return a.cth == b.cth && a.Ls == b.Ls && a.Lt == b.Lt && a.K == b.K; }
@@ -465,7 +468,7 @@ static int class_batch_keys(ifs_ctx *c, ClassBatch &B) {
     const Task &T0 = B.gen[0];
     B.n_d = fold_size(std::max(T0.Ls, T0.Lt), T0.K);
     B.n_s = sect_size(T0.K, T0.Lt + T0.Ls + 2);
-    B.n_ax = ax_size(T0.Lt, T0.Ls, T0.K);
+    B.n_ax = B.n0 > 1 ? ax0_size(T0.Lt, B.n0) : ax_size(T0.Lt, T0.Ls, T0.K);
     // table keys (Ls, Lt, K are common to the batch)
     {
         std::map<double, int> dk;
@@ -497,7 +500,8 @@ static int class_batch_keys(ifs_ctx *c, ClassBatch &B) {
     B.gq.clear();
     for (int g : B.axkey_cls) {
         const Task &T = B.gen[g];
-        B.gq.push_back(gq_plan(T.kind, T.t, T0.Lt, T0.Ls, T0.K, (size_t)1 << 30));
+        B.gq.push_back(B.n0 > 1 ? gq_plan_rem(T.t, T0.Lt, B.n0 + T0.Lt, (size_t)1 << 30)
+                                : gq_plan(T.kind, T.t, T0.Lt, T0.Ls, T0.K, (size_t)1 << 30));
         const double *mu, *w;
         int r = gq_rule(c, B.gq.back().Q, &mu, &w);
         if (r) return r;
@@ -553,8 +557,9 @@ int class_batch_plan(ifs_ctx *c, ClassBatch &B, int nrhs) {
     if (B.gen.empty()) return IFS_OK;
     const Task &T0 = B.gen[0];
     // chunk capacity from the workspace budget (Y/W and Z per column and RHS)
-    const int64_t ycol = 4 * std::max<int64_t>(rows_size(T0.Ls, T0.K), (int64_t)T0.Lt * (T0.Lt + 2));
-    const int64_t zcol = 4 * rows_size(T0.Lt, T0.K);
+    const int64_t rb = rows_off(B.n0, T0.K), e0 = (int64_t)B.n0 * B.n0 - 1;
+    const int64_t ycol = 4 * std::max<int64_t>(rows_size(T0.Ls, T0.K) - rb, (int64_t)T0.Lt * (T0.Lt + 2) - e0);
+    const int64_t zcol = 4 * (rows_size(T0.Lt, T0.K) - rb);
     const int64_t per_col = 8 * (ycol + zcol) * nrhs;
     const int64_t total = (int64_t)B.src.size();
     int64_t cap = std::max<int64_t>(1, (int64_t)(c->ws_budget / (size_t)per_col));
@@ -563,7 +568,6 @@ int class_batch_plan(ifs_ctx *c, ClassBatch &B, int nrhs) {
     cap = std::min<int64_t>(cap, std::max<int64_t>(1, (int64_t)INT32_MAX / (4LL * nrhs * (2LL * T0.K + 2))));
     B.n_y = B.n_z = 0;
     // walk the class columns, cutting chunks of at most cap columns
-    const int64_t nbox = 2LL * T0.Lt * (T0.Lt + 2);
     int cls = 0;
     int64_t done_in_cls = 0;
     for (int64_t c0 = 0; c0 < total; c0 += cap) {
@@ -592,6 +596,7 @@ int class_batch_plan(ifs_ctx *c, ClassBatch &B, int nrhs) {
             d.Ls = T0.Ls;
             d.Lt = T0.Lt;
             d.K = T0.K;
+            d.n0 = B.n0;
             d.ncols = e - b;
             d.col_begin = b;
             d.ycol0 = b - (int)c0;
@@ -652,7 +657,6 @@ int class_batch_plan(ifs_ctx *c, ClassBatch &B, int nrhs) {
         B.n_y = std::max<int64_t>(B.n_y, ycol * ch.ncols * nrhs);
         B.n_z = std::max<int64_t>(B.n_z, zcol * ch.ncols * nrhs);
     }
-    (void)nbox;
     const int L = std::max(T0.Ls, T0.Lt);
     B.n_d = fold_size(L, T0.K);
     int rc;
@@ -708,10 +712,10 @@ int class_batch_plan(ifs_ctx *c, ClassBatch &B, int nrhs) {
     return IFS_OK;
 }
 
-// Rotation block heights chosen by timing, per (Ls, Lt, K, precision, right-hand sides,
-// log2 of the translation count), shared by every context of the process.
+// Rotation block heights chosen by timing, per (Ls, Lt, K, lowest degree, precision,
+// right-hand sides, log2 of the translation count), shared by every context of the process.
 static std::mutex g_rows_mu;
-static std::map<std::array<int, 6>, std::array<int, 2>> g_rows;
+static std::map<std::array<int, 7>, std::array<int, 2>> g_rows;
 static int ilog2(int64_t v) {
     int r = 0;
     while (v > 1) {
@@ -720,12 +724,12 @@ static int ilog2(int64_t v) {
     }
     return r;
 }
-static int tuned_rows(const std::array<int, 6> &k, int st) {
+static int tuned_rows(const std::array<int, 7> &k, int st) {
     std::lock_guard<std::mutex> lk(g_rows_mu);
     auto it = g_rows.find(k);
     return it == g_rows.end() ? 0 : it->second[st];
 }
-static void remember_rows(const std::array<int, 6> &k, int st, int r) {
+static void remember_rows(const std::array<int, 7> &k, int st, int r) {
     std::lock_guard<std::mutex> lk(g_rows_mu);
     g_rows[k][st] = r;
 }
@@ -749,9 +753,8 @@ int class_batch_run(ifs_ctx *c, ClassBatch &B, const double2 *src_pool, double2 
     double *wz = c->ws_z.as<double>();
     const Task &T0 = B.gen[0];
     double ffwd, fax, fback;
-    class_col_flops(T0, ffwd, fax, fback);
+    class_col_flops(T0, B.n0, ffwd, fax, fback);
     const int L = std::max(T0.Ls, T0.Lt);
-    const int64_t nbox = 2LL * T0.Lt * (T0.Lt + 2);
     // the FP32 products take Wigner tables regenerated per matvec in FP32 (half the bytes to
     // store and to read); tables kept across matvecs stay FP64 and are converted at the load
     const int ftab = prec == 1 && !B.d_persist ? 1 : 0;
@@ -803,7 +806,7 @@ int class_batch_run(ifs_ctx *c, ClassBatch &B, const double2 *src_pool, double2 
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     (void)hipStreamIsCapturing(c->stream, &cap);
     const bool can_tune = c->autotune && !c->prof.on && cap == hipStreamCaptureStatusNone;
-    const std::array<int, 6> tkey = {T0.Ls, T0.Lt, T0.K, prec, nrhs, ilog2((int64_t)B.src.size())};
+    const std::array<int, 7> tkey = {T0.Ls, T0.Lt, T0.K, B.n0, prec, nrhs, ilog2((int64_t)B.src.size())};
     for (int st = 0; st < 2; ++st) {
         int r = c->force_rows[st] ? c->force_rows[st] : B.rot_rows[prec & 1][st];
         if (!r) r = tuned_rows(tkey, st);
@@ -854,7 +857,7 @@ int class_batch_run(ifs_ctx *c, ClassBatch &B, const double2 *src_pool, double2 
         {
             Scope s(c, "class_scatter");
             launch_scatter(B.d_scat.as<ScatterSeg>() + ch.scat_begin, ch.scat_end - ch.scat_begin,
-                           B.d_scat_cols.as<int32_t>(), (const double2 *)wy, nbox, dst_pool, ch.ncols, nrhs,
+                           B.d_scat_cols.as<int32_t>(), (const double2 *)wy, T0.Lt, B.n0, dst_pool, ch.ncols, nrhs,
                            B.dst_stride, c->stream);
         }
     }
@@ -884,7 +887,7 @@ void class_batch_cost(const ClassBatch &B, double &flops, double &bytes) {
     if (B.gen.empty()) return;
     const Task &T = B.gen[0];
     double ffwd, fax, fback;
-    class_col_flops(T, ffwd, fax, fback);
+    class_col_flops(T, B.n0, ffwd, fax, fback);
     const double ncol = (double)B.src.size();
     flops += (ffwd + fax + fback) * ncol;
     bytes += (4.0 * T.Ls * (T.Ls + 2) * 16.0 * 0.5 + 4.0 * T.Lt * (T.Lt + 2) * 16.0 * 0.5) * ncol;

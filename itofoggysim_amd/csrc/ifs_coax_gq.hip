@@ -28,6 +28,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "ifs_internal.h"
@@ -126,7 +127,7 @@ __global__ void k_gq_T(const GqPlan g, const double *__restrict__ mu, const doub
             ++band;
         }
         double2 cp = ipowg(p, hsh[p]);
-        const double f = (2.0 * p + 1.0) * pc;
+        const double f = p < g.lo[0] ? 0.0 : (2.0 * p + 1.0) * pc;
         acc.x += f * cp.x;
         acc.y += f * cp.y;
     }
@@ -251,6 +252,134 @@ __global__ __launch_bounds__(256) void k_gq_alpha(const GqPlan g, int nm, const 
         for (int b = 0; b < 4; ++b) {
             const int n = r0 + tr + a, nu = c0 + tc + b;
             if (n < NR && nu < NCc) out[(int64_t)n * NCc + nu] = ipowg(((n - nu) % 4 + 4) & 3, make_double2(ar[a][b], ai[a][b]));
+        }
+}
+
+// V[j][n][q] = sqrt((2n+1)/2) d^n_{m,1}(mu_q), m = m0 + j, n = n0..L (0 for n < m).
+__global__ void k_gq_helicity(int m0, int n0, int L, int Q, const double *__restrict__ mu, double *__restrict__ V) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= Q) return;
+    const int m = m0 + blockIdx.y;
+    double *out = V + (int64_t)blockIdx.y * (L - n0 + 1) * Q + q;
+    const double x = mu[q];
+    const double ch = sqrt(0.5 * (1.0 + x)), sh = sqrt(0.5 * (1.0 - x));
+    double d1, d2 = 0.0, sp = 0.0;
+    if (m == 0) {
+        d1 = sqrt(2.0) * ch * sh;
+    } else {
+        double c = 1.0, p = 1.0;  // d^m_{m,1} = sqrt((2m)!/((m+1)!(m-1)!)) ch^{m+1} (-sh)^{m-1}
+        for (int i = 2; i <= m; ++i) {
+            c *= (double)(2 * i) * (double)(2 * i - 1) / (4.0 * (double)(i + 1) * (double)(i - 1));
+            p *= -2.0 * ch * sh;
+        }
+        d1 = sqrt(c) * p * ch * ch;
+    }
+    const int nf = m < 1 ? 1 : m;
+    for (int n = n0; n < nf && n <= L; ++n) out[(int64_t)(n - n0) * Q] = 0.0;
+    const double mm = (double)m * m;
+    for (int n = nf; n <= L; ++n) {
+        if (n > nf) {
+            const double nn = n, n1 = nn - 1.0;
+            const double sc = sqrt((nn * nn - mm) * (nn * nn - 1.0));
+            const double d = ((2.0 * nn - 1.0) * (nn * n1 * x - (double)m) * d1 - nn * sp * d2) / (n1 * sc);
+            d2 = d1;
+            d1 = d;
+            sp = sc;
+        }
+        if (n >= n0) out[(int64_t)(n - n0) * Q] = sqrt(n + 0.5) * d1;
+    }
+}
+
+// The coaxial blocks of degrees n0..L for the terms p >= lo[0]:
+//   P_m(n,nu) = sum_b [n + nu >= lo_b] sum_q V_n V_nu T_b(mu_q),
+//   Q_m(n,nu) = (-1)^{n+nu} the same with T_b(-mu_q)   (d^n_{m,-1}(mu) = (-1)^{n+m} d^n_{m,1}(-mu)).
+// Block: 64 x 64 entries of P or Q of one order (blockIdx.z = 2 j + type), as k_gq_alpha.
+__global__ __launch_bounds__(256) void k_gq_rem(const GqPlan g, int m0, const double *__restrict__ V,
+                                                const double2 *__restrict__ Tb, double2 *__restrict__ wax) {
+    const int L = g.Lt, n0 = g.n0, Q = g.Q;
+    const int j = blockIdx.z >> 1, type = blockIdx.z & 1;
+    const int m = m0 + j;
+    const int q0 = m < n0 ? n0 : m;
+    const int r0 = q0 + blockIdx.y * GT, c0 = q0 + blockIdx.x * GT;
+    if (m > L || r0 > L || c0 > L) return;
+    __shared__ double Vr[GK][GT + 1];
+    __shared__ double Vc[GK][GT + 1];
+    __shared__ double2 Ts[GK];
+    const double *Vm = V + (int64_t)j * (L - n0 + 1) * Q;
+    const int tid = threadIdx.x;
+    const int tr = (tid >> 4) * 4, tc = (tid & 15) * 4;
+    double ar[4][4], ai[4][4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) ar[a][b] = ai[a][b] = 0.0;
+    const int rmax = min(L, r0 + GT - 1), cmax = min(L, c0 + GT - 1);
+    for (int band = 0; band < g.nb; ++band) {
+        const int lo = g.lo[band];
+        if (lo > rmax + cmax) break;
+        const double2 *T = Tb + (int64_t)band * Q;
+        double br[4][4], bi[4][4];
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) br[a][b] = bi[a][b] = 0.0;
+        for (int k0 = 0; k0 < Q; k0 += GK) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int idx = tid + 256 * e;  // 64 x 16
+                const int rr = idx >> 4, qq = idx & 15;
+                const int gq = k0 + qq, gr = r0 + rr, gc = c0 + rr;
+                Vr[qq][rr] = (gq < Q && gr <= L) ? Vm[(int64_t)(gr - n0) * Q + gq] : 0.0;
+                Vc[qq][rr] = (gq < Q && gc <= L) ? Vm[(int64_t)(gc - n0) * Q + gq] : 0.0;
+            }
+            if (tid < GK)
+                Ts[tid] = (k0 + tid < Q) ? T[type == 0 ? k0 + tid : Q - 1 - k0 - tid] : make_double2(0.0, 0.0);
+            __syncthreads();
+#pragma unroll 4
+            for (int qq = 0; qq < GK; ++qq) {
+                const double2 tq = Ts[qq];
+                double vr[4], vi[4], vc[4];
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    vr[a] = Vr[qq][tr + a] * tq.x;
+                    vi[a] = Vr[qq][tr + a] * tq.y;
+                    vc[a] = Vc[qq][tc + a];
+                }
+#pragma unroll
+                for (int a = 0; a < 4; ++a)
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) {
+                        br[a][b] = fma(vr[a], vc[b], br[a][b]);
+                        bi[a][b] = fma(vi[a], vc[b], bi[a][b]);
+                    }
+            }
+            __syncthreads();
+        }
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+                if (r0 + tr + a + c0 + tc + b >= lo) {
+                    ar[a][b] += br[a][b];
+                    ai[a][b] += bi[a][b];
+                }
+    }
+    const int w = L - q0 + 1;
+    const int64_t blk = (int64_t)w * w;
+    // order +m: P then Q; order -m: the other way round
+    double2 *op = wax + ax0_off(m, L, n0) + (type == 0 ? 0 : blk);
+    double2 *on = wax + ax0_off(-m, L, n0) + (type == 0 ? blk : 0);
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const int n = r0 + tr + a, nu = c0 + tc + b;
+            if (n > L || nu > L) continue;
+            const double f = type == 1 && ((n + nu) & 1) ? -1.0 : 1.0;
+            const double2 v = make_double2(f * ar[a][b], f * ai[a][b]);
+            const int64_t o = (int64_t)(n - q0) * w + (nu - q0);
+            op[o] = v;
+            if (m > 0) on[o] = v;
         }
 }
 
@@ -636,7 +765,50 @@ GqPlan gq_plan(int kind, double t, int Lt, int Ls, int K, size_t ws_cap_bytes) {
     return g;
 }
 
+GqPlan gq_plan_rem(double t, int L, int lo, size_t ws_cap_bytes) {
+    GqPlan g;
+    g.kind = 3;
+    g.t = t;
+    g.Lt = g.Ls = g.K = L;
+    g.P = 2 * L;  // the helicity integrals end at p = n + nu
+    g.n0 = lo - L;
+    g.nb = 1;
+    g.lo[0] = lo;
+    std::vector<double> h;
+    hankel_abs_host(t, g.P, h);
+    double ref = h[lo];
+    for (int p = lo + 1; p <= g.P; ++p)
+        if (h[p] > 1e3 * ref && g.nb < GQ_MAXB) {
+            g.lo[g.nb++] = p;
+            ref = h[p];
+        }
+    g.Q = 2 * L + 2;
+    g.Nr = L;
+    const size_t per_m = (size_t)(L - g.n0 + 1) * g.Q * 8;
+    g.mb = (int)std::min<size_t>(std::max<size_t>(ws_cap_bytes / per_m, 1), (size_t)L + 1);
+    g.ws_bytes = per_m * g.mb + (size_t)g.nb * g.Q * 16;
+    return g;
+}
+
+static void launch_gen_axial_rem(const GqPlan &g, const double *mu, const double *w, void *ws, double2 *wax,
+                                 hipStream_t s) {
+    double2 *Tb = (double2 *)ws;
+    double *V = (double *)(Tb + (size_t)g.nb * g.Q);
+    hipLaunchKernelGGL(k_gq_T, dim3((g.Q + 255) / 256), dim3(256), sizeof(double2) * (size_t)(g.P + 1), s, g, mu, w,
+                       Tb);
+    const int gt = (g.Lt - g.n0 + 1 + GT - 1) / GT;
+    for (int m0 = 0; m0 <= g.K; m0 += g.mb) {
+        const int nm = std::min(g.K + 1 - m0, g.mb);
+        hipLaunchKernelGGL(k_gq_helicity, dim3((g.Q + 63) / 64, nm), dim3(64), 0, s, m0, g.n0, g.Lt, g.Q, mu, V);
+        hipLaunchKernelGGL(k_gq_rem, dim3(gt, gt, 2 * nm), dim3(256), 0, s, g, m0, V, Tb, wax);
+    }
+}
+
 void launch_gen_axial_gq(const GqPlan &g, const double *mu, const double *w, void *ws, double2 *wax, hipStream_t s) {
+    if (g.n0 > 1) {
+        launch_gen_axial_rem(g, mu, w, ws, wax, s);
+        return;
+    }
     double2 *Tb = (double2 *)ws;
     double *V = (double *)(Tb + (size_t)g.nb * g.Q);
     double2 *alpha = (double2 *)(V + (size_t)g.mb * (g.Nr + 1) * g.Q);

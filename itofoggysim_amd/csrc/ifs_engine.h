@@ -210,6 +210,8 @@ struct ClassBatch {
     std::vector<ScatterSeg> scat;
     std::vector<int32_t> scat_cols;
     int PL = 0;
+    int n0 = 1;                        // lowest degree carried: > 1 for the part of an offset that the plane
+                                       // waves leave (terms p >= n0 + L of h1; orders Ls = Lt = K)
     int plan_nrhs = 0;                 // right-hand sides the plan was cut for
     int n_dslots = 1;                  // Wigner tables kept at once (chunk runs share slots r % n_dslots)
     // Table keys: one Wigner table per |cos(theta)| (a run of cos(theta) < 0 mirrors

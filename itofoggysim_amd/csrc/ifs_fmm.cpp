@@ -26,6 +26,7 @@
 
 #include "ifs_engine.h"
 #include "ifs_pair.h"
+#include "ifs_pw.h"
 #include "ifs_tree.h"
 
 namespace ifs {
@@ -51,6 +52,8 @@ struct Fmm {
     Batch p2m, l2p, p2p;
     PairBatch pair;                             // near field, unless the pair kernels do not apply (p2p)
     std::vector<ClassBatch> m2m, m2l, l2l;      // indexed by level
+    std::vector<PwLevel> pw;                    // M2L in the plane-wave basis, by level
+    std::vector<std::vector<ClassBatch>> rem;   // what it leaves of near offsets, by level and length
     int64_t counts[6] = {0, 0, 0, 0, 0, 0};
 };
 
@@ -187,9 +190,15 @@ int build(ifs_ctx *c, Fmm **out) {
     }
     // M2L: I4 of every box, one class per integer offset o = coords(src) - coords(tgt);
     // d = dsign * o * edge.  Classes ordered by |o|^2, then o_z, so consecutive classes share tables.
+    // The offsets the plane waves can carry go there where a level has enough of them.
+    auto o2_of = [](const std::array<int, 3> &o) { return o[0] * o[0] + o[1] * o[1] + o[2] * o[2]; };
     f->m2l.resize(lmax + 1);
+    f->pw.resize(lmax + 1);
+    f->rem.resize(lmax + 1);
     for (int l = lmin; l <= lmax; ++l) {
         const Level &V = f->lv[l];
+        const bool pw_ok = c->prm.z_selector == IFS_ZSEL_HANKEL1 && pw_fits(c, V.L, (int)V.boxes.size(), 1);
+        int64_t pw_cols = 0;
         std::map<std::array<int, 3>, std::vector<std::pair<int64_t, int64_t>>> cls;
         for (size_t q = 0; q < V.boxes.size(); ++q) {
             int64_t vt[3];
@@ -205,8 +214,64 @@ int build(ifs_ctx *c, Fmm **out) {
                 cls[o].push_back({V.off + (int64_t)p * V.per_box(), V.off + (int64_t)q * V.per_box()});
             }
         }
+        auto pw_offset = [&](const std::array<int, 3> &o) {
+            return pw_ok && pw_takes(pw_terms(k, V.edge, o2_of(o), V.L), V.L);
+        };
+        for (auto &kv : cls)
+            if (pw_offset(kv.first)) pw_cols += (int64_t)kv.second.size();
+        const bool use_pw = pw_worth(V.L, (int)V.boxes.size(), pw_cols);
+        if (use_pw) {
+            // sources of every parent: the boxes its children's interaction lists hold
+            PwLevel &P = f->pw[l];
+            P.L = V.L;
+            P.nb = (int)V.boxes.size();
+            P.off = V.off;
+            P.k = k;
+            P.edge = V.edge;
+            P.ncols = pw_cols;
+            f->counts[2] += pw_cols;
+            std::map<int64_t, std::map<int, PwSource>> parents;  // parent -> source box
+            std::map<int64_t, std::array<int, 8>> kids;
+            for (size_t q = 0; q < V.boxes.size(); ++q) {
+                auto it = kids.find(tree::parent(V.boxes[q]));
+                if (it == kids.end()) {
+                    it = kids.emplace(tree::parent(V.boxes[q]), std::array<int, 8>{}).first;
+                    it->second.fill(-1);
+                }
+                it->second[V.boxes[q] & 7] = (int)q;
+            }
+            auto box_at = [&](int64_t off) { return (int)((off - V.off) / V.per_box()); };
+            for (auto &kv : cls) {
+                if (!pw_offset(kv.first)) continue;
+                const auto &o = kv.first;
+                for (auto &sd : kv.second) {
+                    const int sb = box_at(sd.first), tb = box_at(sd.second), ch = (int)(V.boxes[tb] & 7);
+                    const int r[3] = {o[0] + (ch >> 2), o[1] + (ch >> 1 & 1), o[2] + (ch & 1)};
+                    PwSource &S = parents[tree::parent(V.boxes[tb])][sb];
+                    S.box = sb;
+                    S.r = ((r[0] + 2) * 6 + r[1] + 2) * 6 + r[2] + 2;
+                    S.mask |= 1 << ch;
+                }
+            }
+            for (auto &kd : kids) {
+                PwParent G{};
+                for (int ch = 0; ch < 8; ++ch) G.child[ch] = kd.second[ch];
+                G.beg = (int)P.src.size();
+                for (auto &sv : parents[kd.first]) P.src.push_back(sv.second);
+                G.end = (int)P.src.size();
+                P.par.push_back(G);
+            }
+            if ((rc = pw_build(c, P, isg))) {
+                delete f;
+                return rc;
+            }
+            c->flops_mv += pw_flops(P);
+        }
+        // class products: whole offsets, and the terms of near ones that the plane waves leave
         std::vector<std::array<int, 3>> keys;
-        for (auto &kv : cls) keys.push_back(kv.first);
+        for (auto &kv : cls)
+            if (!(use_pw && pw_offset(kv.first) && pw_terms(k, V.edge, o2_of(kv.first), V.L) >= 2 * V.L))
+                keys.push_back(kv.first);
         std::sort(keys.begin(), keys.end(), [](const std::array<int, 3> &a, const std::array<int, 3> &b) {
             int ra = a[0] * a[0] + a[1] * a[1] + a[2] * a[2], rb = b[0] * b[0] + b[1] * b[1] + b[2] * b[2];
             if (ra != rb) return ra < rb;
@@ -218,8 +283,18 @@ int build(ifs_ctx *c, Fmm **out) {
             std::sort(cols.begin(), cols.end(), [](auto &x, auto &y) { return x.second < y.second; });
             int os[3] = {isg * o[0], isg * o[1], isg * o[2]};
             double dv[3] = {os[0] * V.edge, os[1] * V.edge, os[2] * V.edge};
-            add_class(f->m2l[l], dv, k, c->prm.z_selector, V.L, V.L, cols, os, V.edge);
-            f->counts[2] += (int64_t)cols.size();
+            ClassBatch *B = &f->m2l[l];
+            if (use_pw && pw_offset(o)) {
+                const int n0 = pw_terms(k, V.edge, o2_of(o), V.L) + 1 - V.L;
+                if (f->rem[l].empty() || f->rem[l].back().n0 != n0) {  // keys come by length
+                    f->rem[l].emplace_back();
+                    f->rem[l].back().n0 = n0;
+                }
+                B = &f->rem[l].back();
+            } else {
+                f->counts[2] += (int64_t)cols.size();
+            }
+            add_class(*B, dv, k, c->prm.z_selector, V.L, V.L, cols, os, V.edge);
         }
     }
     // L2L: parent (level l-1) -> child (level l), one class per child octant;
@@ -306,6 +381,10 @@ int build(ifs_ctx *c, Fmm **out) {
             }
             if ((rc = cfin(f->m2l[l], "m2l"))) goto fail;
             cls.push_back(&f->m2l[l]);
+            for (auto &B : f->rem[l]) {
+                if ((rc = cfin(B, "m2l"))) goto fail;
+                cls.push_back(&B);
+            }
             if (l > lmin) {
                 if ((rc = cfin(f->l2l[l], "l2l"))) goto fail;
                 cls.push_back(&f->l2l[l]);
@@ -342,6 +421,9 @@ int run(ifs_ctx *c, Fmm *f, const double2 *xh, double2 *acc, int nrhs, int64_t l
     for (int l = f->l_max - 1; l >= f->l_min; --l)
         if ((rc = class_batch_run(c, f->m2m[l], C, C, nrhs, prec))) return rc;
     for (int l = f->l_min; l <= f->l_max; ++l) {
+        if (f->pw[l].active() && (rc = pw_run(c, f->pw[l], C, D, nrhs, st, prec))) return rc;
+        for (auto &B : f->rem[l])
+            if ((rc = class_batch_run(c, B, C, D, nrhs, prec))) return rc;
         if ((rc = class_batch_run(c, f->m2l[l], C, D, nrhs, prec))) return rc;
         if (l > f->l_min && (rc = class_batch_run(c, f->l2l[l], D, D, nrhs, prec))) return rc;
     }
@@ -361,7 +443,10 @@ uint64_t buffers_sig(Fmm *f) {
         for (const DevBuf *d : {&B->d_tasks, &B->d_segs, &B->own_d, &B->own_s, &B->own_ax, &B->own_y, &B->own_z})
             buf(*d);
     mix(pair_sig(f->pair));
-    for (const auto *v : {&f->m2m, &f->m2l, &f->l2l})
+    for (auto &P : f->pw) mix(pw_sig(P));
+    std::vector<const std::vector<ClassBatch> *> all = {&f->m2m, &f->m2l, &f->l2l};
+    for (auto &v : f->rem) all.push_back(&v);
+    for (const auto *v : all)
         for (const ClassBatch &B : *v) {
             mix((uint64_t)B.plan_nrhs);
             for (const DevBuf *d : {&B.own_d, &B.own_ax, &B.d_dkeys, &B.d_desc, &B.d_gen, &B.d_src, &B.d_pidx,

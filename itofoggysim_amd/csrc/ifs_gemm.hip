@@ -103,7 +103,7 @@ __global__ __launch_bounds__(256, MINB) void k_class_rot_fwd(const GroupDesc *__
                                                        const TW *__restrict__ wd, TC *__restrict__ wy) {
     typedef typename Mx<TC>::v4 acc4;
     const GroupDesc C = *desc;
-    const int nu = blockIdx.z + 1;
+    const int nu = blockIdx.z + C.n0;
     if (nu > C.Ls) return;
     const int K = C.K;
     const int kk = nu < K ? nu : K;
@@ -258,7 +258,7 @@ __global__ __launch_bounds__(256, MINB) void k_class_rot_fwd(const GroupDesc *__
     }
     __syncthreads();
     if (g == 1) return;
-    TC *Y = wy + rows_off(nu, K) * (int64_t)NCY + 4 * (int64_t)C.ycol0 * C.nrhs;
+    TC *Y = wy + (rows_off(nu, K) - rows_off(C.n0, K)) * (int64_t)NCY + 4 * (int64_t)C.ycol0 * C.nrhs;
 #pragma unroll
     for (int i = 0; i < NI; ++i)
 #pragma unroll
@@ -291,7 +291,7 @@ __global__ __launch_bounds__(256, MINB) void k_class_rot_back(const GroupDesc *_
                                                         double2 *__restrict__ W) {
     typedef typename Mx<TC>::v4 acc4;
     const GroupDesc C = *desc;
-    const int n = blockIdx.z + 1;
+    const int n = blockIdx.z + C.n0;
     if (n > C.Lt) return;
     const int K = C.K;
     const int kk = n < K ? n : K;
@@ -307,7 +307,7 @@ __global__ __launch_bounds__(256, MINB) void k_class_rot_back(const GroupDesc *_
     __shared__ TC Bs[2][FK][FNB + RPAD];     // s, t
     const TW *E = wd + C.off_d + fold_off(n, K);  // E[k][m], KI x M
     const TW *O = E + (int64_t)KI * M;
-    const TC *Z = wz + rows_off(n, K) * (int64_t)NCY + 4 * (int64_t)C.ycol0 * C.nrhs;  // row kk + k
+    const TC *Z = wz + (rows_off(n, K) - rows_off(C.n0, K)) * (int64_t)NCY + 4 * (int64_t)C.ycol0 * C.nrhs;  // row kk + k
     const int tid = threadIdx.x;
     const int lane = tid & 63, w = tid >> 6;
     const int li = lane & 15, lk = lane >> 4;
@@ -423,7 +423,8 @@ __global__ __launch_bounds__(256, MINB) void k_class_rot_back(const GroupDesc *_
         __syncthreads();
     }
     // w_m and w_{-m}; the 4 parts of a translation sit in lanes li..li+3 (li % 4 == 0)
-    const int64_t ndst = (int64_t)C.Lt * (C.Lt + 2);
+    const int64_t e0 = (int64_t)C.n0 * C.n0 - 1;  // entries below degree n0
+    const int64_t ndst = (int64_t)C.Lt * (C.Lt + 2) - e0;
 #pragma unroll
     for (int i = 0; i < NI; ++i)
 #pragma unroll
@@ -451,7 +452,7 @@ __global__ __launch_bounds__(256, MINB) void k_class_rot_back(const GroupDesc *_
                     // w_m: parts (wp, p1) = z_+, (p2, p3) = z_-; a = (z_+ + z_-)/2, b = (z_+ - z_-)/2; phase e^{-i m phi}
                     double ar = 0.5 * (wp + p2), ai = 0.5 * (p1 + p3);
                     double br = 0.5 * (wp - p2), bi = 0.5 * (p1 - p3);
-                    int64_t o = fidx(n, m);
+                    int64_t o = fidx(n, m) - e0;
                     dst[o] = make_double2(ph.x * ar + ph.y * ai, ph.x * ai - ph.y * ar);
                     dst[o + ndst] = make_double2(ph.x * br + ph.y * bi, ph.x * bi - ph.y * br);
                 }
@@ -460,7 +461,7 @@ __global__ __launch_bounds__(256, MINB) void k_class_rot_back(const GroupDesc *_
                     double sg = (m & 1) ? -1.0 : 1.0;
                     double ar = 0.5 * sg * (wm + q2), ai = 0.5 * sg * (q1 + q3);
                     double br = 0.5 * sg * (wm - q2), bi = 0.5 * sg * (q1 - q3);
-                    int64_t o = fidx(n, -m);
+                    int64_t o = fidx(n, -m) - e0;
                     dst[o] = make_double2(ph.x * ar - ph.y * ai, ph.x * ai + ph.y * ar);
                     dst[o + ndst] = make_double2(ph.x * br - ph.y * bi, ph.x * bi + ph.y * br);
                 }
@@ -490,7 +491,7 @@ __global__ __launch_bounds__(256) void k_class_axial(const GroupDesc *__restrict
     const int K = C.K;
     const int k = (int)blockIdx.z - K;
     const int ak = k < 0 ? -k : k;
-    const int q = ak < 1 ? 1 : ak;
+    const int q = ak < C.n0 ? C.n0 : ak;  // n0 >= 1
     const int Lt = C.Lt, Ls = C.Ls;
     const int M = Lt - q + 1;
     const int KI = Ls - q + 1;
@@ -500,8 +501,9 @@ __global__ __launch_bounds__(256) void k_class_axial(const GroupDesc *__restrict
     const int NC = 4 * C.ncy * C.nrhs;                     // row stride of Y and Z
     const int64_t cb = 4 * (int64_t)C.ycol0 * C.nrhs;      // first real column of the segment
     const int NTOT = C.ncols * C.nrhs;                     // columns of the segment
-    const double2 *Pb = wax + C.off_ax + ax_off(k, Lt, Ls, K);
-    const double2 *Qb = Pb + ax_block(k, Lt, Ls);
+    const double2 *Pb = wax + C.off_ax + (C.n0 > 1 ? ax0_off(k, Lt, C.n0) : ax_off(k, Lt, Ls, K));
+    const double2 *Qb = Pb + (int64_t)M * KI;
+    const int64_t rbase = rows_off(C.n0, K);
     // rows padded by one entry: the tile store writes 8 inner columns of one row from
     // 8 consecutive lanes, which a 1 KiB row stride would put on the same banks
     __shared__ c2 Ps[AK][AM + 1];
@@ -552,7 +554,7 @@ __global__ __launch_bounds__(256) void k_class_axial(const GroupDesc *__restrict
         // inner rows nu = q + k0 + yrow + (256 / (4 AN)) e x 4 AN reals (AN translations x 4);
         // the row of (nu, k) advances by 2 nu + 2 (nu < K) or 2 K + 1 per degree
         int nu = q + k0 + yrow;
-        int64_t row = rows_off(nu, K) + k + (nu < K ? nu : K);
+        int64_t row = rows_off(nu, K) - rbase + k + (nu < K ? nu : K);
 #pragma unroll
         for (int e = 0; e < NY; ++e) {
             py[e] = (ycol_ok && nu <= Ls) ? ybase[row * NC] : (TC)0;
@@ -624,7 +626,7 @@ __global__ __launch_bounds__(256) void k_class_axial(const GroupDesc *__restrict
             int n = q + row0 + w * 16 + 8 * i + (Mx<TC>::F32 ? h + 2 * lk : 4 * h + lk);
             if (n > Lt) continue;
             int kq = n < K ? n : K;
-            TC *row = wz + (rows_off(n, K) + (k + kq)) * (int64_t)NC + cb;
+            TC *row = wz + (rows_off(n, K) - rbase + (k + kq)) * (int64_t)NC + cb;
 #pragma unroll
             for (int j = 0; j < NJ; ++j) {
                 int t = col0 + 16 * j + li;
@@ -640,20 +642,22 @@ __global__ __launch_bounds__(256) void k_class_axial(const GroupDesc *__restrict
 // Deterministic per-target sum of back-rotated columns: grid (targets, element blocks).
 // grid (targets, element blocks, right-hand sides).
 __global__ __launch_bounds__(256) void k_scatter(const ScatterSeg *__restrict__ segs, const int32_t *__restrict__ cols,
-                                                 const double2 *__restrict__ W, int64_t nbox,
+                                                 const double2 *__restrict__ W, int64_t nbox, int64_t e0,
                                                  double2 *__restrict__ dst_pool, int ncy, int64_t dst_stride) {
     const ScatterSeg S = segs[blockIdx.x];
     const int r = blockIdx.z;
-    double2 *dst = dst_pool + r * dst_stride + S.dst;
+    const int64_t half = nbox / 2;
+    double2 *dst = dst_pool + r * dst_stride + S.dst + e0;
     const double2 *Wr = W + (int64_t)r * ncy * nbox;
     for (int64_t e = (int64_t)blockIdx.y * blockDim.x + threadIdx.x; e < nbox; e += (int64_t)blockDim.x * gridDim.y) {
-        double2 acc = dst[e];
+        double2 *d = dst + e + (e < half ? 0 : e0);  // the b-part starts e0 entries later
+        double2 acc = *d;
         for (int i = S.beg; i < S.end; ++i) {
             double2 v = Wr[(int64_t)cols[i] * nbox + e];
             acc.x += v.x;
             acc.y += v.y;
         }
-        dst[e] = acc;
+        *d = acc;
     }
 }
 
@@ -666,7 +670,7 @@ static void launch_class_t(const GroupDesc &h, const GroupDesc *d_desc, const in
     if (stage == 0) {
         const int rm = rows == 32 ? 32 : FMF;
         int mt = ((h.Ls < K ? h.Ls : K) + 1 + rm - 1) / rm;
-        dim3 grid((NC + FNF2 - 1) / FNF2, mt, h.Ls);
+        dim3 grid((NC + FNF2 - 1) / FNF2, mt, h.Ls - h.n0 + 1);
         if (rm == 32)
             hipLaunchKernelGGL((k_class_rot_fwd<TC, TW, 32, 3>), grid, dim3(256), 0, s, d_desc, src_off, pidx, phase,
                                src_pool, wd, wy);
@@ -674,7 +678,7 @@ static void launch_class_t(const GroupDesc &h, const GroupDesc *d_desc, const in
             hipLaunchKernelGGL((k_class_rot_fwd<TC, TW, FMF, 3>), grid, dim3(256), 0, s, d_desc, src_off, pidx, phase,
                                src_pool, wd, wy);
     } else if (stage == 1) {
-        int mt = (h.Lt + AM - 1) / AM;
+        int mt = (h.Lt - h.n0 + 1 + AM - 1) / AM;
         const int nt = h.ncols * h.nrhs;
         int nfull;
         bool tail;
@@ -688,7 +692,7 @@ static void launch_class_t(const GroupDesc &h, const GroupDesc *d_desc, const in
     } else {
         const int fm = rows == 32 ? 32 : FMB;
         int mt = (h.Lt + 1 + fm - 1) / fm;
-        dim3 grid((NC + FNB - 1) / FNB, mt, h.Lt);
+        dim3 grid((NC + FNB - 1) / FNB, mt, h.Lt - h.n0 + 1);
         // W (FP64 columns) aliases the Y workspace, free once the coaxial shifts are done
         if (fm == 32)
             hipLaunchKernelGGL((k_class_rot_back<TC, TW, 32, 3>), grid, dim3(256), 0, s, d_desc, pidx, phase, wd,
@@ -713,11 +717,13 @@ void launch_class(const GroupDesc &h, const GroupDesc *d_desc, const int64_t *sr
         launch_class_t<double, double>(h, d_desc, src_off, pidx, phase, src_pool, wd, wax, wy, wz, stage, rows, s);
 }
 
-void launch_scatter(const ScatterSeg *segs, int nsegs, const int32_t *cols, const double2 *W, int64_t nbox,
+void launch_scatter(const ScatterSeg *segs, int nsegs, const int32_t *cols, const double2 *W, int Lt, int n0,
                     double2 *dst_pool, int ncy, int nrhs, int64_t dst_stride, hipStream_t s) {
     if (nsegs <= 0 || nrhs <= 0) return;
+    const int64_t e0 = (int64_t)n0 * n0 - 1;
+    const int64_t nbox = 2 * ((int64_t)Lt * (Lt + 2) - e0);
     int yb = (int)std::min<int64_t>((nbox + 255) / 256, 64);
-    hipLaunchKernelGGL(k_scatter, dim3(nsegs, yb, nrhs), dim3(256), 0, s, segs, cols, W, nbox, dst_pool, ncy,
+    hipLaunchKernelGGL(k_scatter, dim3(nsegs, yb, nrhs), dim3(256), 0, s, segs, cols, W, nbox, e0, dst_pool, ncy,
                        dst_stride);
 }
 

@@ -58,6 +58,8 @@ struct GroupDesc {
     int32_t nrhs;      // right-hand sides
     int32_t mirror;    // run of the supplementary polar angle pi - b: its tables are those of b,
                        // with d^n_{km}(pi - b) = (-1)^{n+k} d^n_{k,-m}(b) applied in the products
+    int32_t n0;        // lowest degree carried (source and target); rows of Y, Z and W start there
+    int32_t pad_;
     int64_t src_stride, dst_stride;
 };
 
@@ -129,6 +131,20 @@ __host__ __device__ inline int64_t ax_off(int k, int Lt, int Ls, int K) {
     return 2 * ax_sum(1, K, Lt, Ls) + 2 * ax_block(0, Lt, Ls) + 2 * ax_sum(1, k - 1, Lt, Ls);
 }
 __host__ __device__ inline int64_t ax_size(int Lt, int Ls, int K) { return ax_off(K, Lt, Ls, K) + 2 * ax_block(K, Lt, Ls); }
+// Coaxial tables of degrees n0..L only (Lt = Ls = K = L): block k holds rows and columns
+// q..L, q = max(1, |k|, n0); the blocks are ordered as above.
+__host__ __device__ inline int64_t ax0_block(int k, int L, int n0) {
+    int q = k < 0 ? -k : k;
+    if (q < n0) q = n0;
+    return (int64_t)(L - q + 1) * (L - q + 1);
+}
+__host__ __device__ inline int64_t ax0_off(int k, int L, int n0) {
+    if (k <= -n0) return 2 * ax_sum(1 - k, L, L, L);
+    const int64_t neg = 2 * ax_sum(n0, L, L, L), b = 2 * ax0_block(0, L, n0);
+    if (k <= n0) return neg + (int64_t)(k - 1 + n0) * b;
+    return neg + (int64_t)(2 * n0) * b + 2 * ax_sum(n0 + 1, k - 1, L, L);
+}
+__host__ __device__ inline int64_t ax0_size(int L, int n0) { return ax0_off(L, L, n0) + 2 * ax0_block(L, L, n0); }
 __host__ __device__ inline int64_t sect_size(int K, int nmax) { return (int64_t)(K + 1) * (nmax + 2); }
 
 // Coaxial tables by Gauss-Legendre quadrature (ifs_coax_gq.hip): one table of
@@ -141,11 +157,14 @@ struct GqPlan {
     int Lt = 0, Ls = 0, K = 0;
     int P = 0;                         // outgoing kind: Legendre degree of T
     int nb = 1;                        // bands of T: band b holds p in [lo[b], lo[b+1])
-    int lo[GQ_MAXB] = {0};
+    int lo[GQ_MAXB] = {0};             // terms below lo[0] are left out
+    int n0 = 1;                        // > 1: table of degrees n0..L (gq_plan_rem)
     int Q = 0, Nr = 0, mb = 1;         // nodes, Legendre rows, orders per batch
     size_t ws_bytes = 0;
 };
 GqPlan gq_plan(int kind, double t, int Lt, int Ls, int K, size_t ws_cap_bytes);
+// The table of the terms p >= lo of T for the degrees n0 = lo - L .. L of both sides (order L).
+GqPlan gq_plan_rem(double t, int L, int lo, size_t ws_cap_bytes);
 // mu, w: the Q Gauss-Legendre nodes and weights on the device
 void launch_gen_axial_gq(const GqPlan &g, const double *mu, const double *w, void *ws, double2 *wax, hipStream_t s);
 
@@ -215,7 +234,8 @@ void launch_class(const GroupDesc &h, const GroupDesc *d_desc, const int64_t *sr
                   double *wz, int stage, int prec, int ftab, int rows, hipStream_t s);
 // dst_pool[r dst_stride + seg.dst + e] += sum_{i in [beg,end)} W[r ncy + cols[i]][e],
 // e < nbox = 2 Lt(Lt+2), r < nrhs
-void launch_scatter(const ScatterSeg *segs, int nsegs, const int32_t *cols, const double2 *W, int64_t nbox,
+// (degrees n0..L only: W holds L(L+2) - (n0^2 - 1) entries of each part)
+void launch_scatter(const ScatterSeg *segs, int nsegs, const int32_t *cols, const double2 *W, int Lt, int n0,
                     double2 *dst_pool, int ncy, int nrhs, int64_t dst_stride, hipStream_t s);
 
 void launch_mie(int ns, const double *xsize, const double2 *mrel, int N, double2 *an, double2 *bn, hipStream_t s);
