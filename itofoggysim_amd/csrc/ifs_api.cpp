@@ -894,10 +894,16 @@ void class_batch_cost(const ClassBatch &B, double &flops, double &bytes) {
 }
 
 void batch_cost(const Batch &B, double &flops, double &bytes) {
+    // few distinct (source order, target order) pairs
+    std::map<std::pair<int, int>, double> by_order;
     for (auto &T : B.tasks) {
-        double f1, f2, f3;
-        task_flops(T, f1, f2, f3);
-        flops += f1 + f2 + f3;
+        double &f = by_order[{T.Ls, T.Lt}];
+        if (f == 0.0) {
+            double f1, f2, f3;
+            task_flops(T, f1, f2, f3);
+            f = f1 + f2 + f3;
+        }
+        flops += f;
         bytes += 4.0 * T.Ls * (T.Ls + 2) * 16.0 * 0.5 + 4.0 * T.Lt * (T.Lt + 2) * 16.0 * 0.5;
     }
 }

@@ -95,6 +95,14 @@ int pair_plan(ifs_ctx *c, PairBatch &B, int nrhs) {
         }
         first.push_back(tile);
     }
+    // algorithmic flops of a folded rotation of order L with |k| <= K
+    std::vector<double> rot((size_t)(kPairMaxL + 1) * (kPairMaxL + 1), 0.0);
+    for (int L = 1; L <= kPairMaxL; ++L)
+        for (int K = 0; K <= L; ++K) {
+            const double kk = std::min(L, K);
+            const double below = L > 1 ? rot[(L - 1) * (kPairMaxL + 1) + std::min(K, L - 1)] : 0.0;
+            rot[L * (kPairMaxL + 1) + K] = below + 8.0 * ((kk + 1.0) * (L + 1.0) + kk * L);
+        }
     PairBatch::Chunk cur;
     size_t used = 0;
     int64_t tab = 0, ax = 0;  // running table offsets when the tables are kept
@@ -161,20 +169,14 @@ int pair_plan(ifs_ctx *c, PairBatch &B, int nrhs) {
                 for (int s = 0; s < 4; ++s) {
                     PairSlot &S = B.slots[4 * t + s];
                     if (S.src < 0) continue;
-                    for (int n = 1; n <= S.Ls; ++n) {
-                        const double kk = std::min(n, S.K);
-                        cur.f_fwd += 8.0 * ((kk + 1.0) * (n + 1.0) + kk * n);
-                    }
-                    for (int n = 1; n <= T.Lt; ++n) {
-                        const double kk = std::min(n, S.K);
-                        cur.f_back += 8.0 * ((kk + 1.0) * (n + 1.0) + kk * n);
-                    }
-                    cur.f_ax += 16.0 * (double)ax_size(T.Lt, S.Ls, S.K) / 2.0;
+                    cur.f_fwd += rot[S.Ls * (kPairMaxL + 1) + S.K];
+                    cur.f_back += rot[T.Lt * (kPairMaxL + 1) + S.K];
+                    cur.f_ax += 8.0 * (double)ax_size(T.Lt, S.Ls, S.K);
                     if (T.Q) continue;
                     Task K{};
                     K.t = S.t;
-                    K.Ls = S.Ls;
-                    K.Lt = T.Lt;
+                    K.Ls = T.Lt;  // source and target change places (see the kernel)
+                    K.Lt = S.Ls;
                     K.K = S.K;
                     K.kind = IFS_ZSEL_HANKEL1;
                     S.off_ax = K.off_ax = na_;
@@ -189,6 +191,28 @@ int pair_plan(ifs_ctx *c, PairBatch &B, int nrhs) {
         }
     }
     if (cur.t0 < (int)B.tiles.size()) close_chunk();
+    // tiles by node set, 8 to a block of the shift (4 where a chunk has few)
+    B.groups.clear();
+    B.order.clear();
+    for (auto &ch : B.chunks) {
+        ch.waves = ch.t1 - ch.t0 >= 1024 ? 8 : 4;
+        std::vector<int32_t> o;
+        for (int t = ch.t0; t < ch.t1; ++t) o.push_back(t);
+        std::stable_sort(o.begin(), o.end(), [&](int a, int b) { return B.tiles[a].Q < B.tiles[b].Q; });
+        ch.a0 = (int)B.groups.size();
+        for (size_t i = 0; i < o.size();) {
+            const PairTile &T = B.tiles[o[i]];
+            PairGroup G{(int)(B.order.size() + i), 0, T.Q, 0, 0, 0, T.off_q};
+            for (; i < o.size() && G.count < ch.waves && B.tiles[o[i]].Q == G.Q; ++i, ++G.count) {
+                G.Ls = std::max(G.Ls, B.tiles[o[i]].Ls);
+                G.Lt = std::max(G.Lt, B.tiles[o[i]].Lt);
+                G.K = std::max(G.K, B.tiles[o[i]].K);
+            }
+            B.groups.push_back(G);
+        }
+        ch.a1 = (int)B.groups.size();
+        B.order.insert(B.order.end(), o.begin(), o.end());
+    }
     int64_t my = 0, mz = 0, mw = 0, mt = 0, ma = 0, ms = 0;
     for (auto &ch : B.chunks) {
         my = std::max(my, ch.n_y);
@@ -208,6 +232,8 @@ int pair_plan(ifs_ctx *c, PairBatch &B, int nrhs) {
         (rc = upload(B.d_slots, B.slots.data(), sizeof(PairSlot) * B.slots.size())) ||
         (rc = upload(B.d_segs, B.segs.data(), sizeof(PairSeg) * B.segs.size())) ||
         (rc = upload(B.d_targets, B.targets.data(), sizeof(PairTarget) * B.targets.size())) ||
+        (rc = upload(B.d_groups, B.groups.data(), sizeof(PairGroup) * B.groups.size())) ||
+        (rc = upload(B.d_order, B.order.data(), 4 * B.order.size())) ||
         (rc = upload(B.d_close, B.close.data(), sizeof(Task) * B.close.size())))
         return rc;
     B.plan_nrhs = nrhs;
@@ -308,8 +334,9 @@ int pair_run(ifs_ctx *c, PairBatch &B, const double2 *src_pool, double2 *dst_poo
         }
         {
             Scope s(c, B.pn[2], ch.f_ax * nrhs);
-            launch_pair_axial(tiles, slots, ch.t0, nt, ch.max_K, ch.max_Lt, B.NL, quad, tab, wax, Y, ch.n_y, Z,
-                              ch.n_z, nrhs, c->stream);
+            launch_pair_axial(tiles, slots, B.d_groups.as<PairGroup>() + ch.a0, ch.a1 - ch.a0,
+                              B.d_order.as<int32_t>(), ch.waves, ch.max_K, std::max(ch.max_Ls, ch.max_Lt), B.NL, quad,
+                              tab, wax, Y, ch.n_y, Z, ch.n_z, nrhs, c->stream);
         }
         {
             Scope s(c, B.pn[3], ch.f_back * nrhs);
@@ -326,7 +353,7 @@ int pair_run(ifs_ctx *c, PairBatch &B, const double2 *src_pool, double2 *dst_poo
 
 uint64_t pair_sig(const PairBatch &B) {
     uint64_t h = (uint64_t)B.plan_nrhs;
-    for (const DevBuf *d : {&B.d_tiles, &B.d_slots, &B.d_segs, &B.d_targets, &B.d_close, &B.d_delta, &B.d_quad,
+    for (const DevBuf *d : {&B.d_tiles, &B.d_slots, &B.d_segs, &B.d_targets, &B.d_close, &B.d_groups, &B.d_order, &B.d_delta, &B.d_quad,
                             &B.own_tab, &B.own_ax})
         h ^= (uint64_t)(uintptr_t)d->p + 0x9e3779b97f4a7c15ull + (h << 6) + (h >> 2);
     return h;

@@ -37,6 +37,11 @@ struct PairSeg {
     int64_t off_w;    // complex offset of the partial sum, 2 Lt (Lt + 2) entries
     int32_t Lt, t_begin, t_end, pad_;
 };
+// Tiles of one node set (positions first .. of the order list) shifted by one block.
+struct PairGroup {
+    int32_t first, count, Q, Ls, Lt, K;  // largest orders of its tiles
+    int64_t off_q;
+};
 struct PairTarget {
     int64_t dst;      // complex offset of the target expansion
     int32_t Lt, s_begin, s_end, pad_;
@@ -45,6 +50,7 @@ struct PairTarget {
 struct PairBatch {
     struct Chunk {
         int t0 = 0, t1 = 0, s0 = 0, s1 = 0, g0 = 0, g1 = 0, c0 = 0, c1 = 0;  // tiles, segments, targets, close tasks
+        int a0 = 0, a1 = 0, waves = 4;  // groups, tiles of a group
         int64_t n_y = 0, n_z = 0, n_w = 0, n_tab = 0, n_ax = 0, n_s = 0;
         int max_Ls = 0, max_Lt = 0, max_K = 0, maxK_close = 0, max_nmax = 0, max_tabw = 0, max_P = 0;
         double f_fwd = 0.0, f_ax = 0.0, f_back = 0.0;
@@ -53,9 +59,11 @@ struct PairBatch {
     std::vector<PairSlot> slots;
     std::vector<PairSeg> segs;
     std::vector<PairTarget> targets;
+    std::vector<PairGroup> groups;
+    std::vector<int32_t> order;  // tiles of a chunk by node set
     std::vector<Task> close;  // coaxial tables by the degree recurrence
     std::vector<Chunk> chunks;
-    DevBuf d_tiles, d_slots, d_segs, d_targets, d_close;
+    DevBuf d_tiles, d_slots, d_segs, d_targets, d_close, d_groups, d_order;
     DevBuf d_delta, d_quad;   // shared matrices
     DevBuf own_tab, own_ax;   // tables kept across matvecs
     bool kept = false, ready = false;
@@ -92,9 +100,10 @@ void launch_pair_tables(const PairTile *tiles, const PairSlot *slots, int t0, in
 void launch_pair_fwd(const PairTile *tiles, const PairSlot *slots, int t0, int ntiles, int max_Ls, const double *delta,
                      const double2 *tab, const double2 *src, int64_t src_stride, double *Y, int64_t y_stride, int nrhs,
                      hipStream_t s);
-void launch_pair_axial(const PairTile *tiles, const PairSlot *slots, int t0, int ntiles, int max_K, int max_Lt, int NL,
-                       const double *quad, const double2 *tab, const double2 *wax, const double *Y, int64_t y_stride,
-                       double *Z, int64_t z_stride, int nrhs, hipStream_t s);
+void launch_pair_axial(const PairTile *tiles, const PairSlot *slots, const PairGroup *groups, int ngroups,
+                       const int32_t *order, int waves, int max_K, int max_L, int NL, const double *quad,
+                       const double2 *tab, const double2 *wax, const double *Y, int64_t y_stride, double *Z,
+                       int64_t z_stride, int nrhs, hipStream_t s);
 void launch_pair_back(const PairTile *tiles, const PairSeg *segs, int s0, int nsegs, int max_Lt, const double *delta,
                       const double2 *tab, const double *Z, int64_t z_stride, double2 *W, int64_t w_stride, int nrhs,
                       hipStream_t s);

@@ -25,9 +25,9 @@
 //
 // Bound by the matrix cores and their operand reads from L1/L2 (tiles are 50-75% full at
 // orders 10 to 25).  Against per-pair tables: 22650 pairs of orders 9-18 (151 spheres at
-// 800 nm) 3.57 -> 0.72 ms per product, the near field of 2500 spheres at 550 nm (248818
-// pairs, orders 9-23) 40.1 -> 12.2 ms, with four right-hand sides (114758 pairs) 81.9 ->
-// 21.3 ms; error against 64-bit sums unchanged (3e-13, 1.1e-13).
+// 800 nm) 3.57 -> 0.53 ms per product, the near field of 2500 spheres at 550 nm (248818
+// pairs, orders 9-23) 40.1 -> 8.8 ms, with four right-hand sides (114758 pairs) 81.9 ->
+// 15.3 ms; error against 64-bit sums unchanged (3e-13, 1.1e-13).
 #include <hip/hip_runtime.h>
 #include <math.h>
 
@@ -203,16 +203,45 @@ __global__ void k_pair_tables(const PairTile *__restrict__ tiles, const PairSlot
     }
 }
 
-// The two D products of a rotation of degree n on one tile of columns: p_b[s], q_b[s] are
-// the B operands u_m + u_-m and u_m - u_-m of inner class b (m = b + 2c, c = 4s + l/16);
+// The D operands of one degree, [a][b][row tile][inner step]: loaded once per wave, used by
+// both products (and by every tile of a segment).  KS: inner steps, (n >> 3) + 1.
+template <int RT, int KS>
+struct DFrag {
+    double d[2][2][RT][KS];
+    __device__ __forceinline__ void load(const double *__restrict__ D, int lane) {
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int r = 0; r < RT; ++r)
+#pragma unroll
+                    for (int s = 0; s < KS; ++s) d[a][b][r][s] = D[(((a * 2 + b) * RT + r) * KS + s) * 64 + lane];
+    }
+};
+
+// The two D products of a rotation of degree n on one tile of columns: load(b, c, p, q)
+// gives u_m + u_-m and u_m - u_-m of inner class b at m = b + 2c (this lane's column);
 // on return vp[a][i], vm[a][i] (i = 4 rt + v) are the results at +-(a + 2r), r = 16 rt +
-// 4 v + l/16, without the outer phases.  th: e^{-ij theta} of this lane's pair.
-template <int RT, typename Load>
-__device__ __forceinline__ void rotate(int n, const double *__restrict__ D, const double2 *__restrict__ th, int lane,
+// 4 v + l/16, without the outer phases.  th: e^{-ij theta} of this lane's pair.  The
+// inner steps are unrolled: all loads of a step chain are in flight before its products.
+template <int RT, int KS, typename Load>
+__device__ __forceinline__ void rotate(int n, const DFrag<RT, KS> &D, const double2 *__restrict__ th, int lane,
                                        Load load, double (&vp)[2][4 * RT], double (&vm)[2][4 * RT]) {
-    const int ks = pair_ks(n), lk = lane >> 4;
+    const int lk = lane >> 4;
     const double sg = (lane & 1) ? -1.0 : 1.0;   // im lane
     const double sn = (n & 1) ? -1.0 : 1.0;
+    const bool odd = n & 1;
+    double e[KS][2], o[KS][2];
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            double p, q;
+            load(b, 4 * s + lk, p, q);
+            e[s][b] = odd ? q : p;  // n + a even takes p
+            o[s][b] = odd ? p : q;
+        }
     dv4 acc[2][2][RT];
 #pragma unroll
     for (int a = 0; a < 2; ++a)
@@ -220,37 +249,33 @@ __device__ __forceinline__ void rotate(int n, const double *__restrict__ D, cons
         for (int b = 0; b < 2; ++b)
 #pragma unroll
             for (int r = 0; r < RT; ++r) acc[a][b][r] = dv4{0, 0, 0, 0};
-    const bool odd = n & 1;
-    for (int s = 0; s < ks; ++s)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            double p, q;
-            load(b, 4 * s + lk, p, q);
-            const double e = odd ? q : p, o = odd ? p : q;  // n + a even takes p
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
 #pragma unroll
             for (int r = 0; r < RT; ++r) {
-                acc[0][b][r] = mma(D[((b * RT + r) * ks + s) * 64 + lane], e, acc[0][b][r]);
-                acc[1][b][r] = mma(D[(((2 + b) * RT + r) * ks + s) * 64 + lane], o, acc[1][b][r]);
+                acc[0][b][r] = mma(D.d[0][b][r][s], e[s][b], acc[0][b][r]);
+                acc[1][b][r] = mma(D.d[1][b][r][s], o[s][b], acc[1][b][r]);
             }
-        }
-    double P[2][4 * RT], Q[2][4 * RT];
+    // inner step s of the second product is value v = s % 4 of row tile s / 4: the first KS
+    // values hold all of n
+    double P[2][KS], Q[2][KS];
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int r = 0; r < RT; ++r)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int j = a + 2 * (16 * r + 4 * v + lk);
-                const double A = acc[a][0][r][v], B = acc[a][1][r][v];
-                const double x = A + B, y = sn * (A - B);       // v_j, v_-j
-                const double2 e = th[j < n ? j : n];            // cos, -sin
-                const double xo = __shfl_xor(x, 1, 64), yo = __shfl_xor(y, 1, 64);
-                // e^{-ij theta} v_j and e^{ij theta} v_-j: this lane's part from both
-                const double wp = e.x * x - sg * e.y * xo;
-                const double wm = e.x * y + sg * e.y * yo;
-                P[a][4 * r + v] = j == 0 ? wp : wp + wm;
-                Q[a][4 * r + v] = j == 0 ? 0.0 : wp - wm;
-            }
+        for (int s = 0; s < KS; ++s) {
+            const int j = a + 2 * (4 * s + lk);
+            const double A = acc[a][0][s >> 2][s & 3], B = acc[a][1][s >> 2][s & 3];
+            const double x = A + B, y = sn * (A - B);       // v_j, v_-j
+            const double2 f = th[j < n ? j : n];            // cos, -sin
+            const double xo = __shfl_xor(x, 1, 64), yo = __shfl_xor(y, 1, 64);
+            // e^{-ij theta} v_j and e^{ij theta} v_-j: this lane's part from both
+            const double wp = f.x * x - sg * f.y * xo;
+            const double wm = f.x * y + sg * f.y * yo;
+            P[a][s] = j == 0 ? wp : wp + wm;
+            Q[a][s] = j == 0 ? 0.0 : wp - wm;
+        }
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -259,18 +284,16 @@ __device__ __forceinline__ void rotate(int n, const double *__restrict__ D, cons
             for (int r = 0; r < RT; ++r) acc[a][b][r] = dv4{0, 0, 0, 0};
     // D_jk = (-1)^{j+k} D_kj: the same operands, minus where the parities differ
 #pragma unroll
-    for (int s = 0; s < 4 * RT; ++s) {
-        if (s >= ks) break;
+    for (int s = 0; s < KS; ++s)
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
-            const double e = odd ? Q[b][s] : P[b][s], o = odd ? P[b][s] : Q[b][s];
+            const double ev = odd ? Q[b][s] : P[b][s], ov = odd ? P[b][s] : Q[b][s];
 #pragma unroll
             for (int r = 0; r < RT; ++r) {
-                acc[0][b][r] = mma(D[((b * RT + r) * ks + s) * 64 + lane], e, acc[0][b][r]);
-                acc[1][b][r] = mma(D[(((2 + b) * RT + r) * ks + s) * 64 + lane], o, acc[1][b][r]);
+                acc[0][b][r] = mma(D.d[0][b][r][s], ev, acc[0][b][r]);
+                acc[1][b][r] = mma(D.d[1][b][r][s], ov, acc[1][b][r]);
             }
         }
-    }
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -285,53 +308,46 @@ __device__ __forceinline__ void rotate(int n, const double *__restrict__ D, cons
 }
 
 // Forward rotation: wave per (tile, degree), x -> Y.
-template <int RT>
-__global__ __launch_bounds__(256) void k_pair_fwd(const PairTile *__restrict__ tiles,
-                                                  const PairSlot *__restrict__ slots, int t0, int ntiles, int n0,
-                                                  const double *__restrict__ delta, const double2 *__restrict__ tab,
-                                                  const double2 *__restrict__ src, int64_t src_stride,
-                                                  double *__restrict__ Y, int64_t y_stride) {
-    const int ti = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (ti >= ntiles) return;
-    const PairTile T = tiles[t0 + ti];
-    const int n = n0 + blockIdx.y;
-    if (n > T.Ls) return;
+template <int RT, int KS>
+__device__ __forceinline__ void pair_fwd(int n, const PairTile &T, const PairSlot *__restrict__ slots,
+                                         const double *__restrict__ delta, const double2 *__restrict__ tab,
+                                         const double2 *__restrict__ src, double *__restrict__ y) {
     const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
     const int part = li & 3;
-    const PairSlot S = slots[4 * (t0 + ti) + (li >> 2)];
+    DFrag<RT, KS> D;
+    D.load(delta + delta_off(n), lane);
+    const PairSlot S = slots[li >> 2];
     const double2 *ph = tab + T.off_tab + (int64_t)(li >> 2) * T.tabw;
     const double2 *th = ph + T.NL + 1;
     const bool live = S.src >= 0 && n <= S.Ls;
-    const double2 *xa = src + blockIdx.z * src_stride + (live ? S.src + n * n - 1 + n : 0);
-    const int64_t nb = live ? (int64_t)S.Ls * (S.Ls + 2) : 0;
-    const double2 *xb = xa + nb;
+    const double2 *xa = src + (live ? S.src + n * n - 1 + n : 0);
+    const double2 *xb = xa + (live ? (int64_t)S.Ls * (S.Ls + 2) : 0);
     const double s2 = part < 2 ? 1.0 : -1.0;
     const bool im = part & 1;
     double vp[2][4 * RT], vm[2][4 * RT];
-    rotate<RT>(n, delta + delta_off(n), th, lane,
-               [&](int b, int c, double &p, double &q) {
-                   const int m = b + 2 * c;
-                   if (!live || m > n) {
-                       p = q = 0.0;
-                       return;
-                   }
-                   const double2 f = ph[m], a0 = xa[m], b0 = xb[m], a1 = xa[-m], b1 = xb[-m];
-                   const double xr = a0.x + s2 * b0.x, xi = a0.y + s2 * b0.y;
-                   const double yr = a1.x + s2 * b1.x, yi = a1.y + s2 * b1.y;
-                   const double up = im ? f.x * xi + f.y * xr : f.x * xr - f.y * xi;
-                   const double um = im ? f.x * yi - f.y * yr : f.x * yr + f.y * yi;
-                   p = m == 0 ? up : up + um;
-                   q = m == 0 ? 0.0 : up - um;
-               },
-               vp, vm);
+    rotate<RT, KS>(n, D, th, lane,
+                   [&](int b, int c, double &p, double &q) {
+                       const int m = b + 2 * c;
+                       if (!live || m > n) {
+                           p = q = 0.0;
+                           return;
+                       }
+                       const double2 f = ph[m], a0 = xa[m], b0 = xb[m], a1 = xa[-m], b1 = xb[-m];
+                       const double xr = a0.x + s2 * b0.x, xi = a0.y + s2 * b0.y;
+                       const double yr = a1.x + s2 * b1.x, yi = a1.y + s2 * b1.y;
+                       const double up = im ? f.x * xi + f.y * xr : f.x * xr - f.y * xi;
+                       const double um = im ? f.x * yi - f.y * yr : f.x * yr + f.y * yi;
+                       p = m == 0 ? up : up + um;
+                       q = m == 0 ? 0.0 : up - um;
+                   },
+                   vp, vm);
     const int K = T.K;
-    double *y = Y + blockIdx.z * y_stride + T.off_y;
     const int row = yrow(n, 0, K);
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int i = 0; i < 4 * RT; ++i) {
-            const int r = 16 * (i >> 2) + 4 * (i & 3) + lk;
+        for (int i = 0; i < KS; ++i) {
+            const int r = 4 * i + lk;
             const int k = a + 2 * r;
             if (k > n || k > K) continue;
             const double sr = (r & 1) ? -1.0 : 1.0;
@@ -346,39 +362,72 @@ __global__ __launch_bounds__(256) void k_pair_fwd(const PairTile *__restrict__ t
         }
 }
 
+// RT = 1: degrees 1..31, RT = 2: 32..63.
+template <int RT>
+__global__ __launch_bounds__(256) void k_pair_fwd(const PairTile *__restrict__ tiles,
+                                                  const PairSlot *__restrict__ slots, int t0, int ntiles, int n0,
+                                                  const double *__restrict__ delta, const double2 *__restrict__ tab,
+                                                  const double2 *__restrict__ src, int64_t src_stride,
+                                                  double *__restrict__ Y, int64_t y_stride) {
+    const int ti = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+    if (ti >= ntiles) return;
+    const PairTile T = tiles[t0 + ti];
+    const int n = n0 + blockIdx.y;
+    if (n > T.Ls) return;
+    const PairSlot *sl = slots + 4 * (t0 + ti);
+    const double2 *x = src + blockIdx.z * src_stride;
+    double *y = Y + blockIdx.z * y_stride + T.off_y;
+    switch (n >> 3) {
+        case 4 * (RT - 1): pair_fwd<RT, 4 * RT - 3>(n, T, sl, delta, tab, x, y); break;
+        case 4 * (RT - 1) + 1: pair_fwd<RT, 4 * RT - 2>(n, T, sl, delta, tab, x, y); break;
+        case 4 * (RT - 1) + 2: pair_fwd<RT, 4 * RT - 1>(n, T, sl, delta, tab, x, y); break;
+        default: pair_fwd<RT, 4 * RT>(n, T, sl, delta, tab, x, y);
+    }
+}
+
 // Coaxial shift: wave per (tile, order m), Y -> Z at k = +-m.  z_+(m) and z_-(-m) take
-// P_m, z_+(-m) and z_-(m) take Q_m, so each of the two products has 16 columns.
+// P_m, z_+(-m) and z_-(m) take Q_m, so each of the two products has 16 columns.  The tiles
+// of a block share one node set: its matrices pass through LDS one node tile at a time (read
+// per wave from L1 they took 8 cache accesses per 64-cycle product and bounded the kernel:
+// 5740 tiles of orders 9-18 in 343 us; through LDS, rows read whole, 238 us).
 // Node-set matrices at off_q: for [m][P, Q]: A1[Q/16][S1][64] (rows
 // nodes, inner degrees) and after all of them A2[UT][Q/4][64] (rows degrees, inner nodes).
-template <int UT>
-__global__ __launch_bounds__(256) void k_pair_axial(const PairTile *__restrict__ tiles,
-                                                    const PairSlot *__restrict__ slots, int t0, int ntiles, int NL,
+// KS, UT: inner steps of four source degrees and tiles of 16 target degrees that the launch holds.
+template <int UT, int KS>
+__global__ __launch_bounds__(512) void k_pair_axial(const PairTile *__restrict__ tiles,
+                                                    const PairSlot *__restrict__ slots,
+                                                    const PairGroup *__restrict__ groups,
+                                                    const int32_t *__restrict__ order, int NL,
                                                     const double *__restrict__ quad, const double2 *__restrict__ tab,
                                                     const double2 *__restrict__ wax, const double *__restrict__ Y,
                                                     int64_t y_stride, double *__restrict__ Z, int64_t z_stride) {
-    const int ti = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (ti >= ntiles) return;
-    const PairTile T = tiles[t0 + ti];
+    __shared__ double As[2 * KS + 8 * UT][64];  // [type][step] of A1, then [type][t][v] of A2
+    const PairGroup G = groups[blockIdx.x];
     const int m = blockIdx.y;
-    if (m > T.K) return;
+    if (m > G.K) return;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+    const int ti = order[G.first + (wv < G.count ? wv : 0)];
+    const PairTile T = tiles[ti];
+    const bool live = wv < G.count && m <= T.K;
     const int K = T.K, Ls = T.Ls, Lt = T.Lt;
     const int q0 = m < 1 ? 1 : m;
     const double *y = Y + blockIdx.z * y_stride + T.off_y;
     double *z = Z + blockIdx.z * z_stride + T.off_z;
-    if (T.Q == 0) {
-        // close pairs: 16 rows of each of the four slots at a time, from their own tables
-        const PairSlot S = slots[4 * (t0 + ti) + lk];
-        const int ncol = S.Ls - q0 + 1;
-        const bool live = S.src >= 0 && m <= S.K;
-        const double2 *Pb = wax + S.off_ax + (live ? ax_off(m, Lt, S.Ls, S.K) : 0);
-        const double2 *Qb = Pb + (live ? ax_block(m, Lt, S.Ls) : 0);
+    if (G.Q == 0) {
+        if (!live) return;
+        // close pairs: 16 target degrees of each of the four slots at a time, from their own
+        // tables, which hold P(nu, n) = P(n, nu) with the target degree running fastest
+        const PairSlot S = slots[4 * ti + lk];
+        const int ncol = Lt - q0 + 1;
+        const bool on = S.src >= 0 && m <= S.K;
+        const double2 *Pb = wax + S.off_ax + (on ? ax_off(m, S.Ls, Lt, S.K) : 0) - q0;
+        const double2 *Qb = Pb + (on ? ax_block(m, S.Ls, Lt) : 0);
         for (int n = q0 + li; n <= Lt; n += 16) {
             double zr[4] = {0, 0, 0, 0}, zi[4] = {0, 0, 0, 0};  // z_+(m), z_-(m), z_+(-m), z_-(-m)
-            if (live) {
-                const double2 *pr = Pb + (int64_t)(n - q0) * ncol, *qr = Qb + (int64_t)(n - q0) * ncol;
+            if (on) {
                 for (int nu = q0; nu <= S.Ls; ++nu) {
-                    const double2 pv = pr[nu - q0], qv = qr[nu - q0];
+                    const double2 pv = Pb[(nu - q0) * ncol + n], qv = Qb[(nu - q0) * ncol + n];
                     const double2 *yp = (const double2 *)(y + (int64_t)yrow(nu, m, K) * 16 + 4 * lk);
                     const double2 *ym = (const double2 *)(y + (int64_t)yrow(nu, -m, K) * 16 + 4 * lk);
                     const double2 v[4] = {yp[0], yp[1], ym[0], ym[1]};
@@ -401,46 +450,69 @@ __global__ __launch_bounds__(256) void k_pair_axial(const PairTile *__restrict__
         }
         return;
     }
-    const int part = li & 3;
+    const bool plus = (li & 3) < 2;  // a part of x_+
     const double sg = (li & 1) ? 1.0 : -1.0;
     const double2 *tq = tab + T.off_tab + (int64_t)(li >> 2) * T.tabw + 2 * (T.NL + 1);
-    const int QT = T.Q >> 4, S1 = (NL + 3) / 4, UTN = (NL + 15) / 16;
-    const double *A1 = quad + T.off_q + (int64_t)m * 2 * QT * S1 * 64 + lane;
-    const double *A2 = quad + T.off_q + (int64_t)(NL + 1) * 2 * QT * S1 * 64 +
-                       (int64_t)m * 2 * UTN * 4 * QT * 64 + lane;
-    // order of k this lane reads and writes for P; the other one for Q
-    const int kP = part < 2 ? m : -m, kQ = -kP;
-    const int ks = (Ls - q0 + 4) / 4;
+    const int QT = G.Q >> 4, S1 = (NL + 3) / 4, UTN = (NL + 15) / 16;
+    const double *A1 = quad + G.off_q + (int64_t)m * 2 * QT * S1 * 64;
+    const double *A2 = quad + G.off_q + (int64_t)(NL + 1) * 2 * QT * S1 * 64 + (int64_t)m * 2 * UTN * 4 * QT * 64;
+    const int ks = live ? (Ls - q0 + 4) / 4 : 0, ut = live ? (Lt - q0 + 16) / 16 : 0;
+    const int ksg = min((G.Ls - q0 + 4) / 4, KS), utg = min((G.Lt - q0 + 16) / 16, UT);  // of the block
+    // the source columns stay in registers for all node tiles
+    double bp[KS], bq[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+        bp[s] = bq[s] = 0.0;
+        if (s < ks) {
+            const int nu = q0 + 4 * s + lk;
+            const int row = yrow(nu <= Ls ? nu : Ls, 0, K);
+            double a = y[(int64_t)(row + m) * 16 + li], b = y[(int64_t)(row - m) * 16 + li];
+            a = nu <= Ls ? a : 0.0;
+            b = nu <= Ls ? b : 0.0;
+            bp[s] = plus ? a : b;
+            bq[s] = plus ? b : a;
+        }
+    }
     dv4 u[2][UT];
 #pragma unroll
     for (int t = 0; t < UT; ++t) u[0][t] = u[1][t] = dv4{0, 0, 0, 0};
     for (int qt = 0; qt < QT; ++qt) {
-        dv4 g[2] = {dv4{0, 0, 0, 0}, dv4{0, 0, 0, 0}};
-        for (int s = 0; s < ks; ++s) {
-            const int nu = q0 + 4 * s + lk;
-            const bool ok = nu <= Ls;
-            const int nc = ok ? nu : Ls;
-            const int row = yrow(nc, 0, K);
-            double bp = y[(int64_t)(row + kP) * 16 + li], bq = y[(int64_t)(row + kQ) * 16 + li];
-            bp = ok ? bp : 0.0;
-            bq = ok ? bq : 0.0;
-            g[0] = mma(A1[(int64_t)(qt * S1 + s) * 64], bp, g[0]);
-            g[1] = mma(A1[(int64_t)((QT + qt) * S1 + s) * 64], bq, g[1]);
-        }
+        double2 tv[4];
+        if (live)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const double2 tv = tq[16 * qt + 4 * v + lk];
+            for (int v = 0; v < 4; ++v) tv[v] = tq[16 * qt + 4 * v + lk];
+        __syncthreads();
+        for (int i = threadIdx.x; i < 2 * ksg * 64; i += blockDim.x) {
+            const int ty = i >= ksg * 64, r = (i >> 6) - ty * ksg;
+            As[ty * KS + r][i & 63] = A1[(int64_t)((ty * QT + qt) * S1 + r) * 64 + (i & 63)];
+        }
+        for (int i = threadIdx.x; i < 8 * utg * 64; i += blockDim.x) {
+            const int f = i >> 6, v = f & 3, tt = f >> 2;  // tt = ty * utg + t
+            const int ty = tt >= utg, t = tt - ty * utg;
+            As[2 * KS + (ty * UT + t) * 4 + v][i & 63] =
+                A2[((int64_t)(ty * UTN + t) * 4 * QT + 4 * qt + v) * 64 + (i & 63)];
+        }
+        __syncthreads();
+        if (!live) continue;
+        dv4 g[2] = {dv4{0, 0, 0, 0}, dv4{0, 0, 0, 0}};
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+            if (s < ks) {
+                g[0] = mma(As[s][lane], bp[s], g[0]);
+                g[1] = mma(As[KS + s][lane], bq[s], g[1]);
+            }
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
 #pragma unroll
             for (int ty = 0; ty < 2; ++ty) {
                 const double x = g[ty][v], xo = __shfl_xor(x, 1, 64);
-                const double b = tv.x * x + sg * tv.y * xo;
+                const double b = tv[v].x * x + sg * tv[v].y * xo;
 #pragma unroll
                 for (int t = 0; t < UT; ++t)
-                    if (q0 + 16 * t <= Lt)
-                        u[ty][t] = mma(A2[((int64_t)(ty * UTN + t) * 4 * QT + 4 * qt + v) * 64], b, u[ty][t]);
+                    if (t < ut) u[ty][t] = mma(As[2 * KS + (ty * UT + t) * 4 + v][lane], b, u[ty][t]);
             }
-        }
     }
+    if (!live) return;
 #pragma unroll
     for (int t = 0; t < UT; ++t)
 #pragma unroll
@@ -448,65 +520,60 @@ __global__ __launch_bounds__(256) void k_pair_axial(const PairTile *__restrict__
             const int n = q0 + 16 * t + 4 * v + lk;
             if (n > Lt) continue;
             const int row = yrow(n, 0, K);
-            z[(int64_t)(row + kP) * 16 + li] = u[0][t][v];
-            if (m > 0) z[(int64_t)(row + kQ) * 16 + li] = u[1][t][v];
+            z[(int64_t)(row + m) * 16 + li] = plus ? u[0][t][v] : u[1][t][v];
+            if (m > 0) z[(int64_t)(row - m) * 16 + li] = plus ? u[1][t][v] : u[0][t][v];
         }
 }
 
 // Back rotation of a segment's tiles and their sum: wave per (segment, degree), Z -> W.
-template <int RT>
-__global__ __launch_bounds__(256) void k_pair_back(const PairTile *__restrict__ tiles,
-                                                   const PairSeg *__restrict__ segs, int s0, int nsegs, int n0,
-                                                   const double *__restrict__ delta, const double2 *__restrict__ tab,
-                                                   const double *__restrict__ Z, int64_t z_stride,
-                                                   double2 *__restrict__ W, int64_t w_stride) {
-    const int si = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (si >= nsegs) return;
-    const PairSeg G = segs[s0 + si];
-    const int n = n0 + blockIdx.y;
-    if (n > G.Lt) return;
+template <int RT, int KS>
+__device__ __forceinline__ void pair_back(int n, const PairSeg &G, const PairTile *__restrict__ tiles,
+                                          const double *__restrict__ delta, const double2 *__restrict__ tab,
+                                          const double *__restrict__ Z, double *__restrict__ w) {
     const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
     const int part = li & 3;
     const bool im = part & 1;
-    double op[2][4 * RT], om[2][4 * RT];  // this lane's part at +-m, summed over the tiles
+    DFrag<RT, KS> D;
+    D.load(delta + delta_off(n), lane);
+    double op[2][KS], om[2][KS];  // this lane's part at +-m, summed over the tiles
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int i = 0; i < 4 * RT; ++i) op[a][i] = om[a][i] = 0.0;
+        for (int i = 0; i < KS; ++i) op[a][i] = om[a][i] = 0.0;
     for (int ti = G.t_begin; ti < G.t_end; ++ti) {
         const PairTile T = tiles[ti];
         const int K = T.K;
         const double2 *ph = tab + T.off_tab + (int64_t)(li >> 2) * T.tabw;
         const double2 *th = ph + T.NL + 1;
-        const double *z = Z + blockIdx.z * z_stride + T.off_z + (int64_t)yrow(n, 0, K) * 16;
+        const double *z = Z + T.off_z + (int64_t)yrow(n, 0, K) * 16;
         double vp[2][4 * RT], vm[2][4 * RT];
-        rotate<RT>(n, delta + delta_off(n), th, lane,
-                   [&](int b, int c, double &p, double &q) {
-                       const int k = b + 2 * c;
-                       if (k > n || k > K) {
-                           p = q = 0.0;
-                           return;
-                       }
-                       const double sr = (c & 1) ? -1.0 : 1.0;
-                       double up, um;
-                       if (b == 0) {  // i^{+-k} = (-1)^c
-                           up = sr * z[k * 16 + li];
-                           um = sr * z[-k * 16 + li];
-                       } else {       // +-i (-1)^c: the other part
-                           const double f = im ? sr : -sr;
-                           up = f * z[k * 16 + (li ^ 1)];
-                           um = -f * z[-k * 16 + (li ^ 1)];
-                       }
-                       p = k == 0 ? up : up + um;
-                       q = k == 0 ? 0.0 : up - um;
-                   },
-                   vp, vm);
+        rotate<RT, KS>(n, D, th, lane,
+                       [&](int b, int c, double &p, double &q) {
+                           const int k = b + 2 * c;
+                           if (k > n || k > K) {
+                               p = q = 0.0;
+                               return;
+                           }
+                           const double sr = (c & 1) ? -1.0 : 1.0;
+                           double up, um;
+                           if (b == 0) {  // i^{+-k} = (-1)^c
+                               up = sr * z[k * 16 + li];
+                               um = sr * z[-k * 16 + li];
+                           } else {       // +-i (-1)^c: the other part
+                               const double f = im ? sr : -sr;
+                               up = f * z[k * 16 + (li ^ 1)];
+                               um = -f * z[-k * 16 + (li ^ 1)];
+                           }
+                           p = k == 0 ? up : up + um;
+                           q = k == 0 ? 0.0 : up - um;
+                       },
+                       vp, vm);
         const double sg = im ? -1.0 : 1.0;
 #pragma unroll
         for (int a = 0; a < 2; ++a)
 #pragma unroll
-            for (int i = 0; i < 4 * RT; ++i) {
-                const int m = a + 2 * (16 * (i >> 2) + 4 * (i & 3) + lk);
+            for (int i = 0; i < KS; ++i) {
+                const int m = a + 2 * (4 * i + lk);
                 const double2 f = ph[m < n ? m : n];
                 const double x = vp[a][i], y = vm[a][i];
                 const double xo = __shfl_xor(x, 1, 64), yo = __shfl_xor(y, 1, 64);
@@ -518,12 +585,11 @@ __global__ __launch_bounds__(256) void k_pair_back(const PairTile *__restrict__ 
     }
     // sum of the four slots, then a = (w_+ + w_-)/2, b = (w_+ - w_-)/2
     const int nent = G.Lt * (G.Lt + 2);
-    double *w = (double *)(W + blockIdx.z * w_stride + G.off_w);
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int i = 0; i < 4 * RT; ++i) {
-            const int m = a + 2 * (16 * (i >> 2) + 4 * (i & 3) + lk);
+        for (int i = 0; i < KS; ++i) {
+            const int m = a + 2 * (4 * i + lk);
 #pragma unroll
             for (int d = 0; d < 2; ++d) {
                 double x = d == 0 ? op[a][i] : om[a][i];
@@ -536,6 +602,27 @@ __global__ __launch_bounds__(256) void k_pair_back(const PairTile *__restrict__ 
                 w[2 * (int64_t)e + (part & 1)] = r;
             }
         }
+}
+
+template <int RT>
+__global__ __launch_bounds__(256) void k_pair_back(const PairTile *__restrict__ tiles,
+                                                   const PairSeg *__restrict__ segs, int s0, int nsegs, int n0,
+                                                   const double *__restrict__ delta, const double2 *__restrict__ tab,
+                                                   const double *__restrict__ Z, int64_t z_stride,
+                                                   double2 *__restrict__ W, int64_t w_stride) {
+    const int si = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+    if (si >= nsegs) return;
+    const PairSeg G = segs[s0 + si];
+    const int n = n0 + blockIdx.y;
+    if (n > G.Lt) return;
+    const double *z = Z + blockIdx.z * z_stride;
+    double *w = (double *)(W + blockIdx.z * w_stride + G.off_w);
+    switch (n >> 3) {
+        case 4 * (RT - 1): pair_back<RT, 4 * RT - 3>(n, G, tiles, delta, tab, z, w); break;
+        case 4 * (RT - 1) + 1: pair_back<RT, 4 * RT - 2>(n, G, tiles, delta, tab, z, w); break;
+        case 4 * (RT - 1) + 2: pair_back<RT, 4 * RT - 1>(n, G, tiles, delta, tab, z, w); break;
+        default: pair_back<RT, 4 * RT>(n, G, tiles, delta, tab, z, w);
+    }
 }
 
 // dst += the partial sums of a target's segments, in their order.
@@ -592,20 +679,24 @@ void launch_pair_fwd(const PairTile *tiles, const PairSlot *slots, int t0, int n
                            ntiles, 32, delta, tab, src, src_stride, Y, y_stride);
 }
 
-void launch_pair_axial(const PairTile *tiles, const PairSlot *slots, int t0, int ntiles, int max_K, int max_Lt, int NL,
-                       const double *quad, const double2 *tab, const double2 *wax, const double *Y, int64_t y_stride,
-                       double *Z, int64_t z_stride, int nrhs, hipStream_t s) {
-    if (ntiles <= 0) return;
-    const dim3 grid((ntiles + 3) / 4, max_K + 1, nrhs);
-    if (max_Lt <= 16)
-        hipLaunchKernelGGL(k_pair_axial<1>, grid, dim3(256), 0, s, tiles, slots, t0, ntiles, NL, quad, tab, wax, Y,
-                           y_stride, Z, z_stride);
-    else if (max_Lt <= 32)
-        hipLaunchKernelGGL(k_pair_axial<2>, grid, dim3(256), 0, s, tiles, slots, t0, ntiles, NL, quad, tab, wax, Y,
-                           y_stride, Z, z_stride);
+void launch_pair_axial(const PairTile *tiles, const PairSlot *slots, const PairGroup *groups, int ngroups,
+                       const int32_t *order, int waves, int max_K, int max_L, int NL, const double *quad,
+                       const double2 *tab, const double2 *wax, const double *Y, int64_t y_stride, double *Z,
+                       int64_t z_stride, int nrhs, hipStream_t s) {
+    if (ngroups <= 0) return;
+    const dim3 grid(ngroups, max_K + 1, nrhs);
+#define IFS_PAIR_AXIAL(UT, KS)                                                                                       \
+    hipLaunchKernelGGL((k_pair_axial<UT, KS>), grid, dim3(64 * waves), 0, s, tiles, slots, groups, order, NL, quad, tab, \
+                       wax, Y, y_stride, Z, z_stride)
+    if (max_L <= 16)
+        IFS_PAIR_AXIAL(1, 4);
+    else if (max_L <= 24)
+        IFS_PAIR_AXIAL(2, 6);
+    else if (max_L <= 32)
+        IFS_PAIR_AXIAL(2, 8);
     else
-        hipLaunchKernelGGL(k_pair_axial<4>, grid, dim3(256), 0, s, tiles, slots, t0, ntiles, NL, quad, tab, wax, Y,
-                           y_stride, Z, z_stride);
+        IFS_PAIR_AXIAL(4, 16);
+#undef IFS_PAIR_AXIAL
 }
 
 void launch_pair_back(const PairTile *tiles, const PairSeg *segs, int s0, int nsegs, int max_Lt, const double *delta,
