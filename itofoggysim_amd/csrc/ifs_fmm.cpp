@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "ifs_engine.h"
+#include "ifs_leaf.h"
 #include "ifs_pair.h"
 #include "ifs_pw.h"
 #include "ifs_tree.h"
@@ -50,6 +51,7 @@ struct Fmm {
     DevBuf C, D;                                // multipole / local pools
     int64_t nC = 0;
     Batch p2m, l2p, p2p;
+    Leaf leaf;                                  // P2M and L2P by samples, where the level is large enough
     PairBatch pair;                             // near field, unless the pair kernels do not apply (p2p)
     std::vector<ClassBatch> m2m, m2l, l2l;      // indexed by level
     std::vector<PwLevel> pw;                    // M2L in the plane-wave basis, by level
@@ -392,8 +394,16 @@ int build(ifs_ctx *c, Fmm **out) {
         }
         if ((rc = class_batches_prepare(c, cls))) goto fail;
     }
-    if ((rc = fin(f->p2m, "p2m"))) goto fail;
-    if ((rc = fin(f->l2p, "l2p"))) goto fail;
+    if (!f->l2p.tasks.empty() && leaf_worth(c, LL.L, (int)LL.boxes.size(), ns)) {
+        batch_cost(f->p2m, c->flops_mv, c->bytes_mv);
+        batch_cost(f->l2p, c->flops_mv, c->bytes_mv);
+        if ((rc = leaf_build(c, f->leaf, f->p2m.tasks, f->l2p.tasks, LL.L, (int)LL.boxes.size(), LL.off))) goto fail;
+        f->p2m.tasks.clear();
+        f->l2p.tasks.clear();
+    } else {
+        if ((rc = fin(f->p2m, "p2m"))) goto fail;
+        if ((rc = fin(f->l2p, "l2p"))) goto fail;
+    }
     if (pair_takes(f->p2p.tasks)) {
         batch_cost(f->p2p, c->flops_mv, c->bytes_mv);
         if ((rc = pair_finalize(c, f->pair, f->p2p.tasks, "p2p"))) goto fail;
@@ -417,7 +427,8 @@ int run(ifs_ctx *c, Fmm *f, const double2 *xh, double2 *acc, int nrhs, int64_t l
     const int64_t st = f->nC;
     launch_zero(C, f->nC * nrhs, c->stream);
     launch_zero(D, f->nC * nrhs, c->stream);
-    if ((rc = batch_run(c, f->p2m, xh, C, nrhs, ld, st))) return rc;
+    rc = f->leaf.active() ? leaf_p2m(c, f->leaf, xh, C, nrhs, ld, st) : batch_run(c, f->p2m, xh, C, nrhs, ld, st);
+    if (rc) return rc;
     for (int l = f->l_max - 1; l >= f->l_min; --l)
         if ((rc = class_batch_run(c, f->m2m[l], C, C, nrhs, prec))) return rc;
     for (int l = f->l_min; l <= f->l_max; ++l) {
@@ -427,7 +438,8 @@ int run(ifs_ctx *c, Fmm *f, const double2 *xh, double2 *acc, int nrhs, int64_t l
         if ((rc = class_batch_run(c, f->m2l[l], C, D, nrhs, prec))) return rc;
         if (l > f->l_min && (rc = class_batch_run(c, f->l2l[l], D, D, nrhs, prec))) return rc;
     }
-    if ((rc = batch_run(c, f->l2p, D, acc, nrhs, st, ld))) return rc;
+    rc = f->leaf.active() ? leaf_l2p(c, f->leaf, D, acc, nrhs, st, ld) : batch_run(c, f->l2p, D, acc, nrhs, st, ld);
+    if (rc) return rc;
     if (f->pair.active()) return pair_run(c, f->pair, xh, acc, nrhs, ld, ld);
     if ((rc = batch_run(c, f->p2p, xh, acc, nrhs, ld, ld))) return rc;
     return IFS_OK;
@@ -444,6 +456,7 @@ uint64_t buffers_sig(Fmm *f) {
             buf(*d);
     mix(pair_sig(f->pair));
     for (auto &P : f->pw) mix(pw_sig(P));
+    mix(leaf_sig(f->leaf));
     std::vector<const std::vector<ClassBatch> *> all = {&f->m2m, &f->m2l, &f->l2l};
     for (auto &v : f->rem) all.push_back(&v);
     for (const auto *v : all)

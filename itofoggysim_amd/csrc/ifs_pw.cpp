@@ -85,9 +85,9 @@ bool pw_fits(ifs_ctx *c, int L, int nb, int nrhs) {
     return 4 * L + 1 <= kPwMaxN - 96 && 64.0 * (double)x_size(L) * nb * nrhs <= (double)c->ws_budget;
 }
 
-int pw_build(ifs_ctx *c, PwLevel &P, int isg) {
+int pw_grid(ifs_ctx *c, PwLevel &P, int Q2, double tdeg, int tcap, int order) {
     const int L = P.L;
-    P.Q2 = L + 1;
+    P.Q2 = Q2;
     std::vector<double> x, w;
     gauss_legendre(2 * P.Q2, x, w);
     std::vector<double> mu(2 * P.Q2);
@@ -102,7 +102,9 @@ int pw_build(ifs_ctx *c, PwLevel &P, int isg) {
         mu[P.Q2 + j] = w[j];
         const double s = std::sqrt((1.0 - mu[j]) * (1.0 + mu[j]));
         P.mF[j] = m_reach(L + 0.5, s, L);
-        P.N[j] = fft_length(2 * P.mF[j] + m_reach(2 * L + 0.5, s, 2 * L) + 1);
+        P.N[j] = fft_length(P.mF[j] + m_reach(order + 0.5, s, order) + m_reach(tdeg, s, tcap) + 1);
+        // the transform reads every order up to mF
+        if (P.N[j] < 2 * P.mF[j] + 1) P.N[j] = fft_length(2 * P.mF[j] + 1);
         auto it = lens.find(P.N[j]);
         if (it == lens.end()) {
             it = lens.emplace(P.N[j], (int)P.fft.size()).first;
@@ -121,6 +123,22 @@ int pw_build(ifs_ctx *c, PwLevel &P, int isg) {
         gpre[t] = P.SN;
         P.SN += P.N[t % P.Q2];
     }
+    int rc;
+    if ((rc = upload(P.d_mu, mu.data(), 8 * mu.size())) || (rc = upload(P.d_N, P.N.data(), 4 * P.N.size())) ||
+        (rc = upload(P.d_mF, P.mF.data(), 4 * P.mF.size())) || (rc = upload(P.d_jlo, P.jlo.data(), 4 * P.jlo.size())) ||
+        (rc = upload(P.d_fft, P.fft.data(), sizeof(PwFft) * P.fft.size())) ||
+        (rc = upload(P.d_fftof, P.fft_of.data(), 4 * P.fft_of.size())) ||
+        (rc = upload(P.d_tw, tw.data(), 16 * tw.size())) || (rc = upload(P.d_perm, perm.data(), 4 * perm.size())) ||
+        (rc = upload(P.d_gpre, gpre.data(), 8 * gpre.size())))
+        return rc;
+    return IFS_OK;
+}
+
+int pw_build(ifs_ctx *c, PwLevel &P, int isg) {
+    const int L = P.L;
+    // every degree up to 4 L
+    int rc = pw_grid(c, P, L + 1, 2 * L + 0.5, 2 * L, L);
+    if (rc) return rc;
     // offsets -> canonical table: turned and mirrored about z until x >= y >= 0, and z >= 0
     std::map<std::array<int, 3>, int> canon;
     P.map.assign(216 * 8, PwMap{0, 0, 1, 0});
@@ -168,16 +186,9 @@ int pw_build(ifs_ctx *c, PwLevel &P, int isg) {
         t[i] = P.k * (P.edge * r);
         terms[i] = pw_terms(P.k, P.edge, q[0] * q[0] + q[1] * q[1] + q[2] * q[2], L);
     }
-    int rc;
-    if ((rc = upload(P.d_mu, mu.data(), 8 * mu.size())) || (rc = upload(P.d_N, P.N.data(), 4 * P.N.size())) ||
-        (rc = upload(P.d_mF, P.mF.data(), 4 * P.mF.size())) || (rc = upload(P.d_jlo, P.jlo.data(), 4 * P.jlo.size())) ||
-        (rc = upload(P.d_src, P.src.data(), sizeof(PwSource) * P.src.size())) ||
+    if ((rc = upload(P.d_src, P.src.data(), sizeof(PwSource) * P.src.size())) ||
         (rc = upload(P.d_par, P.par.data(), sizeof(PwParent) * P.par.size())) ||
         (rc = upload(P.d_map, P.map.data(), sizeof(PwMap) * P.map.size())) ||
-        (rc = upload(P.d_fft, P.fft.data(), sizeof(PwFft) * P.fft.size())) ||
-        (rc = upload(P.d_fftof, P.fft_of.data(), 4 * P.fft_of.size())) ||
-        (rc = upload(P.d_tw, tw.data(), 16 * tw.size())) || (rc = upload(P.d_perm, perm.data(), 4 * perm.size())) ||
-        (rc = upload(P.d_gpre, gpre.data(), 8 * gpre.size())) ||
         (rc = upload(P.d_canon, dir.data(), 8 * dir.size())))
         return rc;
     // c_p of every table; t and the last terms lie behind them
@@ -251,6 +262,26 @@ int pw_plan(ifs_ctx *c, PwLevel &P, int nrhs) {
     return IFS_OK;
 }
 
+PwArg pw_arg(ifs_ctx *c, const PwLevel &P, int nrhs) {
+    PwArg a{};
+    a.L = P.L;
+    a.nbr = P.nb * nrhs;
+    a.Q2 = P.Q2;
+    a.jlo = P.d_jlo.as<int32_t>();
+    a.mF = P.d_mF.as<int32_t>();
+    a.N = P.d_N.as<int32_t>();
+    a.fftof = P.d_fftof.as<int32_t>();
+    a.fft = P.d_fft.as<PwFft>();
+    a.tw = P.d_tw.as<double2>();
+    a.perm = P.d_perm.as<int32_t>();
+    a.X = c->ws_y.as<double2>();
+    a.Xd = a.X + P.n_x;
+    a.G = a.Xd + P.n_x;
+    a.F = c->ws_z.as<double2>();
+    a.H = a.F + P.n_f;
+    return a;
+}
+
 int pw_run(ifs_ctx *c, PwLevel &P, const double2 *C, double2 *D, int nrhs, int64_t stride, int prec) {
     // right-hand sides that the workspace holds at once
     int g = nrhs;
@@ -264,22 +295,7 @@ int pw_run(ifs_ctx *c, PwLevel &P, const double2 *C, double2 *D, int nrhs, int64
         }
         hipStream_t s = c->stream;
         const int L = P.L, nc = (int)P.canon.size();
-        PwArg a{};
-        a.L = L;
-        a.nbr = P.nb * nr;
-        a.Q2 = P.Q2;
-        a.jlo = P.d_jlo.as<int32_t>();
-        a.mF = P.d_mF.as<int32_t>();
-        a.N = P.d_N.as<int32_t>();
-        a.fftof = P.d_fftof.as<int32_t>();
-        a.fft = P.d_fft.as<PwFft>();
-        a.tw = P.d_tw.as<double2>();
-        a.perm = P.d_perm.as<int32_t>();
-        a.X = c->ws_y.as<double2>();
-        a.Xd = a.X + P.n_x;
-        a.G = a.Xd + P.n_x;
-        a.F = c->ws_z.as<double2>();
-        a.H = a.F + P.n_f;
+        PwArg a = pw_arg(c, P, nr);
         const double *mu = P.d_mu.as<double>();
         double *U = P.kept ? P.own_U.as<double>() : c->ws_d.as<double>();
         double2 *T = P.kept ? P.own_T.as<double2>() : c->ws_ax.as<double2>();

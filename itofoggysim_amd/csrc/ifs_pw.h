@@ -81,6 +81,9 @@ inline bool pw_takes(int P, int L) { return P >= 2 * L || P + 1 - L >= (L + 1) /
 // Whether the level is worth it (rule and figures at the definition), given its
 // translations by plane waves.
 bool pw_worth(int L, int nb, int64_t cols);
+// The grid of a level: 2 Q2 nodes, azimuths for fields of order L and `order` under factors
+// whose azimuthal orders fall like J_m(tdeg sin(theta)), at most tcap.
+int pw_grid(ifs_ctx *c, PwLevel &P, int Q2, double tdeg, int tcap, int order);
 // parents: for every parent box its children and sources; called once per level.
 int pw_build(ifs_ctx *c, PwLevel &P, int isg);
 int pw_plan(ifs_ctx *c, PwLevel &P, int nrhs);
@@ -122,6 +125,7 @@ struct PwArg {
     const float2 *T32;     // mixed precision: T rounded to FP32 (T unused)
     double2 *X, *Xd, *G, *F, *H;
 };
+PwArg pw_arg(ifs_ctx *c, const PwLevel &P, int nrhs);
 void launch_pw_utable(int L, int Q2, int j0, int R2, int a0, int a1, int64_t ustr, const double *mu, double *U,
                       hipStream_t s);
 // terms: last p of every table; c_p = 0 beyond it

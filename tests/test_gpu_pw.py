@@ -62,6 +62,8 @@ def test_plane_wave_m2l_vs_class_products(name):
     f.close()
     d.close()
     assert "m2l_product" in ran, ran.keys()
+    if name == "two levels":  # five spheres a leaf box: P2M and L2P by samples too
+        assert "p2m_samples" in ran and "l2p_samples" in ran
     assert np.array_equal(again, b[0])
     for r in range(3):
         den = np.linalg.norm(ref[r] - X[r])
