@@ -919,11 +919,11 @@ double2 *c_xhat(ifs_ctx *c, int64_t n) { return c->k_xhat.alloc(16ull * n) ? nul
 double2 *c_stage(ifs_ctx *c, int64_t n) { return c->k_stage.alloc(16ull * n) ? nullptr : c->k_stage.as<double2>(); }
 
 int ctx_krylov_alloc(ifs_ctx *c, int restart, int64_t n, double2 **V, double2 **w, double2 **r, double2 **part,
-                     double2 **h, int nblocks) {
+                     double2 **h) {
     int rc;
     if ((rc = c->k_V.alloc(16ull * (restart + 1) * n)) || (rc = c->k_w.alloc(16ull * n)) ||
-        (rc = c->k_r.alloc(16ull * n)) || (rc = c->k_part.alloc(16ull * nblocks * (restart + 1))) ||
-        (rc = c->k_h.alloc(16ull * (restart + 1))))
+        (rc = c->k_r.alloc(16ull * n)) || (rc = c->k_part.alloc(16ull * kDotMax * (restart + 1))) ||
+        (rc = c->k_h.alloc(16ull * (2 * restart + 1))))
         return rc;
     *V = c->k_V.as<double2>();
     *w = c->k_w.as<double2>();

@@ -248,9 +248,13 @@ void launch_zero(double2 *p, int64_t n, hipStream_t s);
 void launch_scale_flat(int ns, int N, const double *snm, const double2 *x, double2 *y, int inverse, hipStream_t s);
 
 // BLAS-1 style kernels for the Krylov solver (FP64 complex).
+// `partial`: kDotMax entries per vector; launch_gemv_sub also writes |w|^2 of its result where
+// `norm2` is given.
+constexpr int kDotMax = 1024;
 void launch_dots(const double2 *V, int64_t ldv, int nv, const double2 *w, int64_t n, double2 *out, double2 *partial,
-                 int nblocks, hipStream_t s);
-void launch_gemv_sub(const double2 *V, int64_t ldv, int nv, const double2 *h, double2 *w, int64_t n, hipStream_t s);
+                 hipStream_t s);
+void launch_gemv_sub(const double2 *V, int64_t ldv, int nv, const double2 *h, double2 *w, int64_t n, double2 *norm2,
+                     double2 *partial, hipStream_t s);
 void launch_axpby(double2 a, const double2 *x, double2 b, double2 *y, int64_t n, hipStream_t s);
 void launch_scale_copy(double2 a, const double2 *x, double2 *y, int64_t n, hipStream_t s);
 void launch_gemv_add(const double2 *V, int64_t ldv, int nv, const double2 *c, double2 *x, int64_t n, hipStream_t s);

@@ -31,7 +31,7 @@ using cplx = std::complex<double>;
 namespace ifs {
 hipStream_t ctx_stream(ifs_ctx *c);
 int ctx_krylov_alloc(ifs_ctx *c, int restart, int64_t n, double2 **V, double2 **w, double2 **r, double2 **part,
-                     double2 **h, int nblocks);
+                     double2 **h);
 double2 *c_bhat(ifs_ctx *c, int64_t n);
 double2 *c_xhat(ifs_ctx *c, int64_t n);
 double2 *c_stage(ifs_ctx *c, int64_t n);
@@ -45,16 +45,33 @@ double flat_rel_residual(ifs_ctx *c, const double2 *r_hat, const double2 *b_hat,
 
 namespace {
 
-constexpr int kDotBlocks = 512;
+int fetch(hipStream_t s, const double2 *d, int cnt, cplx *out) {
+    if (hipMemcpyAsync(out, d, sizeof(double2) * cnt, hipMemcpyDeviceToHost, s) != hipSuccess) return IFS_E_HIP;
+    return hipStreamSynchronize(s) == hipSuccess ? IFS_OK : IFS_E_HIP;
+}
 
 int dots(hipStream_t s, const double2 *V, int64_t ldv, int nv, const double2 *w, int64_t n, double2 *d_out,
          double2 *d_part, std::vector<cplx> &out) {
-    launch_dots(V, ldv, nv, w, n, d_out, d_part, kDotBlocks, s);
+    launch_dots(V, ldv, nv, w, n, d_out, d_part, s);
     out.resize(nv);
-    if (hipMemcpyAsync(out.data(), d_out, sizeof(double2) * nv, hipMemcpyDeviceToHost, s) != hipSuccess)
-        return IFS_E_HIP;
-    if (hipStreamSynchronize(s) != hipSuccess) return IFS_E_HIP;
-    return IFS_OK;
+    return fetch(s, d_out, nv, out.data());
+}
+
+// Classical Gram-Schmidt with one re-orthogonalisation pass, enqueued as a whole: the
+// coefficients of both passes and |w|^2 of the result stay on the device (h: 2 nv + 1
+// entries) and are read once, by cgs2_fetch.
+void cgs2(hipStream_t s, const double2 *V, int64_t ldv, int nv, double2 *w, int64_t n, double2 *h, double2 *d_part) {
+    launch_dots(V, ldv, nv, w, n, h, d_part, s);
+    launch_gemv_sub(V, ldv, nv, h, w, n, nullptr, nullptr, s);
+    launch_dots(V, ldv, nv, w, n, h + nv, d_part, s);
+    launch_gemv_sub(V, ldv, nv, h + nv, w, n, h + 2 * nv, d_part, s);
+}
+
+// coefficients (sum of both passes) into hv, |w| returned; h on the host
+double cgs2_sum(const cplx *h, int nv, std::vector<cplx> &hv) {
+    hv.resize(nv);
+    for (int i = 0; i < nv; ++i) hv[i] = h[i] + h[nv + i];
+    return std::sqrt(std::max(0.0, h[2 * nv].real()));
 }
 
 double norm2(hipStream_t s, const double2 *w, int64_t n, double2 *d_out, double2 *d_part, int &rc) {
@@ -76,7 +93,7 @@ extern "C" int ifs_solve_device(ifs_ctx *c, const void *rhs_dev, void *x_dev, in
     auto t0 = std::chrono::steady_clock::now();
     hipStream_t s = ctx_stream(c);
     double2 *V, *w, *r, *part, *h;
-    int rc = ctx_krylov_alloc(c, m, n, &V, &w, &r, &part, &h, kDotBlocks);
+    int rc = ctx_krylov_alloc(c, m, n, &V, &w, &r, &part, &h);
     if (rc) return rc;
     const double2 *b_in = (const double2 *)rhs_dev;
     double2 *x_out = (double2 *)x_dev;
@@ -117,7 +134,7 @@ extern "C" int ifs_solve_device(ifs_ctx *c, const void *rhs_dev, void *x_dev, in
     }
     double beta = norm2(s, r, n, h, part, rc);
     if (rc) return rc;
-    std::vector<cplx> H((size_t)(m + 1) * m), g(m + 1), cs(m), sn(m), hv, hv2;
+    std::vector<cplx> H((size_t)(m + 1) * m), g(m + 1), cs(m), sn(m), hv, hh(2 * m + 1);
     int converged = beta / bnorm < opts->tol;
     int breakdown = 0;
     while (!converged && iters < opts->max_iter) {
@@ -135,18 +152,9 @@ extern "C" int ifs_solve_device(ifs_ctx *c, const void *rhs_dev, void *x_dev, in
             }
             if (rc) return rc;
             ++iters;
-            // CGS with one re-orthogonalisation pass
-            if ((rc = dots(s, V, n, j + 1, w, n, h, part, hv))) return rc;
-            if (hipMemcpyAsync(h, hv.data(), sizeof(double2) * (j + 1), hipMemcpyHostToDevice, s) != hipSuccess)
-                return IFS_E_HIP;
-            launch_gemv_sub(V, n, j + 1, h, w, n, s);
-            if ((rc = dots(s, V, n, j + 1, w, n, h, part, hv2))) return rc;
-            if (hipMemcpyAsync(h, hv2.data(), sizeof(double2) * (j + 1), hipMemcpyHostToDevice, s) != hipSuccess)
-                return IFS_E_HIP;
-            launch_gemv_sub(V, n, j + 1, h, w, n, s);
-            for (int i = 0; i <= j; ++i) hv[i] += hv2[i];
-            double hn = norm2(s, w, n, h, part, rc);
-            if (rc) return rc;
+            cgs2(s, V, n, j + 1, w, n, h, part);
+            if ((rc = fetch(s, h, 2 * j + 3, hh.data()))) return rc;
+            const double hn = cgs2_sum(hh.data(), j + 1, hv);
             // Hessenberg column j, previous rotations, new rotation
             for (int i = 0; i <= j; ++i) H[(size_t)i * m + j] = hv[i];
             H[(size_t)(j + 1) * m + j] = hn;
@@ -258,7 +266,7 @@ int solve_systems(ifs_ctx *c, const Systems &L, const double2 *bin, double2 *xou
     const int64_t ldv = (int64_t)(m + 1) * n;  // V[column][j][n]
     if ((rc = dV.alloc(16ull * ldv * nc)) || (rc = dW.alloc(16ull * n * nc)) || (rc = dR.alloc(16ull * n * nc)) ||
         (rc = dB.alloc(16ull * n * nc)) || (rc = dX.alloc(16ull * n * nc)) ||
-        (rc = dpart.alloc(16ull * kDotBlocks * (m + 1))) || (rc = dh.alloc(16ull * (m + 1))))
+        (rc = dpart.alloc(16ull * kDotMax * (m + 1))) || (rc = dh.alloc(16ull * (2 * m + 1) * ns)))
         return rc;
     double2 *V = dV.as<double2>(), *W = dW.as<double2>(), *R = dR.as<double2>(), *B = dB.as<double2>(),
             *X = dX.as<double2>(), *part = dpart.as<double2>(), *h = dh.as<double2>();
@@ -317,7 +325,7 @@ int solve_systems(ifs_ctx *c, const Systems &L, const double2 *bin, double2 *xou
     };
     std::vector<St> st(ns);
     auto active = [&](int r) { return !conv[r] && !brk[r] && iters[r] < opts->max_iter; };
-    std::vector<cplx> hv, hv2;
+    std::vector<cplx> hv, hh((size_t)(2 * m + 1) * ns);
     for (;;) {
         bool any = false;
         for (int r = 0; r < ns; ++r) any = any || active(r);
@@ -346,24 +354,18 @@ int solve_systems(ifs_ctx *c, const Systems &L, const double2 *bin, double2 *xou
                 rc = matvec_impl(c, V + (int64_t)j * n, W, 1, nc, ldv, n, kprec);
             }
             if (rc) return rc;
+            // every system's orthogonalisation is enqueued before the one read of all coefficients
+            const int hs = 2 * j + 3;
+            for (int r = 0; r < ns; ++r)
+                if (!st[r].done) cgs2(s, kv(r, 0), n, j + 1, at(W, r), L.len[r], h + (int64_t)r * hs, part);
+            if ((rc = fetch(s, h, ns * hs, hh.data()))) return rc;
             for (int r = 0; r < ns; ++r) {
                 St &S = st[r];
                 if (S.done) continue;
                 ++iters[r];
-                const double2 *Vr = kv(r, 0);
                 double2 *w = at(W, r);
                 const int64_t len = L.len[r];
-                if ((rc = dots(s, Vr, n, j + 1, w, len, h, part, hv))) return rc;
-                if (hipMemcpyAsync(h, hv.data(), sizeof(double2) * (j + 1), hipMemcpyHostToDevice, s) != hipSuccess)
-                    return IFS_E_HIP;
-                launch_gemv_sub(Vr, n, j + 1, h, w, len, s);
-                if ((rc = dots(s, Vr, n, j + 1, w, len, h, part, hv2))) return rc;
-                if (hipMemcpyAsync(h, hv2.data(), sizeof(double2) * (j + 1), hipMemcpyHostToDevice, s) != hipSuccess)
-                    return IFS_E_HIP;
-                launch_gemv_sub(Vr, n, j + 1, h, w, len, s);
-                for (int i = 0; i <= j; ++i) hv[i] += hv2[i];
-                double hn = norm2(s, w, len, h, part, rc);
-                if (rc) return rc;
+                const double hn = cgs2_sum(hh.data() + (size_t)r * hs, j + 1, hv);
                 std::vector<cplx> &H = S.H;
                 for (int i = 0; i <= j; ++i) H[(size_t)i * m + j] = hv[i];
                 H[(size_t)(j + 1) * m + j] = hn;
@@ -478,7 +480,7 @@ static int solve_block(ifs_ctx *c, int p, const double2 *bin, double2 *xout, int
     int rc;
     if ((rc = dV.alloc(16ull * n * mp1)) || (rc = dW.alloc(16ull * n * p)) || (rc = dR.alloc(16ull * n * p)) ||
         (rc = dB.alloc(16ull * n * p)) || (rc = dX.alloc(16ull * n * p)) ||
-        (rc = dpart.alloc(16ull * kDotBlocks * mp1)) || (rc = dh.alloc(16ull * mp1)))
+        (rc = dpart.alloc(16ull * kDotMax * mp1)) || (rc = dh.alloc(16ull * (2 * mp + 1))))
         return rc;
     double2 *V = dV.as<double2>(), *W = dW.as<double2>(), *R = dR.as<double2>(), *B = dB.as<double2>(),
             *X = dX.as<double2>(), *part = dpart.as<double2>(), *h = dh.as<double2>();
@@ -494,6 +496,7 @@ static int solve_block(ifs_ctx *c, int p, const double2 *bin, double2 *xout, int
         bnorm[q] = norm2(s, B + q * n, n, h, part, rc);
         if (rc) return rc;
     }
+    std::vector<cplx> hh(2 * (size_t)mp);
     auto upload = [&](const std::vector<cplx> &v, int cnt) -> int {
         return hipMemcpyAsync(h, v.data(), sizeof(double2) * cnt, hipMemcpyHostToDevice, s) == hipSuccess ? IFS_OK
                                                                                                             : IFS_E_HIP;
@@ -590,13 +593,9 @@ static int solve_block(ifs_ctx *c, int p, const double2 *bin, double2 *xout, int
             for (int q = 0; q < p; ++q) {
                 double2 *w = W + q * n;
                 cplx *hc = &H[(size_t)mp1 * (j * p + q)];
-                for (int pass = 0; pass < 2; ++pass) {
-                    std::vector<cplx> d;
-                    if ((rc = dots(s, V, n, nb, w, n, h, part, d))) return rc;
-                    if ((rc = upload(d, nb))) return rc;
-                    launch_gemv_sub(V, n, nb, h, w, n, s);
-                    for (int i = 0; i < nb; ++i) hc[i] += d[i];
-                }
+                cgs2(s, V, n, nb, w, n, h, part);
+                if ((rc = fetch(s, h, 2 * nb, hh.data()))) return rc;
+                for (int i = 0; i < nb; ++i) hc[i] += hh[i] + hh[nb + i];
             }
             // V_{j+1} T = W
             std::vector<cplx> T;
