@@ -17,6 +17,7 @@
 #include <map>
 #include <mutex>
 #include <new>
+#include <numeric>
 #include <string>
 #include <vector>
 
@@ -1051,14 +1052,19 @@ static int create_impl(ifs_ctx **out, const ifs_cluster *cl, const ifs_params *p
     c->nflat = 2LL * ns * N * (N + 2);
 
     int rc;
-    if ((rc = c->d_Leff.alloc(4 * ns)) || (rc = c->d_active.alloc(4 * ns)) || (rc = c->d_off.alloc(8 * ns)) ||
+    if ((rc = c->d_Leff.alloc(8 * ns)) || (rc = c->d_active.alloc(4 * ns)) || (rc = c->d_off.alloc(8 * ns)) ||
         (rc = c->d_snm.alloc(8ull * N * (N + 2))) || (rc = c->d_an.alloc(16ull * ns * N)) ||
         (rc = c->d_bn.alloc(16ull * ns * N)) || (rc = c->d_xh.alloc(16ull * c->ncompact)) ||
         (rc = c->d_acc.alloc(16ull * c->ncompact)) || (rc = c->d_pos.alloc(24ull * ns)))
         return fail(rc);
     if ((rc = far_field_scratch(c->device, &c->ff_scratch)) != IFS_OK) return fail(rc);
     std::vector<double> snm = make_snm(N);
-    if (hipMemcpy(c->d_Leff.p, c->Leff.data(), 4 * ns, hipMemcpyHostToDevice) != hipSuccess ||
+    // Leff, then the spheres in descending order L (the far field's products)
+    std::vector<int32_t> Lo(c->Leff.begin(), c->Leff.begin() + ns);
+    Lo.resize(2 * (size_t)ns);
+    std::iota(Lo.begin() + ns, Lo.end(), 0);
+    std::stable_sort(Lo.begin() + ns, Lo.end(), [&](int32_t a, int32_t b) { return c->Leff[a] > c->Leff[b]; });
+    if (hipMemcpy(c->d_Leff.p, Lo.data(), 8 * ns, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(c->d_active.p, c->active.data(), 4 * ns, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(c->d_off.p, c->off.data(), 8 * ns, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(c->d_snm.p, snm.data(), 8ull * N * (N + 2), hipMemcpyHostToDevice) != hipSuccess ||

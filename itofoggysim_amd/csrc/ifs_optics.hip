@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include <algorithm>
 #include <cmath>
 #include <complex>
 #include <map>
@@ -38,127 +39,264 @@ __device__ __forceinline__ double2 cmul_(double2 a, double2 b) {
 }
 
 // T_nm, P_nm at the polar angles theta[i]: tab[i * N(N+2) + fidx(n,m)] = (T, P).
-// One block per direction, threads over m = -N..N, each running the recurrences
-// of d^n_{m,1} and d^n_{m,-1} upward in n.
-__global__ void k_ff_tables(int N, const double *__restrict__ theta, double2 *__restrict__ tab) {
-    const int i = blockIdx.x;
-    const double th = theta[i];
-    const double cb = cos(th);
-    const double ch = cos(0.5 * th), sh = sin(0.5 * th);
+// One thread per order m >= 0 and FFT directions, running the recurrences of d^n_{m,1}
+// and d^n_{m,-1} upward in n; the square roots and the division of a step and the
+// log-gammas of the seeds serve all FFT directions, and
+//   T_{n,-m} = (-1)^m T_nm,  P_{n,-m} = -(-1)^m P_nm
+// the negative orders.  Bound by the FP64 chain of the recurrences (6516 directions of order
+// 22: 57 us; 92 us with a thread per signed order and direction).
+constexpr int FFT = 4;
+__global__ __launch_bounds__(256) void k_ff_tables(int N, int ndir, const double *__restrict__ theta,
+                                                   double2 *__restrict__ tab) {
+    const int mw = min(N + 1, 256), subs = 256 / mw, sub = threadIdx.x / mw;
+    if (sub >= subs) return;
+    const int i0 = (blockIdx.x * subs + sub) * FFT;
+    if (i0 >= ndir) return;
     const int64_t blk = (int64_t)N * (N + 2);
-    double2 *out = tab + (int64_t)i * blk;
-    for (int m = -N + (int)threadIdx.x; m <= N; m += blockDim.x) {
-        const int am = m < 0 ? -m : m;
-        const int n0 = am > 1 ? am : 1;
-        const double sg = (am & 1) ? 1.0 : -1.0;  // (-1)^{m+1}
-        double p1 = wigner_seed(m, 1, ch, sh), q1 = wigner_seed(m, -1, ch, sh);
-        double p2 = 0.0, q2 = 0.0;
+    double cb[FFT], ch[FFT], sh[FFT];
+#pragma unroll
+    for (int d = 0; d < FFT; ++d) {
+        const double th = theta[min(i0 + d, ndir - 1)];
+        cb[d] = cos(th);
+        ch[d] = cos(0.5 * th);
+        sh[d] = sin(0.5 * th);
+    }
+    for (int m = threadIdx.x % mw; m <= N; m += mw) {
+        const int n0 = m > 1 ? m : 1;
+        const double sm = (m & 1) ? -1.0 : 1.0;  // (-1)^m
+        const double lp = wigner_seed_ln(m, 1), lq = wigner_seed_ln(m, -1);
+        double p1[FFT], p2[FFT], q1[FFT], q2[FFT];
+#pragma unroll
+        for (int d = 0; d < FFT; ++d) {
+            p1[d] = wigner_seed(m, 1, ch[d], sh[d], lp);
+            q1[d] = wigner_seed(m, -1, ch[d], sh[d], lq);
+            p2[d] = q2[d] = 0.0;
+        }
         for (int n = n0; n <= N; ++n) {
             if (n > n0) {
-                double pn = wigner_step(n, m, 1, cb, p1, p2);
-                double qn = wigner_step(n, m, -1, cb, q1, q2);
-                p2 = p1;
-                p1 = pn;
-                q2 = q1;
-                q1 = qn;
+                const double nn = n, o = nn - 1.0, m2 = (double)m * m;
+                const double inv = 1.0 / (o * sqrt((nn * nn - m2) * (nn * nn - 1.0)));
+                const double F = (2.0 * nn - 1.0) * inv, G = nn * sqrt((o * o - m2) * (o * o - 1.0)) * inv;
+#pragma unroll
+                for (int d = 0; d < FFT; ++d) {
+                    const double pn = F * (nn * o * cb[d] - m) * p1[d] - G * p2[d];
+                    const double qn = F * (nn * o * cb[d] + m) * q1[d] - G * q2[d];
+                    p2[d] = p1[d];
+                    p1[d] = pn;
+                    q2[d] = q1[d];
+                    q1[d] = qn;
+                }
             }
-            double f = 0.5 * sg * sqrt(2.0 * n + 1.0);
-            out[n * n - 1 + m + n] = make_double2(f * (p1 - q1), f * (p1 + q1));
+            const double f = -0.5 * sm * sqrt(2.0 * n + 1.0);
+#pragma unroll
+            for (int d = 0; d < FFT; ++d) {
+                if (i0 + d >= ndir) break;
+                const double T = f * (p1[d] - q1[d]), P = f * (p1[d] + q1[d]);
+                double2 *o = tab + (int64_t)(i0 + d) * blk + (int64_t)n * n - 1 + n;
+                o[m] = make_double2(T, P);
+                if (m > 0) o[-m] = make_double2(sm * T, -sm * P);
+            }
         }
     }
 }
 
-constexpr int FFD = 4;  // directions per block
+// The sum over spheres first: for every entry e = (n, m),
+//   Y_a[d, e] = sum_j e^{-ik rhat_d.d_j} a_j[e]   (and Y_b), a complex matrix product of the
+// phases [directions x spheres] with the coefficients [spheres x entries], in FP64 MFMA
+// (16 directions x 16 entries x 4 spheres a step, a and b with the same phases); then the
+// contraction with T, P, s_nm and e^{i m phi} once per (d, e) instead of once per
+// (d, e, sphere): 16 instead of about 30 flops per (d, e, sphere), and the phases and
+// coefficients of a step serve 16 directions.
+// A block: 16 directions, the phases of FFC spheres at a time in LDS; its waves share out
+// the entries in tiles of 16, strided by all waves of the directions' blocks (gridDim.y of
+// them).  Spheres come in descending order L_j, so a tile of degrees >= n ends its product
+// at the first sphere with L_j < n.  Coefficients beyond a sphere's L_j are not read.
+// out[(blockIdx.y * ndir + i) * 2 + {0, 1}]: this block's part of (F_theta, F_phi).
+// 200 spheres of orders up to 22, 6516 directions: 224 us (6.5 GFLOP in the matrix cores, 90 us
+// at their rate; the rest the phases' sincos, the contraction and the first loads of a tile)
+// against 1641 us with a thread per entry and sphere.  Two tiles of directions a wave, for
+// half the coefficient reads: 252 us, so those do not bound it.
+constexpr int FFC = 128;  // spheres per chunk of phases
+constexpr int FFE = 112;  // orders up to which e^{i m phi} is kept in LDS: 64 KB with the phases
+typedef double ffv4 __attribute__((ext_vector_type(4)));
 
-// F_theta, F_phi for FFD directions per block; threads run over the entries of
-// every sphere, then reduce through LDS.  out[i] = (F_theta, F_phi) complex.
-__global__ __launch_bounds__(256) void k_far_field(int N, int ns, const int32_t *__restrict__ Leff,
+template <bool EM>
+__global__ __launch_bounds__(256, EM ? 3 : 2) void k_far_field(
+    int N, int ns, const int32_t *__restrict__ Leff, const int32_t *__restrict__ order,
                                                    const double *__restrict__ pos, double k,
                                                    const double *__restrict__ snm, const double2 *__restrict__ x,
                                                    int ndir, const double *__restrict__ theta,
                                                    const double *__restrict__ phi, const double2 *__restrict__ tab,
                                                    double2 *__restrict__ out) {
-    extern __shared__ double2 sh[];
-    const int W = 2 * N + 1;
-    double2 *em = sh;                    // [FFD][W]: e^{i m phi_i}
-    double2 *red = sh + FFD * W;         // [256] reduction scratch
-    __shared__ double rh[FFD][3];
-    const int i0 = blockIdx.x * FFD;
-    const int nd = (ndir - i0) < FFD ? (ndir - i0) : FFD;
-    for (int q = threadIdx.x; q < FFD * W; q += blockDim.x) {
-        int d = q / W, m = q % W - N;
-        double s = 0.0, c = 1.0;
-        if (d < nd) sincos((double)m * phi[i0 + d], &s, &c);
-        em[q] = make_double2(c, s);
-    }
-    if (threadIdx.x < FFD) {
-        int d = threadIdx.x;
-        double t = d < nd ? theta[i0 + d] : 0.0, f = d < nd ? phi[i0 + d] : 0.0;
-        rh[d][0] = sin(t) * cos(f);
-        rh[d][1] = sin(t) * sin(f);
-        rh[d][2] = cos(t);
-    }
-    __syncthreads();
+    extern __shared__ double2 em[];  // EM: [16][N + 1], e^{i m phi}
+    __shared__ double2 ph[FFC * 16];  // [sphere][direction]
+    __shared__ int2 sp[FFC];           // (sphere, entries of a block)
+    __shared__ double rh[16][3];
+    __shared__ double2 red[4][16][2];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, lk = lane >> 4;
+    const int i0 = blockIdx.x * 16;
     const int64_t blk = (int64_t)N * (N + 2);
-    double2 at[FFD], ap[FFD];
-#pragma unroll
-    for (int d = 0; d < FFD; ++d) at[d] = ap[d] = make_double2(0.0, 0.0);
-    for (int j = 0; j < ns; ++j) {
-        const int L = Leff[j];
-        const int cnt = L * (L + 2);
-        double2 ph[FFD];
-#pragma unroll
-        for (int d = 0; d < FFD; ++d) {
-            double arg = -k * (rh[d][0] * pos[3 * j] + rh[d][1] * pos[3 * j + 1] + rh[d][2] * pos[3 * j + 2]);
+    const int nt = (int)((blk + 15) / 16);
+    if (EM)
+        for (int q = tid; q < 16 * (N + 1); q += 256) {
+            const int d = q / (N + 1), m = q % (N + 1);
             double s, c;
-            sincos(arg, &s, &c);
-            ph[d] = make_double2(c, s);
+            sincos((double)m * phi[min(i0 + d, ndir - 1)], &s, &c);
+            em[q] = make_double2(c, s);
         }
-        const double2 *xa = x + (int64_t)j * 2 * blk;
-        for (int e = threadIdx.x; e < cnt; e += blockDim.x) {
+    if (tid < 16) {
+        const int i = min(i0 + tid, ndir - 1);
+        const double t = theta[i], f = phi[i];
+        rh[tid][0] = sin(t) * cos(f);
+        rh[tid][1] = sin(t) * sin(f);
+        rh[tid][2] = cos(t);
+    }
+    double2 ft[4] = {}, fp[4] = {};
+    for (int j0 = 0; j0 < ns; j0 += FFC) {
+        const int jn = min(FFC, ns - j0), jp = (jn + 3) & ~3;
+        __syncthreads();
+        for (int q = tid; q < jp; q += 256) {
+            int2 v = make_int2(0, 0);
+            if (q < jn) {
+                v.x = order[j0 + q];
+                const int L = Leff[v.x];
+                v.y = L * (L + 2);
+            }
+            sp[q] = v;
+        }
+        for (int q = tid; q < jp * 16; q += 256) {
+            const int j = q >> 4, d = q & 15;
+            double2 v = make_double2(0.0, 0.0);
+            if (j < jn) {
+                const double *p = pos + 3 * (int64_t)order[j0 + j];
+                const double arg = -k * (rh[d][0] * p[0] + rh[d][1] * p[1] + rh[d][2] * p[2]);
+                sincos(arg, &v.y, &v.x);
+            }
+            ph[q] = v;
+        }
+        __syncthreads();
+        for (int t = blockIdx.y * 4 + wave; t < nt; t += gridDim.y * 4) {
+            const int e = t * 16 + col;
+            ffv4 ar = {}, ai = {}, br = {}, bi = {};
+            int je = 0;  // spheres that hold any entry of this tile
+            for (int lo = jn; lo > 0; lo >>= 1)
+                while (je + lo <= jn && __builtin_amdgcn_readfirstlane(sp[je + lo - 1].y) > t * 16) je += lo;
+            auto load = [&](int j, double2 &a, double2 &b) {
+                const int2 s = sp[j + lk];
+                a = b = make_double2(0.0, 0.0);
+                if (e < s.y) {
+                    const double2 *xa = x + (int64_t)s.x * 2 * blk + e;
+                    a = xa[0];
+                    b = xa[blk];
+                }
+            };
+            double2 an, bn;
+            if (je > 0) load(0, an, bn);
+            for (int j = 0; j < je; j += 4) {
+                const double2 a = an, b = bn;
+                if (j + 4 < je) load(j + 4, an, bn);
+                const double2 f = ph[(j + lk) * 16 + col];
+                ar = __builtin_amdgcn_mfma_f64_16x16x4f64(f.x, a.x, ar, 0, 0, 0);
+                ai = __builtin_amdgcn_mfma_f64_16x16x4f64(f.x, a.y, ai, 0, 0, 0);
+                br = __builtin_amdgcn_mfma_f64_16x16x4f64(f.x, b.x, br, 0, 0, 0);
+                bi = __builtin_amdgcn_mfma_f64_16x16x4f64(f.x, b.y, bi, 0, 0, 0);
+                ar = __builtin_amdgcn_mfma_f64_16x16x4f64(-f.y, a.y, ar, 0, 0, 0);
+                ai = __builtin_amdgcn_mfma_f64_16x16x4f64(f.y, a.x, ai, 0, 0, 0);
+                br = __builtin_amdgcn_mfma_f64_16x16x4f64(-f.y, b.y, br, 0, 0, 0);
+                bi = __builtin_amdgcn_mfma_f64_16x16x4f64(f.y, b.x, bi, 0, 0, 0);
+            }
+            if (e >= blk) continue;
             int n = (int)sqrt((double)(e + 1));
             while ((n + 1) * (n + 1) - 1 <= e) ++n;
             while (n * n - 1 > e) --n;
-            const int m = e - (n * n - 1) - n;
+            const int m = e - (n * n - 1) - n, am = m < 0 ? -m : m;
             const double s = snm[e];
-            const double2 a = make_double2(s * xa[e].x, s * xa[e].y);
-            const double2 b = make_double2(s * xa[e + blk].x, s * xa[e + blk].y);
 #pragma unroll
-            for (int d = 0; d < FFD; ++d) {
-                if (d >= nd) break;
-                const double2 tp = tab[(int64_t)(i0 + d) * blk + e];  // (T, P)
-                const double2 w = cmul_(ph[d], em[d * W + m + N]);
-                double2 vt = make_double2(a.x * tp.x + b.x * tp.y, a.y * tp.x + b.y * tp.y);  // a T + b P
-                double2 vp = make_double2(a.x * tp.y + b.x * tp.x, a.y * tp.y + b.y * tp.x);  // a P + b T
-                vt = cmul_(w, vt);
-                vp = cmul_(w, vp);
-                at[d].x += vt.x;
-                at[d].y += vt.y;
-                ap[d].x += vp.x;
-                ap[d].y += vp.y;
+            for (int v = 0; v < 4; ++v) {
+                const int d = 4 * v + lk, i = min(i0 + d, ndir - 1);
+                double2 w;
+                if (EM)
+                    w = em[d * (N + 1) + am];
+                else
+                    sincos((double)am * phi[i], &w.y, &w.x);
+                if (m < 0) w.y = -w.y;
+                const double2 tp = tab[(int64_t)i * blk + e];  // (T, P)
+                const double2 a = make_double2(s * ar[v], s * ai[v]), b = make_double2(s * br[v], s * bi[v]);
+                const double2 vt = cmul_(w, make_double2(a.x * tp.x + b.x * tp.y, a.y * tp.x + b.y * tp.y));
+                const double2 vp = cmul_(w, make_double2(a.x * tp.y + b.x * tp.x, a.y * tp.y + b.y * tp.x));
+                ft[v].x += vt.x;
+                ft[v].y += vt.y;
+                fp[v].x += vp.x;
+                fp[v].y += vp.y;
             }
         }
     }
-    // block reduction, one direction and component at a time (fixed order)
-    for (int d = 0; d < nd; ++d) {
-        for (int comp = 0; comp < 2; ++comp) {
-            red[threadIdx.x] = comp == 0 ? at[d] : ap[d];
-            __syncthreads();
-            for (int h = blockDim.x / 2; h > 0; h >>= 1) {
-                if ((int)threadIdx.x < h) {
-                    red[threadIdx.x].x += red[threadIdx.x + h].x;
-                    red[threadIdx.x].y += red[threadIdx.x + h].y;
-                }
-                __syncthreads();
-            }
-            if (threadIdx.x == 0) {
-                double2 v = red[0];
-                // F_theta = i * sum, F_phi = - sum
-                out[2 * (int64_t)(i0 + d) + comp] = comp == 0 ? make_double2(-v.y, v.x) : make_double2(-v.x, -v.y);
-            }
-            __syncthreads();
+    // over the 16 entries' lanes, then over the waves (fixed order)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        for (int o = 8; o > 0; o >>= 1) {
+            ft[v].x += __shfl_xor(ft[v].x, o);
+            ft[v].y += __shfl_xor(ft[v].y, o);
+            fp[v].x += __shfl_xor(fp[v].x, o);
+            fp[v].y += __shfl_xor(fp[v].y, o);
+        }
+        if (col == 0) {
+            red[wave][4 * v + lk][0] = ft[v];
+            red[wave][4 * v + lk][1] = fp[v];
         }
     }
+    __syncthreads();
+    if (tid < 32 && i0 + (tid >> 1) < ndir) {
+        const int d = tid >> 1, c = tid & 1;
+        double2 s = red[0][d][c];
+        for (int w = 1; w < 4; ++w) {
+            s.x += red[w][d][c].x;
+            s.y += red[w][d][c].y;
+        }
+        // F_theta = i * sum, F_phi = - sum
+        out[((int64_t)blockIdx.y * ndir + i0 + d) * 2 + c] = c == 0 ? make_double2(-s.y, s.x) : make_double2(-s.x, -s.y);
+    }
+}
+
+// out[q] = sum over the parts of part[g * n + q]
+__global__ void k_ff_sum(int64_t n, int parts, const double2 *__restrict__ part, double2 *__restrict__ out) {
+    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= n) return;
+    double2 s = part[q];
+    for (int g = 1; g < parts; ++g) {
+        s.x += part[g * n + q].x;
+        s.y += part[g * n + q].y;
+    }
+    out[q] = s;
+}
+
+// Blocks that share 16 directions' entries, at most `room` for their parts of the sums:
+// enough for 1024 blocks, each with a tile for
+// every wave (6516 directions: 224 us; for 512 blocks 262, for 2048 235).
+int ff_parts(int N, int ndir, int64_t room) {
+    const int64_t rows = (ndir + 15) / 16, nt = ((int64_t)N * (N + 2) + 15) / 16;
+    int64_t g = std::min<int64_t>((1024 + rows - 1) / rows, (nt + 3) / 4);
+    g = std::min<int64_t>(g, room / (2 * (int64_t)ndir));
+    return (int)std::max<int64_t>(1, g);
+}
+
+// tab: ndir * N(N+2) entries, then 2 ndir per part where there is more than one
+int ff_launch(ifs_ctx *c, const void *x, int ndir, const double *theta, const double *phi, double2 *tab, int parts,
+              double2 *out) {
+    const int N = c->N, per = 256 / std::min(N + 1, 256) * FFT;
+    double2 *dst = parts > 1 ? tab + (int64_t)ndir * N * (N + 2) : out;
+    hipLaunchKernelGGL(k_ff_tables, dim3((ndir + per - 1) / per), dim3(256), 0, c->stream, N, ndir, theta, tab);
+    const int32_t *Leff = c->d_Leff.as<int32_t>();
+    const bool em = N <= FFE;
+    auto far = em ? k_far_field<true> : k_far_field<false>;
+    hipLaunchKernelGGL(far, dim3((ndir + 15) / 16, parts), dim3(256), em ? sizeof(double2) * 16 * (N + 1) : 0,
+                       c->stream, N, c->ns, Leff, Leff + c->ns,
+                       c->d_pos.as<double>(), c->prm.k, c->d_snm.as<double>(), (const double2 *)x, ndir, theta, phi,
+                       tab, dst);
+    if (parts > 1)
+        hipLaunchKernelGGL(k_ff_sum, dim3((unsigned)((2 * (int64_t)ndir + 255) / 256)), dim3(256), 0, c->stream,
+                           2 * (int64_t)ndir, parts, dst, out);
+    return hipGetLastError() == hipSuccess ? IFS_OK : IFS_E_HIP;
 }
 
 // Per-sphere partial sums for the cross sections: part[j] = (extinction, absorption)
@@ -262,8 +400,8 @@ void d_pm1_host(int N, long double beta, std::vector<long double> &dp, std::vect
 
 }  // namespace ifs
 
-// Scratch of ifs_far_field_device_noalloc: the per-direction T/P tables, in a
-// fixed array of this library on every GPU it runs on (held until the process
+// Scratch of ifs_far_field_device_noalloc: the per-direction T/P tables and,
+// as far as there is room, parts of the sums, in a fixed array of this library on every GPU it runs on (held until the process
 // ends).  Host code never uses the array's name as an address: its device address
 // is looked up once per device (far_field_scratch) and passed to the kernels.
 static __device__ __align__(256) double2 scratch[IFS_FF_SCRATCH_ENTRIES];
@@ -402,21 +540,15 @@ extern "C" int ifs_far_field_device(ifs_ctx *c, const void *x_dev, int64_t n, in
     if (!c || !x_dev || !theta_dev || !phi_dev || !out_dev || n != ifs_vector_length(c) || ndir < 0)
         return IFS_E_ARG;
     if (ndir == 0) return IFS_OK;
-    const int N = c->N;
+    const int64_t entries = (int64_t)ndir * c->N * (c->N + 2);
+    const int parts = ifs::ff_parts(c->N, ndir, INT64_MAX);
     int rc;
-    ifs::DevBuf tab, dpos;
-    if ((rc = tab.alloc(16ull * ndir * N * (N + 2))) || (rc = dpos.alloc(24ull * c->ns))) return rc;
-    if (hipMemcpyAsync(dpos.p, c->pos.data(), 24ull * c->ns, hipMemcpyHostToDevice, c->stream) != hipSuccess)
-        return IFS_E_HIP;
-    hipLaunchKernelGGL(ifs::k_ff_tables, dim3(ndir), dim3(256), 0, c->stream, N, (const double *)theta_dev,
-                       tab.as<double2>());
-    const size_t shm = sizeof(double2) * ((size_t)ifs::FFD * (2 * N + 1) + 256);
-    hipLaunchKernelGGL(ifs::k_far_field, dim3((ndir + ifs::FFD - 1) / ifs::FFD), dim3(256), shm, c->stream, N, c->ns,
-                       c->d_Leff.as<int32_t>(), dpos.as<double>(), c->prm.k, c->d_snm.as<double>(),
-                       (const double2 *)x_dev, ndir, (const double *)theta_dev, (const double *)phi_dev,
-                       tab.as<double2>(), (double2 *)out_dev);
-    if (hipGetLastError() != hipSuccess) return IFS_E_HIP;
-    if (hipStreamSynchronize(c->stream) != hipSuccess) return IFS_E_HIP;  // tab, dpos are freed on return
+    ifs::DevBuf tab;
+    if ((rc = tab.alloc(16ull * (entries + 2ll * ndir * (parts > 1 ? parts : 0))))) return rc;
+    if ((rc = ifs::ff_launch(c, x_dev, ndir, (const double *)theta_dev, (const double *)phi_dev, tab.as<double2>(),
+                             parts, (double2 *)out_dev)))
+        return rc;
+    if (hipStreamSynchronize(c->stream) != hipSuccess) return IFS_E_HIP;  // tab is freed on return
     return IFS_OK;
 }
 
@@ -425,36 +557,35 @@ extern "C" int ifs_far_field_device_noalloc(ifs_ctx *c, const void *x_dev, int64
     if (!c || !x_dev || !theta_dev || !phi_dev || !out_dev || n != ifs_vector_length(c) || ndir < 0)
         return IFS_E_ARG;
     if (ndir == 0) return IFS_OK;
-    const int N = c->N;
-    if ((int64_t)ndir * N * (N + 2) > (int64_t)IFS_FF_SCRATCH_ENTRIES) return IFS_E_ARG;
+    const int64_t entries = (int64_t)ndir * c->N * (c->N + 2);
+    if (entries > (int64_t)IFS_FF_SCRATCH_ENTRIES) return IFS_E_ARG;
     if (!c->ff_scratch || !c->d_pos.p) return IFS_E_ARG;
-    double2 *tab = (double2 *)c->ff_scratch;  // every entry the far-field kernel reads is written first
-    hipLaunchKernelGGL(ifs::k_ff_tables, dim3(ndir), dim3(256), 0, c->stream, N, (const double *)theta_dev, tab);
-    const size_t shm = sizeof(double2) * ((size_t)ifs::FFD * (2 * N + 1) + 256);
-    hipLaunchKernelGGL(ifs::k_far_field, dim3((ndir + ifs::FFD - 1) / ifs::FFD), dim3(256), shm, c->stream, N, c->ns,
-                       c->d_Leff.as<int32_t>(), c->d_pos.as<double>(), c->prm.k, c->d_snm.as<double>(),
-                       (const double2 *)x_dev, ndir, (const double *)theta_dev, (const double *)phi_dev, tab,
-                       (double2 *)out_dev);
-    if (hipGetLastError() != hipSuccess) return IFS_E_HIP;
-    return IFS_OK;
+    // every entry that a kernel reads of the scratch array is written first
+    return ifs::ff_launch(c, x_dev, ndir, (const double *)theta_dev, (const double *)phi_dev,
+                          (double2 *)c->ff_scratch,
+                          ifs::ff_parts(c->N, ndir, (int64_t)IFS_FF_SCRATCH_ENTRIES - entries), (double2 *)out_dev);
 }
 
 extern "C" int ifs_far_field(ifs_ctx *c, const double *x, int64_t n, int32_t ndir, const double *theta,
                              const double *phi, double *out) {
     if (!c || !x || !theta || !phi || !out || n != ifs_vector_length(c) || ndir < 0) return IFS_E_ARG;
     if (ndir == 0) return IFS_OK;
-    ifs::DevBuf dx, dt, dph, dout;
+    // one allocation: x, theta, phi, out, tables and parts
+    const int64_t entries = (int64_t)ndir * c->N * (c->N + 2);
+    const int parts = ifs::ff_parts(c->N, ndir, INT64_MAX);
+    ifs::DevBuf d;
     int rc;
-    if ((rc = dx.alloc(16ull * n)) || (rc = dt.alloc(8ull * ndir)) || (rc = dph.alloc(8ull * ndir)) ||
-        (rc = dout.alloc(32ull * ndir)))
-        return rc;
-    if (hipMemcpy(dx.p, x, 16ull * n, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(dt.p, theta, 8ull * ndir, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(dph.p, phi, 8ull * ndir, hipMemcpyHostToDevice) != hipSuccess)
-        return IFS_E_HIP;
-    if ((rc = ifs_far_field_device(c, dx.p, n, ndir, dt.p, dph.p, dout.p))) return rc;
-    if (hipMemcpy(out, dout.p, 32ull * ndir, hipMemcpyDeviceToHost) != hipSuccess) return IFS_E_HIP;
-    return IFS_OK;
+    if ((rc = d.alloc(16ull * (n + 3ll * ndir + entries + 2ll * ndir * (parts > 1 ? parts : 0))))) return rc;
+    double2 *dx = d.as<double2>(), *dout = dx + n;
+    double *dt = (double *)(dout + 2ll * ndir), *dph = dt + ndir;
+    hipStream_t s = c->stream;
+    if (hipMemcpyAsync(dx, x, 16ull * n, hipMemcpyHostToDevice, s) != hipSuccess ||
+        hipMemcpyAsync(dt, theta, 8ull * ndir, hipMemcpyHostToDevice, s) != hipSuccess ||
+        hipMemcpyAsync(dph, phi, 8ull * ndir, hipMemcpyHostToDevice, s) != hipSuccess ||
+        (rc = ifs::ff_launch(c, dx, ndir, dt, dph, dout + 3ll * ndir, parts, dout)) ||
+        hipMemcpyAsync(out, dout, 32ull * ndir, hipMemcpyDeviceToHost, s) != hipSuccess)
+        rc = rc ? rc : IFS_E_HIP;
+    return hipStreamSynchronize(s) == hipSuccess ? rc : IFS_E_HIP;
 }
 
 extern "C" int ifs_amplitude_matrix(int32_t ndir, const double *phi, const double *Fx, const double *Fy, double *S) {

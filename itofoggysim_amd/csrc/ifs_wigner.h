@@ -10,8 +10,15 @@ namespace ifs {
 //   d^j_{j,m}  = sqrt((2j)!/((j+m)!(j-m)!)) c^{j+m} (-s)^{j-m}
 //   d^j_{-j,m} = sqrt((2j)!/((j+m)!(j-m)!)) c^{j-m} s^{j+m}
 //   d^j_{k,m}  = (-1)^{k-m} d^j_{m,k}
-// with c = cos(beta/2), s = sin(beta/2), evaluated in logs.
-__device__ inline double wigner_seed(int k, int m, double c, double s) {
+// with c = cos(beta/2), s = sin(beta/2), evaluated in logs; ln is the log of the square
+// root (wigner_seed_ln), the same for every angle.
+__device__ inline double wigner_seed_ln(int k, int m) {
+    const int ak = k < 0 ? -k : k, am = m < 0 ? -m : m;
+    const int j = ak < am ? am : ak, q = ak < am ? k : m;
+    return 0.5 * (lgamma(2.0 * j + 1.0) - lgamma((double)(j + q) + 1.0) - lgamma((double)(j - q) + 1.0));
+}
+
+__device__ inline double wigner_seed(int k, int m, double c, double s, double ln) {
     double sign = 1.0;
     if ((k < 0 ? -k : k) < (m < 0 ? -m : m)) {
         int t = k;
@@ -29,7 +36,7 @@ __device__ inline double wigner_seed(int k, int m, double c, double s) {
         ec = j - m;
         es = j + m;
     }
-    double lv = 0.5 * (lgamma(2.0 * j + 1.0) - lgamma((double)(j + m) + 1.0) - lgamma((double)(j - m) + 1.0));
+    double lv = ln;
     if (ec > 0) {
         if (c <= 0.0) return 0.0;
         lv += ec * log(c);
@@ -39,6 +46,10 @@ __device__ inline double wigner_seed(int k, int m, double c, double s) {
         lv += es * log(s);
     }
     return sign * exp(lv);
+}
+
+__device__ inline double wigner_seed(int k, int m, double c, double s) {
+    return wigner_seed(k, m, c, s, wigner_seed_ln(k, m));
 }
 
 // One step of the three-term recurrence in n for d^n_{km}, from d^{n-1} (d1) and d^{n-2} (d2).
