@@ -141,7 +141,7 @@ int pw_build(ifs_ctx *c, PwLevel &P, int isg) {
     if (rc) return rc;
     // offsets -> canonical table: turned and mirrored about z until x >= y >= 0, and z >= 0
     std::map<std::array<int, 3>, int> canon;
-    P.map.assign(216 * 8, PwMap{0, 0, 1, 0});
+    P.map.assign(216, PwMaps{});
     std::vector<char> used(216 * 8, 0);
     for (auto &S : P.src)
         for (int ch = 0; ch < 8; ++ch)
@@ -152,7 +152,7 @@ int pw_build(ifs_ctx *c, PwLevel &P, int isg) {
             const int o[3] = {r / 36 - 2 - (ch >> 2), r / 6 % 6 - 2 - (ch >> 1 & 1), r % 6 - 2 - (ch & 1)};
             // direction of the phase factor: the translation vector isg * o turned by pi about z
             int v[3] = {-isg * o[0], -isg * o[1], isg * o[2]};
-            PwMap M{0, 0, 1, v[2] < 0};
+            PwMap M{0, v[2] < 0, 1, 0};
             int a = v[0], b = v[1], q = 0;
             while (!(a > 0 && b >= 0) && !(a == 0 && b == 0)) {  // turn by -pi/2 into the first quadrant
                 const int t = a;
@@ -161,10 +161,11 @@ int pw_build(ifs_ctx *c, PwLevel &P, int isg) {
                 ++q;
             }
             // (a, b) = turn by -q quarters of v; mirror about the diagonal: angle -> pi/2 - angle
-            M.quarter = q;
+            // (i -> i - q N / 4, mirrored: -(i - (q + 1) N / 4))
+            M.shift = -q;
             if (b > a) {
                 std::swap(a, b);
-                M.quarter = (q + 1) & 3;
+                M.shift = (q + 1) & 3;
                 M.sign = -1;
             }
             const std::array<int, 3> key = {a, b, std::abs(v[2])};
@@ -174,7 +175,7 @@ int pw_build(ifs_ctx *c, PwLevel &P, int isg) {
                 P.canon.push_back(key);
             }
             M.table = it->second;
-            P.map[r * 8 + ch] = M;
+            P.map[r].child[ch] = M;
         }
     const int nc = (int)P.canon.size();
     std::vector<double> dir(4 * nc), t(nc);
@@ -188,7 +189,7 @@ int pw_build(ifs_ctx *c, PwLevel &P, int isg) {
     }
     if ((rc = upload(P.d_src, P.src.data(), sizeof(PwSource) * P.src.size())) ||
         (rc = upload(P.d_par, P.par.data(), sizeof(PwParent) * P.par.size())) ||
-        (rc = upload(P.d_map, P.map.data(), sizeof(PwMap) * P.map.size())) ||
+        (rc = upload(P.d_map, P.map.data(), sizeof(PwMaps) * P.map.size())) ||
         (rc = upload(P.d_canon, dir.data(), 8 * dir.size())))
         return rc;
     // c_p of every table; t and the last terms lie behind them
@@ -351,7 +352,7 @@ int pw_run(ifs_ctx *c, PwLevel &P, const double2 *C, double2 *D, int nrhs, int64
             }
             {
                 Scope sc(c, "m2l_product");
-                launch_pw_m2l(a, P.d_par.as<PwParent>(), (int)P.par.size(), P.d_src.as<PwSource>(), P.d_map.as<PwMap>(),
+                launch_pw_m2l(a, P.d_par.as<PwParent>(), (int)P.par.size(), P.d_src.as<PwSource>(), P.d_map.as<PwMaps>(),
                               P.nb, nr, ch.maxN, s);
             }
             {

@@ -27,9 +27,12 @@ struct PwParent {
 // How the offset of (source position, child) reads the canonical tables.
 struct PwMap {
     int32_t table;   // canonical offset
-    int32_t quarter; // azimuth turned by quarter * pi / 2
-    int32_t sign;    // +1, -1: azimuth mirrored
     int32_t flip;    // 1: polar angle mirrored
+    int32_t sign;    // +1, -1: azimuth i -> sign * i + shift * N / 4
+    int32_t shift;
+};
+struct PwMaps {
+    PwMap child[8];
 };
 // Azimuthal transform of one length.
 struct PwFft {
@@ -47,7 +50,7 @@ struct PwLevel {
     std::vector<int> jlo;     // per |m|: first node with mF >= |m|
     std::vector<PwSource> src;
     std::vector<PwParent> par;
-    std::vector<PwMap> map;   // [216][8]
+    std::vector<PwMaps> map;  // [216]
     std::vector<std::array<int, 3>> canon;
     std::vector<PwFft> fft;   // distinct lengths
     std::vector<int> fft_of;  // per node
@@ -137,7 +140,7 @@ void launch_pw_ttable(int ncanon, int P, int Q2, int j0, int R2, int a0, int a1,
 void launch_pw_pack(const PwArg &a, int nb, int64_t off, const double2 *C, int64_t stride, hipStream_t s);
 void launch_pw_synth(const PwArg &a, hipStream_t s);
 void launch_pw_fft(const PwArg &a, int inverse, int maxN, hipStream_t s);
-void launch_pw_m2l(const PwArg &a, const PwParent *par, int npar, const PwSource *src, const PwMap *map, int nb,
+void launch_pw_m2l(const PwArg &a, const PwParent *par, int npar, const PwSource *src, const PwMaps *map, int nb,
                    int nrhs, int maxN, hipStream_t s);
 void launch_pw_anal(const PwArg &a, int accumulate, hipStream_t s);
 void launch_pw_unpack(const PwArg &a, int nb, int64_t off, double2 *D, int64_t stride, hipStream_t s);

@@ -457,13 +457,20 @@ __global__ __launch_bounds__(512) void k_pw_fft(PwArg a, int NBmax) {
     }
 }
 
-// (mixed precision reads T rounded to FP32, half of the loads; samples and sums stay FP64)
 // H(target) = sum over its sources of T F: wave per (row, 64 azimuths, parent), the eight
 // children's sums of both helicities in registers; a source's samples are read once per
-// parent, the tables by neighbouring waves of the same azimuths from one L2.
+// parent, the tables by neighbouring waves of the same azimuths from one L2 (mixed precision
+// reads them rounded to FP32, half of the bytes; samples and sums stay FP64).
+// Bound by the tables' reads: 16 bytes per 16 flops, through L1 from L2.  The loads of a
+// source and all eight children are in flight while the previous source's products run, also
+// for children that the source does not reach (they read some entry of the first table): with
+// a branch around each load every product waited for its own load.  56046 translations of
+// orders 97 and 174: 9.5 ms with loads behind branches, 7.2 with a source's loads first and
+// the next source's beside the products, 5.2 as here with 32-bit offsets from scalar row
+// addresses (12 TB/s of tables).
 template <typename TT>
 __global__ __launch_bounds__(256) void k_pw_m2l(const TT *__restrict__ T, PwArg a, const PwParent *__restrict__ par, int npar,
-                                                const PwSource *__restrict__ src, const PwMap *__restrict__ map,
+                                                const PwSource *__restrict__ src, const PwMaps *__restrict__ map,
                                                 int nb, int ptiles, int64_t nblocks) {
     const int64_t id = die_order(blockIdx.x, nblocks);
     const int pt = (int)(id % ptiles);
@@ -488,21 +495,24 @@ __global__ __launch_bounds__(256) void k_pw_m2l(const TT *__restrict__ T, PwArg 
     double2 hp[8], hm[8];
 #pragma unroll
     for (int c = 0; c < 8; ++c) hp[c] = hm[c] = make_double2(0.0, 0.0);
-    const int N4 = N >> 2;
-    for (int e = P.beg; e < P.end; ++e) {
-        const PwSource S = src[e];
-        const double2 fp = Fp[(int64_t)S.box * N], fm = Fm[(int64_t)S.box * N];
-        const PwMap *mp = map + S.r * 8;
+    // azimuth i of a child's table: +-(i - quarter N / 4) mod N, in bytes from the row's start
+    const int nB = N * (int)sizeof(TT), n4B = (N >> 2) * (int)sizeof(TT);
+    const uint32_t tB = (uint32_t)(a.tsn * sizeof(TT));
+    const char *r0 = (const char *)(T + t0), *r1 = (const char *)(T + t1);
+    auto load_T = [&](const PwMaps &M, TT tv[8]) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const PwMap q = M.child[c];
+            const uint32_t o = (uint32_t)(__mul24(i, q.sign * (int)sizeof(TT)) + q.shift * n4B);
+            const char *row = (q.flip ? r1 : r0) + (uint64_t)(uint32_t)q.table * tB;
+            tv[c] = *(const TT *)(row + min(o, o + (uint32_t)nB));
+        }
+    };
+    auto product = [&](const PwSource &S, const TT tv[8], double2 fp, double2 fm) {
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
             if (!(S.mask >> c & 1)) continue;
-            const PwMap q = mp[c];
-            int ii = i - q.quarter * N4;
-            ii = q.sign < 0 ? -ii : ii;
-            ii = ii < 0 ? ii + N : ii;
-            ii = ii >= N ? ii - N : ii;
-            const TT tv = T[(int64_t)q.table * a.tsn + (q.flip ? t1 : t0) + ii];
-            const double2 t = make_double2(tv.x, tv.y);
+            const double2 t = make_double2(tv[c].x, tv[c].y);
             hp[c].x = fma(t.x, fp.x, hp[c].x);
             hp[c].x = fma(-t.y, fp.y, hp[c].x);
             hp[c].y = fma(t.x, fp.y, hp[c].y);
@@ -512,6 +522,32 @@ __global__ __launch_bounds__(256) void k_pw_m2l(const TT *__restrict__ T, PwArg 
             hm[c].y = fma(t.x, fm.y, hm[c].y);
             hm[c].y = fma(t.y, fm.x, hm[c].y);
         }
+    };
+    if (P.beg < P.end) {
+        // two sources in flight: the tables' and samples' loads of one during the products of
+        // the other; a source's map is read one source ahead of its loads
+        PwSource S[2], S1 = src[P.beg], S2 = src[min(P.beg + 1, P.end - 1)];
+        PwMaps M1 = map[S1.r];
+        double2 fp[2], fm[2];
+        TT tv[2][8];
+        auto load = [&](int e, int q) {
+            S[q] = S1;
+            fp[q] = Fp[(int64_t)S1.box * N];
+            fm[q] = Fm[(int64_t)S1.box * N];
+            load_T(M1, tv[q]);
+            M1 = map[S2.r];
+            S1 = S2;
+            S2 = src[min(e + 2, P.end - 1)];
+        };
+        load(P.beg, 0);
+        int e = P.beg;
+        for (; e + 1 < P.end; e += 2) {
+            load(e + 1, 1);
+            product(S[0], tv[0], fp[0], fm[0]);
+            load(min(e + 2, P.end - 1), 0);
+            product(S[1], tv[1], fp[1], fm[1]);
+        }
+        if (e < P.end) product(S[0], tv[0], fp[0], fm[0]);
     }
     if (i0 >= N) return;
     double2 *Hp = a.H + fb + (int64_t)rhs * nb * N + i;
@@ -564,7 +600,7 @@ void launch_pw_fft(const PwArg &a, int inverse, int maxN, hipStream_t s) {
     else
         hipLaunchKernelGGL(k_pw_fft<false>, grid, dim3(512), shm, s, a, NB);
 }
-void launch_pw_m2l(const PwArg &a, const PwParent *par, int npar, const PwSource *src, const PwMap *map, int nb,
+void launch_pw_m2l(const PwArg &a, const PwParent *par, int npar, const PwSource *src, const PwMaps *map, int nb,
                    int nrhs, int maxN, hipStream_t s) {
     const int ptiles = (npar + 3) / 4;
     const int64_t nblocks = (int64_t)ptiles * ((maxN + 63) / 64);
