@@ -191,14 +191,17 @@ int pair_plan(ifs_ctx *c, PairBatch &B, int nrhs) {
         }
     }
     if (cur.t0 < (int)B.tiles.size()) close_chunk();
-    // tiles by node set, 8 to a block of the shift (4 where a chunk has few)
+    // tiles by node set, then by order, 8 to a block of the shift (4 where a chunk has few)
     B.groups.clear();
     B.order.clear();
     for (auto &ch : B.chunks) {
         ch.waves = ch.t1 - ch.t0 >= 1024 ? 8 : 4;
         std::vector<int32_t> o;
         for (int t = ch.t0; t < ch.t1; ++t) o.push_back(t);
-        std::stable_sort(o.begin(), o.end(), [&](int a, int b) { return B.tiles[a].Q < B.tiles[b].Q; });
+        std::stable_sort(o.begin(), o.end(), [&](int a, int b) {
+            const PairTile &x = B.tiles[a], &y = B.tiles[b];
+            return x.Q != y.Q ? x.Q < y.Q : x.K < y.K;
+        });
         ch.a0 = (int)B.groups.size();
         for (size_t i = 0; i < o.size();) {
             const PairTile &T = B.tiles[o[i]];

@@ -389,19 +389,22 @@ __global__ __launch_bounds__(256) void k_pair_fwd(const PairTile *__restrict__ t
 // P_m, z_+(-m) and z_-(m) take Q_m, so each of the two products has 16 columns.  The tiles
 // of a block share one node set: its matrices pass through LDS one node tile at a time (read
 // per wave from L1 they took 8 cache accesses per 64-cycle product and bounded the kernel:
-// 5740 tiles of orders 9-18 in 343 us; through LDS, rows read whole, 238 us).
+// 5740 tiles of orders 9-18 in 343 us; through LDS, rows read whole, 238 us).  A wave fetches
+// its rows of the next node tile while the block works on this one, and a block's tiles have
+// similar orders (few waves without work at high m): 48 clusters 588 -> 522 us, 5740 tiles 234.
 // Node-set matrices at off_q: for [m][P, Q]: A1[Q/16][S1][64] (rows
 // nodes, inner degrees) and after all of them A2[UT][Q/4][64] (rows degrees, inner nodes).
 // KS, UT: inner steps of four source degrees and tiles of 16 target degrees that the launch holds.
-template <int UT, int KS>
-__global__ __launch_bounds__(512) void k_pair_axial(const PairTile *__restrict__ tiles,
+template <int UT, int KS, int NW>
+__global__ __launch_bounds__(64 * NW) void k_pair_axial(const PairTile *__restrict__ tiles,
                                                     const PairSlot *__restrict__ slots,
                                                     const PairGroup *__restrict__ groups,
                                                     const int32_t *__restrict__ order, int NL,
                                                     const double *__restrict__ quad, const double2 *__restrict__ tab,
                                                     const double2 *__restrict__ wax, const double *__restrict__ Y,
                                                     int64_t y_stride, double *__restrict__ Z, int64_t z_stride) {
-    __shared__ double As[2 * KS + 8 * UT][64];  // [type][step] of A1, then [type][t][v] of A2
+    constexpr int AR = 2 * KS + 8 * UT, PF = (AR + NW - 1) / NW;
+    __shared__ double As[2][AR][64];  // [buffer][type][step] of A1, then [type][t][v] of A2
     const PairGroup G = groups[blockIdx.x];
     const int m = blockIdx.y;
     if (m > G.K) return;
@@ -476,41 +479,58 @@ __global__ __launch_bounds__(512) void k_pair_axial(const PairTile *__restrict__
     dv4 u[2][UT];
 #pragma unroll
     for (int t = 0; t < UT; ++t) u[0][t] = u[1][t] = dv4{0, 0, 0, 0};
+    // a wave stages rows wv, wv + NW, ...: in registers while the block works on the other buffer
+    double2 tv[4];
+    double pre[PF];
+    auto fetch = [&](int qt) {
+#pragma unroll
+        for (int i = 0; i < PF; ++i) {
+            const int r = wv + NW * i;
+            pre[i] = 0.0;
+            if (r < 2 * KS) {
+                const int ty = r >= KS, s = r - ty * KS;
+                if (s < ksg) pre[i] = A1[(int64_t)((ty * QT + qt) * S1 + s) * 64 + lane];
+            } else if (r < AR) {
+                const int q = r - 2 * KS, ty = q >= 4 * UT, t = (q >> 2) - ty * UT;
+                if (t < utg) pre[i] = A2[((int64_t)(ty * UTN + t) * 4 * QT + 4 * qt + (q & 3)) * 64 + lane];
+            }
+        }
+    };
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < PF; ++i)
+            if (wv + NW * i < AR) As[buf][wv + NW * i][lane] = pre[i];
+    };
+    fetch(0);
+    stage(0);
+    __syncthreads();
     for (int qt = 0; qt < QT; ++qt) {
-        double2 tv[4];
+        const double(*A)[64] = As[qt & 1];
         if (live)
 #pragma unroll
             for (int v = 0; v < 4; ++v) tv[v] = tq[16 * qt + 4 * v + lk];
-        __syncthreads();
-        for (int i = threadIdx.x; i < 2 * ksg * 64; i += blockDim.x) {
-            const int ty = i >= ksg * 64, r = (i >> 6) - ty * ksg;
-            As[ty * KS + r][i & 63] = A1[(int64_t)((ty * QT + qt) * S1 + r) * 64 + (i & 63)];
+        if (qt + 1 < QT) fetch(qt + 1);
+        if (live) {
+            dv4 g[2] = {dv4{0, 0, 0, 0}, dv4{0, 0, 0, 0}};
+#pragma unroll
+            for (int s = 0; s < KS; ++s)
+                if (s < ks) {
+                    g[0] = mma(A[s][lane], bp[s], g[0]);
+                    g[1] = mma(A[KS + s][lane], bq[s], g[1]);
+                }
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+#pragma unroll
+                for (int ty = 0; ty < 2; ++ty) {
+                    const double x = g[ty][v], xo = __shfl_xor(x, 1, 64);
+                    const double b = tv[v].x * x + sg * tv[v].y * xo;
+#pragma unroll
+                    for (int t = 0; t < UT; ++t)
+                        if (t < ut) u[ty][t] = mma(A[2 * KS + (ty * UT + t) * 4 + v][lane], b, u[ty][t]);
+                }
         }
-        for (int i = threadIdx.x; i < 8 * utg * 64; i += blockDim.x) {
-            const int f = i >> 6, v = f & 3, tt = f >> 2;  // tt = ty * utg + t
-            const int ty = tt >= utg, t = tt - ty * utg;
-            As[2 * KS + (ty * UT + t) * 4 + v][i & 63] =
-                A2[((int64_t)(ty * UTN + t) * 4 * QT + 4 * qt + v) * 64 + (i & 63)];
-        }
+        if (qt + 1 < QT) stage((qt + 1) & 1);
         __syncthreads();
-        if (!live) continue;
-        dv4 g[2] = {dv4{0, 0, 0, 0}, dv4{0, 0, 0, 0}};
-#pragma unroll
-        for (int s = 0; s < KS; ++s)
-            if (s < ks) {
-                g[0] = mma(As[s][lane], bp[s], g[0]);
-                g[1] = mma(As[KS + s][lane], bq[s], g[1]);
-            }
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-#pragma unroll
-            for (int ty = 0; ty < 2; ++ty) {
-                const double x = g[ty][v], xo = __shfl_xor(x, 1, 64);
-                const double b = tv[v].x * x + sg * tv[v].y * xo;
-#pragma unroll
-                for (int t = 0; t < UT; ++t)
-                    if (t < ut) u[ty][t] = mma(As[2 * KS + (ty * UT + t) * 4 + v][lane], b, u[ty][t]);
-            }
     }
     if (!live) return;
 #pragma unroll
@@ -685,9 +705,9 @@ void launch_pair_axial(const PairTile *tiles, const PairSlot *slots, const PairG
                        int64_t z_stride, int nrhs, hipStream_t s) {
     if (ngroups <= 0) return;
     const dim3 grid(ngroups, max_K + 1, nrhs);
-#define IFS_PAIR_AXIAL(UT, KS)                                                                                       \
-    hipLaunchKernelGGL((k_pair_axial<UT, KS>), grid, dim3(64 * waves), 0, s, tiles, slots, groups, order, NL, quad, tab, \
-                       wax, Y, y_stride, Z, z_stride)
+#define IFS_PAIR_AXIAL(UT, KS)                                                                                      \
+    hipLaunchKernelGGL((waves == 8 ? k_pair_axial<UT, KS, 8> : k_pair_axial<UT, KS, 4>), grid, dim3(64 * waves), 0, s,  \
+                       tiles, slots, groups, order, NL, quad, tab, wax, Y, y_stride, Z, z_stride)
     if (max_L <= 16)
         IFS_PAIR_AXIAL(1, 4);
     else if (max_L <= 24)
