@@ -29,6 +29,8 @@
 // pairs, orders 9-23) 40.1 -> 8.8 ms, with four right-hand sides (114758 pairs) 81.9 ->
 // 15.3 ms; error against 64-bit sums unchanged (3e-13, 1.1e-13).
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 #include <math.h>
 
 #include "ifs_pair.h"
@@ -362,8 +364,11 @@ __device__ __forceinline__ void pair_fwd(int n, const PairTile &T, const PairSlo
         }
 }
 
-// RT = 1: degrees 1..31, RT = 2: 32..63.
-template <int RT>
+// RT = 1: degrees 1..31, RT = 2: 32..63.  KSM: the most inner steps that the launch meets.  The
+// operands of KSM steps set the registers (forward / backward 67 / 127 for two, 84 / 165 for
+// three, 114 / 219 for four) and so the waves that hide the loads, which bound both kernels:
+// each range of degrees has a launch of its own.
+template <int RT, int KSM>
 __global__ __launch_bounds__(256) void k_pair_fwd(const PairTile *__restrict__ tiles,
                                                   const PairSlot *__restrict__ slots, int t0, int ntiles, int n0,
                                                   const double *__restrict__ delta, const double2 *__restrict__ tab,
@@ -380,8 +385,11 @@ __global__ __launch_bounds__(256) void k_pair_fwd(const PairTile *__restrict__ t
     switch (n >> 3) {
         case 4 * (RT - 1): pair_fwd<RT, 4 * RT - 3>(n, T, sl, delta, tab, x, y); break;
         case 4 * (RT - 1) + 1: pair_fwd<RT, 4 * RT - 2>(n, T, sl, delta, tab, x, y); break;
-        case 4 * (RT - 1) + 2: pair_fwd<RT, 4 * RT - 1>(n, T, sl, delta, tab, x, y); break;
-        default: pair_fwd<RT, 4 * RT>(n, T, sl, delta, tab, x, y);
+        case 4 * (RT - 1) + 2:
+            if constexpr (KSM > 4 * RT - 2) pair_fwd<RT, 4 * RT - 1>(n, T, sl, delta, tab, x, y);
+            break;
+        default:
+            if constexpr (KSM > 4 * RT - 1) pair_fwd<RT, 4 * RT>(n, T, sl, delta, tab, x, y);
     }
 }
 
@@ -624,7 +632,7 @@ __device__ __forceinline__ void pair_back(int n, const PairSeg &G, const PairTil
         }
 }
 
-template <int RT>
+template <int RT, int KSM>
 __global__ __launch_bounds__(256) void k_pair_back(const PairTile *__restrict__ tiles,
                                                    const PairSeg *__restrict__ segs, int s0, int nsegs, int n0,
                                                    const double *__restrict__ delta, const double2 *__restrict__ tab,
@@ -640,8 +648,11 @@ __global__ __launch_bounds__(256) void k_pair_back(const PairTile *__restrict__ 
     switch (n >> 3) {
         case 4 * (RT - 1): pair_back<RT, 4 * RT - 3>(n, G, tiles, delta, tab, z, w); break;
         case 4 * (RT - 1) + 1: pair_back<RT, 4 * RT - 2>(n, G, tiles, delta, tab, z, w); break;
-        case 4 * (RT - 1) + 2: pair_back<RT, 4 * RT - 1>(n, G, tiles, delta, tab, z, w); break;
-        default: pair_back<RT, 4 * RT>(n, G, tiles, delta, tab, z, w);
+        case 4 * (RT - 1) + 2:
+            if constexpr (KSM > 4 * RT - 2) pair_back<RT, 4 * RT - 1>(n, G, tiles, delta, tab, z, w);
+            break;
+        default:
+            if constexpr (KSM > 4 * RT - 1) pair_back<RT, 4 * RT>(n, G, tiles, delta, tab, z, w);
     }
 }
 
@@ -687,18 +698,35 @@ void launch_pair_tables(const PairTile *tiles, const PairSlot *slots, int t0, in
                        slots, t0, quad, tab);
 }
 
+// Calls launch(KSM, first degree, degrees) for the degrees up to 31: by range from 512 waves a
+// degree, else at once (small calls are bound by launches).  Near field of 2500 spheres,
+// orders up to 23, forward and backward: 302 + 451 us a chunk in one launch with room for four
+// steps, 270 + 333 with three for the backward one, 270 + 302 by range; a range of its own for
+// degrees up to 7 gave nothing more.
+template <typename F> static void by_steps(int64_t waves, int max_n, F launch) {
+    const int lo = std::min(max_n, 31);
+    if (waves < 512) {
+        launch(std::max(2, (lo >> 3) + 1), 1, lo);
+        return;
+    }
+    launch(2, 1, std::min(lo, 15));
+    if (lo > 15) launch(3, 16, std::min(lo, 23) - 15);
+    if (lo > 23) launch(4, 24, lo - 23);
+}
+
 void launch_pair_fwd(const PairTile *tiles, const PairSlot *slots, int t0, int ntiles, int max_Ls, const double *delta,
                      const double2 *tab, const double2 *src, int64_t src_stride, double *Y, int64_t y_stride, int nrhs,
                      hipStream_t s) {
     if (ntiles <= 0) return;
-    const int lo = max_Ls < 31 ? max_Ls : 31;
-    hipLaunchKernelGGL(k_pair_fwd<1>, dim3((ntiles + 3) / 4, lo, nrhs), dim3(256), 0, s, tiles, slots, t0, ntiles, 1,
-                       delta, tab, src, src_stride, Y, y_stride);
+    by_steps((int64_t)ntiles * nrhs, max_Ls, [&](int ksm, int n0, int cnt) {
+        auto k = ksm == 2 ? k_pair_fwd<1, 2> : ksm == 3 ? k_pair_fwd<1, 3> : k_pair_fwd<1, 4>;
+        hipLaunchKernelGGL(k, dim3((ntiles + 3) / 4, cnt, nrhs), dim3(256), 0, s, tiles, slots, t0, ntiles, n0, delta,
+                           tab, src, src_stride, Y, y_stride);
+    });
     if (max_Ls > 31)
-        hipLaunchKernelGGL(k_pair_fwd<2>, dim3((ntiles + 3) / 4, max_Ls - 31, nrhs), dim3(256), 0, s, tiles, slots, t0,
-                           ntiles, 32, delta, tab, src, src_stride, Y, y_stride);
+        hipLaunchKernelGGL((k_pair_fwd<2, 8>), dim3((ntiles + 3) / 4, max_Ls - 31, nrhs), dim3(256), 0, s, tiles, slots,
+                           t0, ntiles, 32, delta, tab, src, src_stride, Y, y_stride);
 }
-
 void launch_pair_axial(const PairTile *tiles, const PairSlot *slots, const PairGroup *groups, int ngroups,
                        const int32_t *order, int waves, int max_K, int max_L, int NL, const double *quad,
                        const double2 *tab, const double2 *wax, const double *Y, int64_t y_stride, double *Z,
@@ -723,14 +751,15 @@ void launch_pair_back(const PairTile *tiles, const PairSeg *segs, int s0, int ns
                       const double2 *tab, const double *Z, int64_t z_stride, double2 *W, int64_t w_stride, int nrhs,
                       hipStream_t s) {
     if (nsegs <= 0) return;
-    const int lo = max_Lt < 31 ? max_Lt : 31;
-    hipLaunchKernelGGL(k_pair_back<1>, dim3((nsegs + 3) / 4, lo, nrhs), dim3(256), 0, s, tiles, segs, s0, nsegs, 1,
-                       delta, tab, Z, z_stride, W, w_stride);
+    by_steps((int64_t)nsegs * nrhs, max_Lt, [&](int ksm, int n0, int cnt) {
+        auto k = ksm == 2 ? k_pair_back<1, 2> : ksm == 3 ? k_pair_back<1, 3> : k_pair_back<1, 4>;
+        hipLaunchKernelGGL(k, dim3((nsegs + 3) / 4, cnt, nrhs), dim3(256), 0, s, tiles, segs, s0, nsegs, n0, delta, tab,
+                           Z, z_stride, W, w_stride);
+    });
     if (max_Lt > 31)
-        hipLaunchKernelGGL(k_pair_back<2>, dim3((nsegs + 3) / 4, max_Lt - 31, nrhs), dim3(256), 0, s, tiles, segs, s0,
-                           nsegs, 32, delta, tab, Z, z_stride, W, w_stride);
+        hipLaunchKernelGGL((k_pair_back<2, 8>), dim3((nsegs + 3) / 4, max_Lt - 31, nrhs), dim3(256), 0, s, tiles, segs,
+                           s0, nsegs, 32, delta, tab, Z, z_stride, W, w_stride);
 }
-
 void launch_pair_reduce(const PairTarget *targets, const PairSeg *segs, int g0, int ntargets, int max_Lt,
                         const double2 *W, int64_t w_stride, double2 *dst, int64_t dst_stride, int nrhs, hipStream_t s) {
     if (ntargets <= 0) return;
