@@ -1128,6 +1128,7 @@ static int create_impl(ifs_ctx **out, const ifs_cluster *cl, const ifs_params *p
         if (pair_takes(B.tasks)) {
             c->pair = new (std::nothrow) PairBatch();
             if (!c->pair) return fail(IFS_E_NOMEM);
+            c->pair->rows.assign(c->off.begin(), c->off.begin() + ns);
             rc = pair_finalize(c, *c->pair, B.tasks, "direct");
         } else {
             rc = batch_finalize(c, B, std::min<size_t>(c->ws_budget, (size_t)8 << 30), true);
@@ -1189,7 +1190,9 @@ int matvec_impl(ifs_ctx *c, const double2 *x, double2 *b, int normalised, int nr
         launch_pack_in(c->ns, c->N, c->d_Leff.as<int32_t>(), c->d_off.as<int64_t>(), snm, x, c->d_xh.as<double2>(),
                        nrhs, ld, nc, c->stream);
     }
-    {
+    if (!c->fmm && c->pair && (rc = pair_prepare(c, *c->pair, nrhs))) return rc;
+    const bool parts = !c->fmm && c->pair && c->pair->partial;  // sums left to the last kernel
+    if (!parts) {
         Scope s(c, "zero");
         launch_zero(c->d_acc.as<double2>(), nc * nrhs, c->stream);
     }
@@ -1204,8 +1207,10 @@ int matvec_impl(ifs_ctx *c, const double2 *x, double2 *b, int normalised, int nr
     {
         Scope s(c, "finalize");
         launch_finalize(c->ns, c->N, c->d_Leff.as<int32_t>(), c->d_active.as<int32_t>(), c->d_off.as<int64_t>(),
-                        snm, c->d_an.as<double2>(), c->d_bn.as<double2>(), x, c->d_acc.as<double2>(), b, nrhs, ld,
-                        ldb, nc, c->stream);
+                        snm, c->d_an.as<double2>(), c->d_bn.as<double2>(), x,
+                        parts ? c->ws_s.as<double2>() : c->d_acc.as<double2>(),
+                        parts ? c->pair->d_parts.as<SphereParts>() : nullptr, b, nrhs, ld, ldb,
+                        parts ? c->pair->chunks[0].n_w : nc, c->stream);
     }
     if (hipPeekAtLastError() != hipSuccess) return IFS_E_HIP;
     return IFS_OK;

@@ -241,9 +241,16 @@ void launch_scatter(const ScatterSeg *segs, int nsegs, const int32_t *cols, cons
 void launch_mie(int ns, const double *xsize, const double2 *mrel, int N, double2 *an, double2 *bn, hipStream_t s);
 void launch_pack_in(int ns, int N, const int32_t *Leff, const int64_t *off, const double *snm, const double2 *x,
                     double2 *xh, int nrhs, int64_t ldx, int64_t ldxh, hipStream_t s);
+// A sphere's partial sums: `count` blocks of its 2 L (L + 2) entries from `off`.
+struct SphereParts {
+    int64_t off;
+    int32_t count, pad_;
+};
+// acc: the spheres' sums at off, or with `parts` their partial sums.
 void launch_finalize(int ns, int N, const int32_t *Leff, const int32_t *active, const int64_t *off,
                      const double *snm, const double2 *an, const double2 *bn, const double2 *x, const double2 *acc,
-                     double2 *b, int nrhs, int64_t ldx, int64_t ldb, int64_t ldacc, hipStream_t s);
+                     const SphereParts *parts, double2 *b, int nrhs, int64_t ldx, int64_t ldb, int64_t ldacc,
+                     hipStream_t s);
 void launch_zero(double2 *p, int64_t n, hipStream_t s);
 void launch_scale_flat(int ns, int N, const double *snm, const double2 *x, double2 *y, int inverse, hipStream_t s);
 

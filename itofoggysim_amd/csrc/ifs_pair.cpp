@@ -216,6 +216,15 @@ int pair_plan(ifs_ctx *c, PairBatch &B, int nrhs) {
         ch.a1 = (int)B.groups.size();
         B.order.insert(B.order.end(), o.begin(), o.end());
     }
+    B.partial = !B.rows.empty() && B.chunks.size() == 1;
+    std::vector<SphereParts> parts;
+    if (B.partial) {
+        std::map<int64_t, size_t> at;
+        for (size_t j = 0; j < B.rows.size(); ++j) at[B.rows[j]] = j;
+        parts.assign(B.rows.size(), SphereParts{0, 0, 0});
+        for (const PairTarget &T : B.targets)
+            parts[at[T.dst]] = SphereParts{B.segs[T.s_begin].off_w, T.s_end - T.s_begin, 0};
+    }
     int64_t my = 0, mz = 0, mw = 0, mt = 0, ma = 0, ms = 0;
     for (auto &ch : B.chunks) {
         my = std::max(my, ch.n_y);
@@ -236,6 +245,7 @@ int pair_plan(ifs_ctx *c, PairBatch &B, int nrhs) {
         (rc = upload(B.d_segs, B.segs.data(), sizeof(PairSeg) * B.segs.size())) ||
         (rc = upload(B.d_targets, B.targets.data(), sizeof(PairTarget) * B.targets.size())) ||
         (rc = upload(B.d_groups, B.groups.data(), sizeof(PairGroup) * B.groups.size())) ||
+        (B.partial && (rc = upload(B.d_parts, parts.data(), sizeof(SphereParts) * parts.size()))) ||
         (rc = upload(B.d_order, B.order.data(), 4 * B.order.size())) ||
         (rc = upload(B.d_close, B.close.data(), sizeof(Task) * B.close.size())))
         return rc;
@@ -304,13 +314,16 @@ int pair_finalize(ifs_ctx *c, PairBatch &B, std::vector<Task> &tasks, const char
     return pair_plan(c, B, 1);
 }
 
+int pair_prepare(ifs_ctx *c, PairBatch &B, int nrhs) {
+    if (B.plan_nrhs == nrhs) return IFS_OK;
+    if (hipStreamSynchronize(c->stream) != hipSuccess) return IFS_E_HIP;
+    return pair_plan(c, B, nrhs);
+}
+
 int pair_run(ifs_ctx *c, PairBatch &B, const double2 *src_pool, double2 *dst_pool, int nrhs, int64_t src_stride,
              int64_t dst_stride) {
-    if (B.plan_nrhs != nrhs) {
-        if (hipStreamSynchronize(c->stream) != hipSuccess) return IFS_E_HIP;
-        int rc = pair_plan(c, B, nrhs);
-        if (rc) return rc;
-    }
+    int rc = pair_prepare(c, B, nrhs);
+    if (rc) return rc;
     const PairTile *tiles = B.d_tiles.as<PairTile>();
     const PairSlot *slots = B.d_slots.as<PairSlot>();
     const PairSeg *segs = B.d_segs.as<PairSeg>();
@@ -345,8 +358,9 @@ int pair_run(ifs_ctx *c, PairBatch &B, const double2 *src_pool, double2 *dst_poo
             Scope s(c, B.pn[3], ch.f_back * nrhs);
             launch_pair_back(tiles, segs, ch.s0, ch.s1 - ch.s0, ch.max_Lt, delta, tab, Z, ch.n_z, W, ch.n_w, nrhs,
                              c->stream);
-            launch_pair_reduce(B.d_targets.as<PairTarget>(), segs, ch.g0, ch.g1 - ch.g0, ch.max_Lt, W, ch.n_w,
-                               dst_pool, dst_stride, nrhs, c->stream);
+            if (!B.partial)
+                launch_pair_reduce(B.d_targets.as<PairTarget>(), segs, ch.g0, ch.g1 - ch.g0, ch.max_Lt, W,
+                                   ch.n_w, dst_pool, dst_stride, nrhs, c->stream);
         }
     }
     if (hipPeekAtLastError() != hipSuccess) return IFS_E_HIP;
@@ -356,7 +370,7 @@ int pair_run(ifs_ctx *c, PairBatch &B, const double2 *src_pool, double2 *dst_poo
 
 uint64_t pair_sig(const PairBatch &B) {
     uint64_t h = (uint64_t)B.plan_nrhs;
-    for (const DevBuf *d : {&B.d_tiles, &B.d_slots, &B.d_segs, &B.d_targets, &B.d_close, &B.d_groups, &B.d_order, &B.d_delta, &B.d_quad,
+    for (const DevBuf *d : {&B.d_tiles, &B.d_slots, &B.d_segs, &B.d_targets, &B.d_parts, &B.d_close, &B.d_groups, &B.d_order, &B.d_delta, &B.d_quad,
                             &B.own_tab, &B.own_ax})
         h ^= (uint64_t)(uintptr_t)d->p + 0x9e3779b97f4a7c15ull + (h << 6) + (h >> 2);
     return h;

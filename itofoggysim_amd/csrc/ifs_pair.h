@@ -67,6 +67,11 @@ struct PairBatch {
     DevBuf d_delta, d_quad;   // shared matrices
     DevBuf own_tab, own_ax;   // tables kept across matvecs
     bool kept = false, ready = false;
+    // Offsets of the spheres' sums, where the caller can take partial sums: with all tiles in
+    // one chunk no pass adds them, and parts holds those of every sphere.
+    std::vector<int64_t> rows;
+    DevBuf d_parts;
+    bool partial = false;
     int plan_nrhs = 0;
     int NL = 0;               // orders of the shared matrices
     std::vector<Task> tasks;  // the translations, sorted by target
@@ -79,6 +84,8 @@ struct PairBatch {
 bool pair_takes(const std::vector<Task> &tasks);
 // Takes the tasks over and plans them for one right-hand side.
 int pair_finalize(ifs_ctx *c, PairBatch &B, std::vector<Task> &tasks, const char *name);
+// Plans again where the number of right-hand sides changed.
+int pair_prepare(ifs_ctx *c, PairBatch &B, int nrhs);
 int pair_run(ifs_ctx *c, PairBatch &B, const double2 *src_pool, double2 *dst_pool, int nrhs, int64_t src_stride,
              int64_t dst_stride);
 uint64_t pair_sig(const PairBatch &B);
