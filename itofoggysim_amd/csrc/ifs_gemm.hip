@@ -639,6 +639,67 @@ __global__ __launch_bounds__(256) void k_class_axial(const GroupDesc *__restrict
         }
 }
 
+// The same shift where it carries the last degrees only (n0 > 1, at most kRemDegrees rows):
+// thread per translation, 8 rows n at a time in registers, P and Q from scalar registers.  A
+// 64-row block of the product kernel above costs 10 us whatever the rows it holds (loads and
+// stores through two resident blocks a CU); FP64 FMAs run at the matrix cores' rate.  Bound by
+// the scalar loads of P and Q.  Box translations of 2500 spheres (24 and 9 last degrees of 97):
+// 1302 -> 768 us, of 3000 small-order spheres (1 to 23 of 45): 1100 -> 508 us.  With 41 and
+// 50 degrees the 64-row blocks are the faster (474 against 591 us).
+constexpr int kRemDegrees = 32, RR = 8;
+template <typename TC>
+__global__ __launch_bounds__(256) void k_class_axial_rem(const GroupDesc *__restrict__ desc,
+                                                         const double2 *__restrict__ wax, const TC *__restrict__ wy,
+                                                         TC *__restrict__ wz) {
+    const GroupDesc C = *desc;
+    const int K = C.K;
+    const int k = (int)blockIdx.z - K;
+    const int ak = k < 0 ? -k : k;
+    const int q = ak < C.n0 ? C.n0 : ak;
+    const int Lt = C.Lt, Ls = C.Ls;
+    const int M = Lt - q + 1, KI = Ls - q + 1;
+    const int row0 = blockIdx.y * RR;
+    if (row0 >= M) return;
+    const int NC = 4 * C.ncy * C.nrhs, NTOT = C.ncols * C.nrhs;
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= NTOT) return;
+    const double2 *Pb = wax + C.off_ax + ax0_off(k, Lt, C.n0);
+    const double2 *Qb = Pb + (int64_t)M * KI;
+    const int64_t rbase = rows_off(C.n0, K), cb = 4 * ((int64_t)C.ycol0 * C.nrhs + t);
+    TC z[RR][4];
+#pragma unroll
+    for (int r = 0; r < RR; ++r)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) z[r][i] = 0;
+    for (int c = 0; c < KI; ++c) {
+        const int nu = q + c;
+        const TC *y = wy + (rows_off(nu, K) - rbase + k + (nu < K ? nu : K)) * NC + cb;
+        const TC y0 = y[0], y1 = y[1], y2 = y[2], y3 = y[3];
+#pragma unroll
+        for (int r = 0; r < RR; ++r) {
+            const int gr = row0 + r < M ? row0 + r : M - 1;  // rows beyond M are not stored
+            const double2 pd = Pb[(int64_t)gr * KI + c], qd = Qb[(int64_t)gr * KI + c];
+            const TC px = (TC)pd.x, py = (TC)pd.y, qx = (TC)qd.x, qy = (TC)qd.y;
+            z[r][0] += px * y0;
+            z[r][0] -= py * y1;
+            z[r][1] += px * y1;
+            z[r][1] += py * y0;
+            z[r][2] += qx * y2;
+            z[r][2] -= qy * y3;
+            z[r][3] += qx * y3;
+            z[r][3] += qy * y2;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < RR; ++r) {
+        const int n = q + row0 + r;
+        if (n > Lt) break;
+        TC *o = wz + (rows_off(n, K) - rbase + (k + (n < K ? n : K))) * (int64_t)NC + cb;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = z[r][i];
+    }
+}
+
 // Deterministic per-target sum of back-rotated columns: grid (targets, element blocks).
 // grid (targets, element blocks, right-hand sides).
 __global__ __launch_bounds__(256) void k_scatter(const ScatterSeg *__restrict__ segs, const int32_t *__restrict__ cols,
@@ -677,6 +738,10 @@ static void launch_class_t(const GroupDesc &h, const GroupDesc *d_desc, const in
         else
             hipLaunchKernelGGL((k_class_rot_fwd<TC, TW, FMF, 3>), grid, dim3(256), 0, s, d_desc, src_off, pidx, phase,
                                src_pool, wd, wy);
+    } else if (stage == 1 && h.n0 > 1 && h.Lt - h.n0 < kRemDegrees) {
+        hipLaunchKernelGGL(k_class_axial_rem<TC>,
+                           dim3((h.ncols * h.nrhs + 255) / 256, (h.Lt - h.n0 + RR) / RR, 2 * K + 1), dim3(256), 0, s,
+                           d_desc, wax, (const TC *)wy, wz);
     } else if (stage == 1) {
         int mt = (h.Lt - h.n0 + 1 + AM - 1) / AM;
         const int nt = h.ncols * h.nrhs;
