@@ -454,8 +454,9 @@ def main():
         "rel_error_vs_fp64_normalised": mixed_err,
         "kernels_ms": {k: round(v[0], 2) for k, v in prof32.items()},
         "kernels_tflops": {k: round(v[2] / (v[0] * 1e-3) / 1e12, 2) for k, v in prof32.items() if v[2] > 0 and v[0] > 0},
-        "note": "M2M/M2L/L2L as FP32 matrix-core products (FP32 accumulation) on the FP64 tables; "
-                "sphere-level translations, T-apply and vectors FP64; FP32 peak 157.3 TFLOP/s"}
+        "note": "M2M, L2L and M2L's class products as FP32 matrix-core products (FP32 accumulation) on the FP64 "
+                "tables, plane-wave M2L tables in FP32; samples, sphere-level translations, T-apply and vectors "
+                "FP64; FP32 peak 157.3 TFLOP/s"}
     if not args.no_solve:
         rhs = torch.from_numpy(s.get_vector_b()).to("cuda")
         # the single-sphere solution of (I + T A) x = T p is x_j = T_j p_j, the right-hand side itself

@@ -75,8 +75,9 @@ typedef struct {
 
 /* Precision of a matvec or of a solve's Krylov products:
  *   IFS_PREC_FP64   FP64 throughout;
- *   IFS_PREC_MIXED  the box translations (M2M, M2L, L2L: the MLFMM's dense products) run
- *                   as FP32 matrix-core products with FP32 accumulation on the FP64 tables;
+ *   IFS_PREC_MIXED  the MLFMM's dense box products (M2M, L2L, the class products of M2L) run
+ *                   as FP32 matrix-core products with FP32 accumulation on the FP64 tables, and
+ *                   the plane-wave M2L reads its tables in FP32 (samples and sums FP64);
  *                   sphere-level translations, T-apply, vectors and solver state stay FP64. */
 #define IFS_PREC_FP64 0
 #define IFS_PREC_MIXED 1
@@ -161,8 +162,8 @@ int ifs_far_field(ifs_ctx *ctx, const double *x, int64_t n, int32_t ndir, const 
                   double *out);
 int ifs_far_field_device(ifs_ctx *ctx, const void *x_dev, int64_t n, int32_t ndir, const void *theta_dev,
                          const void *phi_dev, void *out_dev);
-/* Far field as ifs_far_field_device, allocating nothing: the per-direction tables go to
- * a fixed device array of the library, IFS_FF_SCRATCH_ENTRIES complex (32 MiB) on every GPU
+/* Far field as ifs_far_field_device, allocating nothing: the per-direction tables (and, as
+ * far as there is room, parts of the sums) go to a fixed device array of the library, IFS_FF_SCRATCH_ENTRIES complex (32 MiB) on every GPU
  * the library runs on, held until the process ends; the sphere centres are kept in the
  * context.  ndir * N(N+2) must not exceed IFS_FF_SCRATCH_ENTRIES (else IFS_E_ARG and nothing
  * runs: split the directions).  Enqueued on the context stream, no synchronisation.  All
