@@ -1140,6 +1140,9 @@ static int create_impl(ifs_ctx **out, const ifs_cluster *cl, const ifs_params *p
     for (int j = 0; j < ns; ++j) c->flops_mv += 12.0 * c->Leff[j] * (c->Leff[j] + 2);
     c->flops_mv += 4.0 * (double)c->nflat;
     c->bytes_mv += 2.0 * 16.0 * (double)c->nflat;
+    // the plans' shared matrices are made on the context's own stream, which is not ordered
+    // against the one a caller may set next
+    if (hipStreamSynchronize(c->stream) != hipSuccess) return fail(IFS_E_HIP);
     *out = c;
     return IFS_OK;
 }
