@@ -98,6 +98,21 @@ static void task_flops(const Task &T, double &ffwd, double &fax, double &fback) 
     for (int k = -T.K; k <= T.K; ++k) fax += 16.0 * (double)ax_block(k, T.Lt, T.Ls);
 }
 
+int ws_reserve(ifs_ctx *c, const WsNeed &need) {
+    const std::pair<DevBuf *, size_t> all[] = {{&c->ws_d, need.d}, {&c->ws_s, need.s}, {&c->ws_ax, need.ax},
+                                               {&c->ws_y, need.y}, {&c->ws_z, need.z}, {&c->ws_gq, need.gq}};
+    for (auto &q : all) {
+        const size_t old = q.first->bytes;
+        if (q.second <= old) continue;
+        const int rc = q.first->alloc(q.second);
+        if (rc) {
+            (void)q.first->alloc(old);
+            return rc;
+        }
+    }
+    return IFS_OK;
+}
+
 // Split a target-sorted task list into segments and workspace chunks and upload it.
 // The tables are kept across matvecs when they fit the context's cache budget.
 int batch_finalize(ifs_ctx *c, Batch &B, size_t budget_bytes, bool allow_cache) {
@@ -216,7 +231,7 @@ int batch_finalize(ifs_ctx *c, Batch &B, size_t budget_bytes, bool allow_cache) 
             if ((rc = gq_rule(c, ch.gqb.Q, &mu, &w)) != IFS_OK) return rc;
             vb = std::max(vb, (size_t)(ch.gqb.maxK + 1) * (ch.gqb.Nr + 1) * ch.gqb.Q * 8);
         }
-        if ((rc = c->ws_gq.alloc(std::max(c->ws_gq.bytes, vb))) != IFS_OK) return rc;
+        B.ws.gq = vb;
     }
     if (B.cached) {
         if ((rc = B.own_d.alloc(md * 8)) || (rc = B.own_s.alloc(ms * 16)) || (rc = B.own_ax.alloc(ma * 16)) ||
@@ -224,12 +239,13 @@ int batch_finalize(ifs_ctx *c, Batch &B, size_t budget_bytes, bool allow_cache) 
             return rc;
         c->ws_cached += (size_t)(md * 8 + (ms + ma + my + mz) * 16);
     } else {
-        if ((rc = c->ws_d.alloc(std::max<size_t>(c->ws_d.bytes, md * 8))) != IFS_OK) return rc;
-        if ((rc = c->ws_s.alloc(std::max<size_t>(c->ws_s.bytes, ms * 16))) != IFS_OK) return rc;
-        if ((rc = c->ws_ax.alloc(std::max<size_t>(c->ws_ax.bytes, ma * 16))) != IFS_OK) return rc;
-        if ((rc = c->ws_y.alloc(std::max<size_t>(c->ws_y.bytes, my * 16))) != IFS_OK) return rc;
-        if ((rc = c->ws_z.alloc(std::max<size_t>(c->ws_z.bytes, mz * 16))) != IFS_OK) return rc;
+        B.ws.d = md * 8;
+        B.ws.s = ms * 16;
+        B.ws.ax = ma * 16;
+        B.ws.y = my * 16;
+        B.ws.z = mz * 16;
     }
+    if ((rc = ws_reserve(c, B.ws)) != IFS_OK) return rc;
     if ((rc = B.d_tasks.alloc(sizeof(Task) * std::max<size_t>(1, n))) != IFS_OK) return rc;
     if ((rc = B.d_segs.alloc(sizeof(Segment) * std::max<size_t>(1, B.segs.size()))) != IFS_OK) return rc;
     if (n) HIP_OK(hipMemcpy(B.d_tasks.p, B.tasks.data(), sizeof(Task) * n, hipMemcpyHostToDevice));
@@ -255,6 +271,7 @@ Scope::~Scope() {
 
 int batch_run(ifs_ctx *c, Batch &B, const double2 *src_pool, double2 *dst_pool, int nrhs, int64_t src_stride,
               int64_t dst_stride) {
+    if (int rc = ws_reserve(c, B.ws)) return rc;
     const Task *dt = B.d_tasks.as<Task>();
     double *wd = B.cached ? B.own_d.as<double>() : c->ws_d.as<double>();
     double2 *wsc = B.cached ? B.own_s.as<double2>() : c->ws_s.as<double2>();
@@ -551,6 +568,7 @@ int class_batches_prepare(ifs_ctx *c, const std::vector<ClassBatch *> &bs) {
 }
 
 int class_batch_plan(ifs_ctx *c, ClassBatch &B, int nrhs) {
+    B.plan_nrhs = 0;
     B.chunks.clear();
     B.descs.clear();
     B.scat.clear();
@@ -689,12 +707,12 @@ int class_batch_plan(ifs_ctx *c, ClassBatch &B, int nrhs) {
             B.descs[P.di] = P.g;
         }
     }
-    if ((rc = c->ws_d.alloc(std::max<size_t>(c->ws_d.bytes, B.n_d * 8 * (size_t)B.n_dslots))) ||
-        (rc = c->ws_gq.alloc(std::max<size_t>(c->ws_gq.bytes, gq_ws))) ||
-        (rc = c->ws_ax.alloc(std::max<size_t>(c->ws_ax.bytes, B.ax_persist ? 16 : B.n_ax * 16))) ||
-        (rc = c->ws_y.alloc(std::max<size_t>(c->ws_y.bytes, B.n_y * 8))) ||
-        (rc = c->ws_z.alloc(std::max<size_t>(c->ws_z.bytes, B.n_z * 8))))
-        return rc;
+    B.ws.d = B.n_d * 8 * (size_t)B.n_dslots;
+    B.ws.gq = gq_ws;
+    B.ws.ax = B.ax_persist ? 16 : B.n_ax * 16;
+    B.ws.y = B.n_y * 8;
+    B.ws.z = B.n_z * 8;
+    if ((rc = ws_reserve(c, B.ws))) return rc;
     auto up = [](DevBuf &d, const void *h, size_t bytes) -> int {
         int r = d.alloc(std::max<size_t>(bytes, 16));
         if (r) return r;
@@ -741,6 +759,7 @@ int class_batch_run(ifs_ctx *c, ClassBatch &B, const double2 *src_pool, double2 
         int rc = class_batch_plan(c, B, nrhs);
         if (rc) return rc;
     }
+    if (int rc = ws_reserve(c, B.ws)) return rc;
     const GroupDesc *dd = B.d_desc.as<GroupDesc>();
     const Task *dg = B.d_gen.as<Task>();
     const Task *dk = B.d_dkeys.as<Task>();

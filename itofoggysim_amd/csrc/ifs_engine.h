@@ -29,6 +29,7 @@ struct DevBuf {
         bytes = 0;
         if (b == 0) return IFS_OK;
         if (hipMalloc(&p, b) != hipSuccess) {
+            (void)hipGetLastError();  // reported here, not by the next launch's check
             p = nullptr;
             return IFS_E_NOMEM;
         }
@@ -36,6 +37,11 @@ struct DevBuf {
         return IFS_OK;
     }
     template <class T> T *as() const { return (T *)p; }
+};
+
+// What a plan needs of the context's shared translation workspaces (bytes).
+struct WsNeed {
+    size_t d = 0, s = 0, ax = 0, y = 0, z = 0, gq = 0;
 };
 
 // Chunk of a translation batch that fits the workspace.
@@ -55,6 +61,7 @@ struct Batch {
     std::vector<Task> tasks;     // sorted by target
     std::vector<Segment> segs;
     std::vector<Chunk> chunks;
+    WsNeed ws;
     DevBuf d_tasks, d_segs;
     DevBuf own_d, own_s, own_ax, own_y, own_z;  // workspace of a cached batch
     bool cached = false;         // tables generated once and kept
@@ -178,6 +185,10 @@ struct ifs_ctx {
 
 
 namespace ifs {
+// Grows the shared workspaces to what a plan needs; every run asks before it takes their
+// addresses.  One that cannot grow gets its old size back for the plans that fit it, and
+// where even that fails the next run that needs it asks again.
+int ws_reserve(ifs_ctx *c, const WsNeed &need);
 // Device address of the far-field scratch array on the current device (looked up
 // once per device); ifs_create calls it with the context's device current.
 int far_field_scratch(int device, void **out);
@@ -212,7 +223,8 @@ struct ClassBatch {
     int PL = 0;
     int n0 = 1;                        // lowest degree carried: > 1 for the part of an offset that the plane
                                        // waves leave (terms p >= n0 + L of h1; orders Ls = Lt = K)
-    int plan_nrhs = 0;                 // right-hand sides the plan was cut for
+    int plan_nrhs = 0;                 // right-hand sides the plan was cut for, 0: no valid plan
+    WsNeed ws;
     int n_dslots = 1;                  // Wigner tables kept at once (chunk runs share slots r % n_dslots)
     // Table keys: one Wigner table per |cos(theta)| (a run of cos(theta) < 0 mirrors
     // it), one coaxial table per (length, kind).  When the context's cache budget

@@ -63,15 +63,19 @@ void box_matrices(ifs_ctx *c, Leaf &F, LeafArg &a, const PwLevel::Chunk &ch, siz
     }
 }
 
+// The plan for nrhs right-hand sides and its workspaces.
 int replan(ifs_ctx *c, Leaf &F, int nrhs) {
-    if (F.g.plan_nrhs == nrhs) return IFS_OK;
-    if (hipStreamSynchronize(c->stream) != hipSuccess) return IFS_E_HIP;
-    int rc = pw_plan(c, F.g, nrhs);
-    if (rc) return rc;
-    // row coefficients of the spheres: an eighth of the workspace, at least one sphere
-    const int64_t per = row_coefs(F) * nrhs;
-    F.gcap = std::max<int64_t>(1, std::min<int64_t>((int64_t)std::max(F.up.size(), F.down.size()), (int64_t)(c->ws_budget / 8 / 16) / per));
-    return c->ws_s.alloc(std::max<size_t>(c->ws_s.bytes, 16 * (size_t)(F.gcap * per)));
+    if (F.g.plan_nrhs != nrhs) {
+        if (hipStreamSynchronize(c->stream) != hipSuccess) return IFS_E_HIP;
+        // row coefficients of the spheres: an eighth of the workspace, at least one sphere
+        const int64_t per = row_coefs(F) * nrhs;
+        F.gcap = std::max<int64_t>(1, std::min<int64_t>((int64_t)std::max(F.up.size(), F.down.size()),
+                                                        (int64_t)(c->ws_budget / 8 / 16) / per));
+        F.g.ws.s = 16 * (size_t)(F.gcap * per);
+        int rc = pw_plan(c, F.g, nrhs);
+        if (rc) return rc;
+    }
+    return ws_reserve(c, F.g.ws);
 }
 
 int group_rhs(ifs_ctx *c, const Leaf &F, int nrhs) {

@@ -75,6 +75,7 @@ void build_tiles(PairBatch &B, std::map<int, int64_t> &quads) {
 
 // Chunks, segments and per-chunk target lists; workspace offsets.
 int pair_plan(ifs_ctx *c, PairBatch &B, int nrhs) {
+    B.plan_nrhs = 0;
     B.chunks.clear();
     B.segs.clear();
     B.targets.clear();
@@ -235,11 +236,12 @@ int pair_plan(ifs_ctx *c, PairBatch &B, int nrhs) {
         ms = std::max(ms, ch.n_s);
     }
     int rc;
-    auto grow = [](DevBuf &d, size_t b) { return d.alloc(std::max(d.bytes, std::max<size_t>(b, 16))); };
-    if ((rc = grow(c->ws_y, 8 * (size_t)my * nrhs)) || (rc = grow(c->ws_z, 8 * (size_t)mz * nrhs)) ||
-        (rc = grow(c->ws_s, 16 * std::max<size_t>((size_t)mw * nrhs, (size_t)ms))))
-        return rc;
-    if (!B.kept && ((rc = grow(c->ws_d, 16 * (size_t)mt)) || (rc = grow(c->ws_ax, 16 * (size_t)ma)))) return rc;
+    B.ws.y = 8 * (size_t)my * nrhs;
+    B.ws.z = 8 * (size_t)mz * nrhs;
+    B.ws.s = 16 * std::max<size_t>((size_t)mw * nrhs, (size_t)ms);
+    B.ws.d = B.kept ? 0 : 16 * (size_t)mt;
+    B.ws.ax = B.kept ? 0 : 16 * (size_t)ma;
+    if ((rc = ws_reserve(c, B.ws))) return rc;
     if ((rc = upload(B.d_tiles, B.tiles.data(), sizeof(PairTile) * B.tiles.size())) ||
         (rc = upload(B.d_slots, B.slots.data(), sizeof(PairSlot) * B.slots.size())) ||
         (rc = upload(B.d_segs, B.segs.data(), sizeof(PairSeg) * B.segs.size())) ||
@@ -323,7 +325,7 @@ int pair_prepare(ifs_ctx *c, PairBatch &B, int nrhs) {
 int pair_run(ifs_ctx *c, PairBatch &B, const double2 *src_pool, double2 *dst_pool, int nrhs, int64_t src_stride,
              int64_t dst_stride) {
     int rc = pair_prepare(c, B, nrhs);
-    if (rc) return rc;
+    if (rc || (rc = ws_reserve(c, B.ws))) return rc;
     const PairTile *tiles = B.d_tiles.as<PairTile>();
     const PairSlot *slots = B.d_slots.as<PairSlot>();
     const PairSeg *segs = B.d_segs.as<PairSeg>();

@@ -72,7 +72,8 @@ struct PairBatch {
     std::vector<int64_t> rows;
     DevBuf d_parts;
     bool partial = false;
-    int plan_nrhs = 0;
+    int plan_nrhs = 0;        // right-hand sides the plan was cut for, 0: no valid plan
+    WsNeed ws;
     int NL = 0;               // orders of the shared matrices
     std::vector<Task> tasks;  // the translations, sorted by target
     double cost_flops = 0.0, cost_bytes = 0.0;

@@ -220,6 +220,7 @@ int pw_build(ifs_ctx *c, PwLevel &P, int isg) {
 }
 
 int pw_plan(ifs_ctx *c, PwLevel &P, int nrhs) {
+    P.plan_nrhs = 0;
     const int L = P.L, nc = (int)P.canon.size();
     const int64_t nbr = (int64_t)P.nb * nrhs;
     P.n_x = x_size(L) * nbr;
@@ -255,9 +256,11 @@ int pw_plan(ifs_ctx *c, PwLevel &P, int nrhs) {
         j += ch.R2;
     }
     int rc;
-    auto grow = [](DevBuf &d, size_t b) { return d.alloc(std::max(d.bytes, b)); };
-    if ((rc = grow(c->ws_y, 16 * (size_t)(2 * P.n_x + P.n_g))) || (rc = grow(c->ws_z, 32 * (size_t)P.n_f))) return rc;
-    if (!P.kept && ((rc = grow(c->ws_d, 8 * (size_t)P.n_u)) || (rc = grow(c->ws_ax, 16 * (size_t)P.n_t)))) return rc;
+    P.ws.y = 16 * (size_t)(2 * P.n_x + P.n_g);
+    P.ws.z = 32 * (size_t)P.n_f;
+    P.ws.d = P.kept ? 0 : 8 * (size_t)P.n_u;
+    P.ws.ax = P.kept ? 0 : 16 * (size_t)P.n_t;
+    if ((rc = ws_reserve(c, P.ws))) return rc;
     if ((rc = upload(P.d_cpre, cpre.data(), 8 * cpre.size()))) return rc;
     P.plan_nrhs = nrhs;
     return IFS_OK;
@@ -294,6 +297,7 @@ int pw_run(ifs_ctx *c, PwLevel &P, const double2 *C, double2 *D, int nrhs, int64
             int rc = pw_plan(c, P, nr);
             if (rc) return rc;
         }
+        if (int rc = ws_reserve(c, P.ws)) return rc;
         hipStream_t s = c->stream;
         const int L = P.L, nc = (int)P.canon.size();
         PwArg a = pw_arg(c, P, nr);

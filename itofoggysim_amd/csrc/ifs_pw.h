@@ -68,7 +68,8 @@ struct PwLevel {
     std::vector<Chunk> chunks;
     DevBuf d_cpre;            // per chunk: prefix of N over its 2 R2 rows, chunk after chunk
     std::vector<int64_t> cpre_at;
-    int plan_nrhs = 0;
+    int plan_nrhs = 0;        // right-hand sides the plan was cut for, 0: no valid plan
+    WsNeed ws;
     int64_t n_x = 0, n_g = 0, n_f = 0, n_u = 0, n_t = 0;  // complex (u: doubles)
     bool active() const { return ncols > 0; }
 };
@@ -89,7 +90,7 @@ bool pw_worth(int L, int nb, int64_t cols);
 int pw_grid(ifs_ctx *c, PwLevel &P, int Q2, double tdeg, int tcap, int order);
 // parents: for every parent box its children and sources; called once per level.
 int pw_build(ifs_ctx *c, PwLevel &P, int isg);
-int pw_plan(ifs_ctx *c, PwLevel &P, int nrhs);
+int pw_plan(ifs_ctx *c, PwLevel &P, int nrhs);  // leaves ws.s as it is
 int pw_run(ifs_ctx *c, PwLevel &P, const double2 *C, double2 *D, int nrhs, int64_t stride, int prec);
 bool pw_fits(ifs_ctx *c, int L, int nb, int nrhs);
 // Algorithmic flops of one product: the two GEMMs (8 Q degrees^2 each way per box), the

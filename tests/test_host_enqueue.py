@@ -23,3 +23,63 @@ stream = own.pop()
 last = max(i for i, c in enumerate(seen) if c[0] == "launch")
 assert ["sync", stream] in seen[last:], seen[last:]
 """)
+
+
+WATCH = """
+pointers = [("k_pair_fwdI", 9, 0), ("k_pair_axialI", 8, 0), ("k_pair_axialI", 10, 0), ("k_pair_backI", 7, 0),
+            ("k_pair_backI", 9, 0), ("k_class_rot_fwd", 5, 0), ("k_class_rot_fwd", 6, 0), ("k_leaf_rows", 5, 0)]
+pointers += [("k_pw_fft", 0, 144 + 8 * i) for i in range(5)]
+for name, arg, offset in pointers:
+    fake.fake_watch(name.encode(), arg, offset)
+def behind(seen):
+    out = {}
+    for c in seen:
+        if c[0] == "arg":
+            key = tuple(c[1:4])
+            out[key] = min(out.get(key, 1 << 62), int(c[4]))
+    return out
+"""
+
+
+@pytest.mark.parametrize("args", ["12, 40.0, 1, 9", "400, 160.0, 1, 9, use_fmm=True, leaf_size=32"])
+def test_a_failed_allocation_leaves_the_context_usable(so, args):
+    """A batched product that runs out of memory at any of its allocations returns an error; the
+    single product after it and the batched one, once there is memory again, find every
+    workspace in place and as large as their plan needs."""
+    n, side, lo, hi, *kw = args.split(", ")
+    host_runtime.run(so, WATCH + f"""
+import numpy as np
+from itofoggysim_amd._lib import IfsError
+def make():
+    return solver(*spheres({n}, {side}, {lo}, {hi}), {", ".join(kw)})
+s = make()
+x = np.zeros((3, s.n), complex)
+fake.calls()
+s.calculate_vector_b(x[0])
+single = behind(fake.calls())
+before = fake.fake_allocs()
+s.calculate_vector_b_batch(x)
+batch = behind(fake.calls())
+count = fake.fake_allocs() - before
+assert single and batch and min(single.values()) > 0 and count > 4
+s.close()
+for granted in range(count):
+    s = make()
+    s.calculate_vector_b(x[0])
+    fake.fake_fail_after(granted)
+    try:
+        s.calculate_vector_b_batch(x)
+        failed = False
+    except IfsError as e:
+        failed = e.code == -2
+    fake.fake_fail_after(-1)
+    assert failed, granted
+    for call, want in ((lambda: s.calculate_vector_b(x[0]), single), (lambda: s.calculate_vector_b_batch(x), batch)):
+        fake.calls()
+        call()
+        got = behind(fake.calls())
+        assert got.keys() == want.keys()
+        assert all(got[k] >= want[k] for k in want if "pair" in k[0]), (granted, got, want)
+        assert min(got.values()) > 0, (granted, got)
+    s.close()
+""")
