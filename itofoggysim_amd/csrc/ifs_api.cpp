@@ -756,6 +756,8 @@ static void remember_rows(const std::array<int, 7> &k, int st, int r) {
 int class_batch_run(ifs_ctx *c, ClassBatch &B, const double2 *src_pool, double2 *dst_pool, int nrhs, int prec) {
     if (B.gen.empty() || nrhs <= 0) return IFS_OK;
     if (B.plan_nrhs != nrhs) {
+        // the kernels of an earlier product read the lists that a new cut replaces
+        if (hipStreamSynchronize(c->stream) != hipSuccess) return IFS_E_HIP;
         int rc = class_batch_plan(c, B, nrhs);
         if (rc) return rc;
     }

@@ -83,3 +83,28 @@ for granted in range(count):
         assert min(got.values()) > 0, (granted, got)
     s.close()
 """)
+
+
+@pytest.mark.parametrize("kw", ["", ", workspace_mb=4"])
+def test_a_new_cut_of_box_translations_waits_for_the_old_one(so, kw):
+    """Products with another number of right-hand sides replace the lists that the kernels of the
+    product before them may still read: no list is written while a launch is outstanding."""
+    host_runtime.run(so, f"""
+s = solver(*spheres(400, 160.0, 1, 9), use_fmm=True, leaf_size=32{kw})
+x, b = (ctypes.create_string_buffer(16 * 3 * s.n) for _ in range(2))
+x, b = ctypes.addressof(x), ctypes.addressof(b)
+replaced = 0
+fake.calls()
+for nrhs in (1, 3, 1, 3):
+    s.calculate_vector_b_batch_device(x, b, nrhs)
+outstanding = False
+for c in fake.calls():
+    if c[0] == "launch":
+        outstanding = True
+    elif c[0] == "sync":
+        outstanding = False
+    elif c[0] == "copy":
+        replaced += 1
+        assert not outstanding, c
+assert replaced > 10
+""")
