@@ -1214,8 +1214,7 @@ int matvec_impl(ifs_ctx *c, const double2 *x, double2 *b, int normalised, int nr
         launch_pack_in(c->ns, c->N, c->d_Leff.as<int32_t>(), c->d_off.as<int64_t>(), snm, x, c->d_xh.as<double2>(),
                        nrhs, ld, nc, c->stream);
     }
-    if (!c->fmm && c->pair && (rc = pair_prepare(c, *c->pair, nrhs))) return rc;
-    const bool parts = !c->fmm && c->pair && c->pair->partial;  // sums left to the last kernel
+    const bool parts = !c->fmm && c->pair && pair_parts(c, *c->pair, nrhs);  // sums left to the last kernel
     if (!parts) {
         Scope s(c, "zero");
         launch_zero(c->d_acc.as<double2>(), nc * nrhs, c->stream);

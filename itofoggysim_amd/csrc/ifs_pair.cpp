@@ -9,7 +9,6 @@ namespace ifs {
 
 namespace {
 
-// Chunk of rotated and shifted columns held at once.
 constexpr size_t kPairChunk = (size_t)1 << 30;
 
 // Largest growth of |h1_p(t)| up to the last order P = Ls + Lt that the quadrature may
@@ -73,14 +72,25 @@ void build_tiles(PairBatch &B, std::map<int, int64_t> &quads) {
     }
 }
 
-// Chunks, segments and per-chunk target lists; workspace offsets.
-int pair_plan(ifs_ctx *c, PairBatch &B, int nrhs) {
-    B.plan_nrhs = 0;
+// Chunk of rotated and shifted columns held at once, of all right-hand sides that run together.
+size_t pair_budget(const ifs_ctx *c) { return std::max<size_t>(std::min(c->ws_budget, kPairChunk), 1); }
+
+WsNeed pair_need(const PairBatch &B, int nrhs) {
+    WsNeed w = B.ws;
+    w.y = 8 * (size_t)B.n_y * nrhs;
+    w.z = 8 * (size_t)B.n_z * nrhs;
+    w.s = 16 * (size_t)std::max<int64_t>(B.n_w * nrhs, B.n_s);
+    return w;
+}
+
+// Chunks, segments and per-chunk target lists; workspace offsets.  Cut for one right-hand
+// side: products of several run as many together as the largest chunk leaves room for.
+int pair_plan(ifs_ctx *c, PairBatch &B) {
     B.chunks.clear();
     B.segs.clear();
     B.targets.clear();
     B.close.clear();
-    const size_t budget = std::max<size_t>(std::min(c->ws_budget, kPairChunk), 1);
+    const size_t budget = pair_budget(c);
     // first tile of every target
     std::vector<size_t> first;
     std::vector<int64_t> dst;
@@ -132,7 +142,7 @@ int pair_plan(ifs_ctx *c, PairBatch &B, int nrhs) {
             size_t bytes = 0;
             for (size_t t = a; t < b; ++t) {
                 const PairTile &T = B.tiles[t];
-                bytes += 128 * (size_t)(rows_size(T.Ls, T.K) + rows_size(T.Lt, T.K)) * nrhs;
+                bytes += 128 * (size_t)(rows_size(T.Ls, T.K) + rows_size(T.Lt, T.K));
                 if (!B.kept) {
                     bytes += 64 * (size_t)T.tabw;
                     for (int s = 0; s < 4 && T.Q == 0; ++s)
@@ -140,7 +150,7 @@ int pair_plan(ifs_ctx *c, PairBatch &B, int nrhs) {
                                                sect_size(B.slots[4 * t + s].K, T.Lt + B.slots[4 * t + s].Ls + 2));
                 }
             }
-            bytes += 32 * (size_t)B.tiles[a].Lt * (B.tiles[a].Lt + 2) * nrhs;
+            bytes += 32 * (size_t)B.tiles[a].Lt * (B.tiles[a].Lt + 2);
             if (used && used + bytes > budget) {
                 close_chunk();
                 open = false;
@@ -217,42 +227,45 @@ int pair_plan(ifs_ctx *c, PairBatch &B, int nrhs) {
         ch.a1 = (int)B.groups.size();
         B.order.insert(B.order.end(), o.begin(), o.end());
     }
-    B.partial = !B.rows.empty() && B.chunks.size() == 1;
     std::vector<SphereParts> parts;
-    if (B.partial) {
+    if (!B.rows.empty() && B.chunks.size() == 1) {
         std::map<int64_t, size_t> at;
         for (size_t j = 0; j < B.rows.size(); ++j) at[B.rows[j]] = j;
         parts.assign(B.rows.size(), SphereParts{0, 0, 0});
         for (const PairTarget &T : B.targets)
             parts[at[T.dst]] = SphereParts{B.segs[T.s_begin].off_w, T.s_end - T.s_begin, 0};
     }
-    int64_t my = 0, mz = 0, mw = 0, mt = 0, ma = 0, ms = 0;
+    B.n_y = B.n_z = B.n_w = B.n_s = 0;
+    int64_t mt = 0, ma = 0;
     for (auto &ch : B.chunks) {
-        my = std::max(my, ch.n_y);
-        mz = std::max(mz, ch.n_z);
-        mw = std::max(mw, ch.n_w);
+        B.n_y = std::max(B.n_y, ch.n_y);
+        B.n_z = std::max(B.n_z, ch.n_z);
+        B.n_w = std::max(B.n_w, ch.n_w);
+        B.n_s = std::max(B.n_s, ch.n_s);
         mt = std::max(mt, ch.n_tab);
         ma = std::max(ma, ch.n_ax);
-        ms = std::max(ms, ch.n_s);
     }
     int rc;
-    B.ws.y = 8 * (size_t)my * nrhs;
-    B.ws.z = 8 * (size_t)mz * nrhs;
-    B.ws.s = 16 * std::max<size_t>((size_t)mw * nrhs, (size_t)ms);
     B.ws.d = B.kept ? 0 : 16 * (size_t)mt;
     B.ws.ax = B.kept ? 0 : 16 * (size_t)ma;
-    if ((rc = ws_reserve(c, B.ws))) return rc;
+    if ((rc = ws_reserve(c, pair_need(B, 1)))) return rc;
     if ((rc = upload(B.d_tiles, B.tiles.data(), sizeof(PairTile) * B.tiles.size())) ||
         (rc = upload(B.d_slots, B.slots.data(), sizeof(PairSlot) * B.slots.size())) ||
         (rc = upload(B.d_segs, B.segs.data(), sizeof(PairSeg) * B.segs.size())) ||
         (rc = upload(B.d_targets, B.targets.data(), sizeof(PairTarget) * B.targets.size())) ||
         (rc = upload(B.d_groups, B.groups.data(), sizeof(PairGroup) * B.groups.size())) ||
-        (B.partial && (rc = upload(B.d_parts, parts.data(), sizeof(SphereParts) * parts.size()))) ||
+        (!parts.empty() && (rc = upload(B.d_parts, parts.data(), sizeof(SphereParts) * parts.size()))) ||
         (rc = upload(B.d_order, B.order.data(), 4 * B.order.size())) ||
         (rc = upload(B.d_close, B.close.data(), sizeof(Task) * B.close.size())))
         return rc;
-    B.plan_nrhs = nrhs;
     return IFS_OK;
+}
+
+// Right-hand sides run together.
+int pair_group(const ifs_ctx *c, const PairBatch &B, int nrhs) {
+    const size_t budget = pair_budget(c), tab = B.ws.d + B.ws.ax, one = 8 * (size_t)(B.n_y + B.n_z + 2 * B.n_w);
+    const size_t g = budget > tab ? (budget - tab) / std::max<size_t>(one, 1) : 1;
+    return (int)std::min<size_t>((size_t)nrhs, std::max<size_t>(g, 1));
 }
 
 }  // namespace
@@ -313,19 +326,18 @@ int pair_finalize(ifs_ctx *c, PairBatch &B, std::vector<Task> &tasks, const char
             return rc;
         c->ws_cached += need;
     }
-    return pair_plan(c, B, 1);
+    return pair_plan(c, B);
 }
 
-int pair_prepare(ifs_ctx *c, PairBatch &B, int nrhs) {
-    if (B.plan_nrhs == nrhs) return IFS_OK;
-    if (hipStreamSynchronize(c->stream) != hipSuccess) return IFS_E_HIP;
-    return pair_plan(c, B, nrhs);
+bool pair_parts(const ifs_ctx *c, const PairBatch &B, int nrhs) {
+    return B.d_parts.p && pair_group(c, B, nrhs) == nrhs;
 }
 
 int pair_run(ifs_ctx *c, PairBatch &B, const double2 *src_pool, double2 *dst_pool, int nrhs, int64_t src_stride,
              int64_t dst_stride) {
-    int rc = pair_prepare(c, B, nrhs);
-    if (rc || (rc = ws_reserve(c, B.ws))) return rc;
+    const int group = pair_group(c, B, nrhs);
+    const bool parts = pair_parts(c, B, nrhs);
+    if (int rc = ws_reserve(c, pair_need(B, group))) return rc;
     const PairTile *tiles = B.d_tiles.as<PairTile>();
     const PairSlot *slots = B.d_slots.as<PairSlot>();
     const PairSeg *segs = B.d_segs.as<PairSeg>();
@@ -345,24 +357,27 @@ int pair_run(ifs_ctx *c, PairBatch &B, const double2 *src_pool, double2 *dst_poo
                 launch_gen_axial(tk, ch.c1 - ch.c0, ch.maxK_close, ch.max_nmax, c->ws_s.as<double2>(), wax, c->stream);
             }
         }
-        {
-            Scope s(c, B.pn[1], ch.f_fwd * nrhs);
-            launch_pair_fwd(tiles, slots, ch.t0, nt, ch.max_Ls, delta, tab, src_pool, src_stride, Y, ch.n_y, nrhs,
-                            c->stream);
-        }
-        {
-            Scope s(c, B.pn[2], ch.f_ax * nrhs);
-            launch_pair_axial(tiles, slots, B.d_groups.as<PairGroup>() + ch.a0, ch.a1 - ch.a0,
-                              B.d_order.as<int32_t>(), ch.waves, ch.max_K, std::max(ch.max_Ls, ch.max_Lt), B.NL, quad,
-                              tab, wax, Y, ch.n_y, Z, ch.n_z, nrhs, c->stream);
-        }
-        {
-            Scope s(c, B.pn[3], ch.f_back * nrhs);
-            launch_pair_back(tiles, segs, ch.s0, ch.s1 - ch.s0, ch.max_Lt, delta, tab, Z, ch.n_z, W, ch.n_w, nrhs,
-                             c->stream);
-            if (!B.partial)
-                launch_pair_reduce(B.d_targets.as<PairTarget>(), segs, ch.g0, ch.g1 - ch.g0, ch.max_Lt, W,
-                                   ch.n_w, dst_pool, dst_stride, nrhs, c->stream);
+        for (int r0 = 0; r0 < nrhs; r0 += group) {
+            const int nr = std::min(group, nrhs - r0);
+            {
+                Scope s(c, B.pn[1], ch.f_fwd * nr);
+                launch_pair_fwd(tiles, slots, ch.t0, nt, ch.max_Ls, delta, tab, src_pool + r0 * src_stride, src_stride,
+                                Y, ch.n_y, nr, c->stream);
+            }
+            {
+                Scope s(c, B.pn[2], ch.f_ax * nr);
+                launch_pair_axial(tiles, slots, B.d_groups.as<PairGroup>() + ch.a0, ch.a1 - ch.a0,
+                                  B.d_order.as<int32_t>(), ch.waves, ch.max_K, std::max(ch.max_Ls, ch.max_Lt), B.NL,
+                                  quad, tab, wax, Y, ch.n_y, Z, ch.n_z, nr, c->stream);
+            }
+            {
+                Scope s(c, B.pn[3], ch.f_back * nr);
+                launch_pair_back(tiles, segs, ch.s0, ch.s1 - ch.s0, ch.max_Lt, delta, tab, Z, ch.n_z, W, ch.n_w, nr,
+                                 c->stream);
+                if (!parts)
+                    launch_pair_reduce(B.d_targets.as<PairTarget>(), segs, ch.g0, ch.g1 - ch.g0, ch.max_Lt, W, ch.n_w,
+                                       dst_pool + r0 * dst_stride, dst_stride, nr, c->stream);
+            }
         }
     }
     if (hipPeekAtLastError() != hipSuccess) return IFS_E_HIP;
@@ -371,7 +386,7 @@ int pair_run(ifs_ctx *c, PairBatch &B, const double2 *src_pool, double2 *dst_poo
 }
 
 uint64_t pair_sig(const PairBatch &B) {
-    uint64_t h = (uint64_t)B.plan_nrhs;
+    uint64_t h = 0;
     for (const DevBuf *d : {&B.d_tiles, &B.d_slots, &B.d_segs, &B.d_targets, &B.d_parts, &B.d_close, &B.d_groups, &B.d_order, &B.d_delta, &B.d_quad,
                             &B.own_tab, &B.own_ax})
         h ^= (uint64_t)(uintptr_t)d->p + 0x9e3779b97f4a7c15ull + (h << 6) + (h >> 2);

@@ -68,12 +68,11 @@ struct PairBatch {
     DevBuf own_tab, own_ax;   // tables kept across matvecs
     bool kept = false, ready = false;
     // Offsets of the spheres' sums, where the caller can take partial sums: with all tiles in
-    // one chunk no pass adds them, and parts holds those of every sphere.
+    // one chunk no pass adds them, and d_parts holds those of every sphere.
     std::vector<int64_t> rows;
     DevBuf d_parts;
-    bool partial = false;
-    int plan_nrhs = 0;        // right-hand sides the plan was cut for, 0: no valid plan
-    WsNeed ws;
+    int64_t n_y = 0, n_z = 0, n_w = 0, n_s = 0;  // largest chunk, per right-hand side (n_s: for all)
+    WsNeed ws;                // tables that are not kept
     int NL = 0;               // orders of the shared matrices
     std::vector<Task> tasks;  // the translations, sorted by target
     double cost_flops = 0.0, cost_bytes = 0.0;
@@ -83,10 +82,10 @@ struct PairBatch {
 
 // Whether the pair kernels take these translations (outgoing -> regular, orders <= kPairMaxL).
 bool pair_takes(const std::vector<Task> &tasks);
-// Takes the tasks over and plans them for one right-hand side.
+// Takes the tasks over and plans them, for any number of right-hand sides.
 int pair_finalize(ifs_ctx *c, PairBatch &B, std::vector<Task> &tasks, const char *name);
-// Plans again where the number of right-hand sides changed.
-int pair_prepare(ifs_ctx *c, PairBatch &B, int nrhs);
+// Whether a product leaves partial sums in ws_s to its caller (d_parts) and adds nothing to dst_pool.
+bool pair_parts(const ifs_ctx *c, const PairBatch &B, int nrhs);
 int pair_run(ifs_ctx *c, PairBatch &B, const double2 *src_pool, double2 *dst_pool, int nrhs, int64_t src_stride,
              int64_t dst_stride);
 uint64_t pair_sig(const PairBatch &B);

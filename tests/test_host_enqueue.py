@@ -108,3 +108,38 @@ for c in fake.calls():
         assert not outstanding, c
 assert replaced > 10
 """)
+
+
+@pytest.mark.parametrize("kw", ["", "workspace_mb=1", "workspace_mb=1, cache_mb=-1"])
+def test_direct_products_of_any_number_of_right_hand_sides_only_enqueue(so, kw):
+    """A direct plan serves every number of right-hand sides: once the vectors of the largest
+    number have their room, products neither wait nor copy nor allocate, a caller's own capture of
+    a batched one holds, and a captured single product is replayed beside batched ones."""
+    host_runtime.run(so, f"""
+s = solver(*spheres(40, 60.0, 1, 9), {kw})
+x, b = (ctypes.create_string_buffer(16 * 5 * s.n) for _ in range(2))
+x, b = ctypes.addressof(x), ctypes.addressof(b)
+s.calculate_vector_b_batch_device(x, b, 5)
+fake.calls()
+for nrhs in (1, 3, 5, 2, 1):
+    s.calculate_vector_b_batch_device(x, b, nrhs)
+seen = fake.calls()
+assert len(launches(seen, "k_finalize")) == 5 and len(launches(seen)) == len(seen), seen
+stream = ctypes.c_void_p()
+fake.hipStreamCreate(ctypes.byref(stream))
+s.set_stream(stream.value)
+graph = ctypes.c_void_p()
+for nrhs in (1, 4):
+    assert fake.hipStreamBeginCapture(stream, 1) == 0
+    s.calculate_vector_b_batch_device(x, b, nrhs)
+    assert fake.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+for _ in range(2):
+    s.calculate_vector_b_graph_device(x, b)
+fake.calls()
+for _ in range(3):
+    s.calculate_vector_b_graph_device(x, b)
+    s.calculate_vector_b_batch_device(x, b, 3)
+seen = fake.calls()
+assert len([c for c in seen if c[0] == "graph"]) == 3
+assert not [c for c in seen if c[0] not in ("graph", "launch")], seen
+""")
