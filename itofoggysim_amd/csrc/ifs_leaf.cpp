@@ -78,12 +78,6 @@ int replan(ifs_ctx *c, Leaf &F, int nrhs) {
     return ws_reserve(c, F.g.ws);
 }
 
-int group_rhs(ifs_ctx *c, const Leaf &F, int nrhs) {
-    int g = nrhs;
-    while (g > 1 && !pw_fits(c, F.g.L, F.g.nb, g)) --g;
-    return g;
-}
-
 }  // namespace
 
 // The synthesis and analysis of a box cost about what one sphere of order 20 does one by one
@@ -143,11 +137,10 @@ int leaf_build(ifs_ctx *c, Leaf &F, const std::vector<Task> &p2m, const std::vec
 }
 
 int leaf_p2m(ifs_ctx *c, Leaf &F, const double2 *xh, double2 *C, int nrhs, int64_t ldx, int64_t ldC) {
-    const int g = group_rhs(c, F, nrhs);
+    const int g = pw_group(c, F.g, nrhs);
+    if (int rc = replan(c, F, g)) return rc;
     for (int r0 = 0; r0 < nrhs; r0 += g) {
         const int nr = std::min(g, nrhs - r0);
-        int rc = replan(c, F, nr);
-        if (rc) return rc;
         LeafArg a = leaf_arg(c, F, nr);
         double2 *rows = c->ws_s.as<double2>();
         const int ns = (int)F.up.size();
@@ -172,11 +165,10 @@ int leaf_p2m(ifs_ctx *c, Leaf &F, const double2 *xh, double2 *C, int nrhs, int64
 }
 
 int leaf_l2p(ifs_ctx *c, Leaf &F, const double2 *D, double2 *acc, int nrhs, int64_t ldD, int64_t ldacc) {
-    const int g = group_rhs(c, F, nrhs);
+    const int g = pw_group(c, F.g, nrhs);
+    if (int rc = replan(c, F, g)) return rc;
     for (int r0 = 0; r0 < nrhs; r0 += g) {
         const int nr = std::min(g, nrhs - r0);
-        int rc = replan(c, F, nr);
-        if (rc) return rc;
         LeafArg a = leaf_arg(c, F, nr);
         double2 *rows = c->ws_s.as<double2>();
         const int ns = (int)F.down.size();

@@ -85,6 +85,11 @@ bool pw_fits(ifs_ctx *c, int L, int nb, int nrhs) {
     return 4 * L + 1 <= kPwMaxN - 96 && 64.0 * (double)x_size(L) * nb * nrhs <= (double)c->ws_budget;
 }
 
+int pw_group(ifs_ctx *c, const PwLevel &P, int nrhs) {
+    while (nrhs > 1 && !pw_fits(c, P.L, P.nb, nrhs)) --nrhs;
+    return nrhs;
+}
+
 int pw_grid(ifs_ctx *c, PwLevel &P, int Q2, double tdeg, int tcap, int order) {
     const int L = P.L;
     P.Q2 = Q2;
@@ -287,17 +292,15 @@ PwArg pw_arg(ifs_ctx *c, const PwLevel &P, int nrhs) {
 }
 
 int pw_run(ifs_ctx *c, PwLevel &P, const double2 *C, double2 *D, int nrhs, int64_t stride, int prec) {
-    // right-hand sides that the workspace holds at once
-    int g = nrhs;
-    while (g > 1 && !pw_fits(c, P.L, P.nb, g)) --g;
+    const int g = pw_group(c, P, nrhs);
+    if (P.plan_nrhs != g) {
+        if (hipStreamSynchronize(c->stream) != hipSuccess) return IFS_E_HIP;
+        int rc = pw_plan(c, P, g);
+        if (rc) return rc;
+    }
+    if (int rc = ws_reserve(c, P.ws)) return rc;
     for (int r0 = 0; r0 < nrhs; r0 += g) {
         const int nr = std::min(g, nrhs - r0);
-        if (P.plan_nrhs != nr) {
-            if (hipStreamSynchronize(c->stream) != hipSuccess) return IFS_E_HIP;
-            int rc = pw_plan(c, P, nr);
-            if (rc) return rc;
-        }
-        if (int rc = ws_reserve(c, P.ws)) return rc;
         hipStream_t s = c->stream;
         const int L = P.L, nc = (int)P.canon.size();
         PwArg a = pw_arg(c, P, nr);

@@ -143,3 +143,26 @@ seen = fake.calls()
 assert len([c for c in seen if c[0] == "graph"]) == 3
 assert not [c for c in seen if c[0] not in ("graph", "launch")], seen
 """)
+
+
+def test_groups_of_right_hand_sides_share_one_plan(so):
+    """Three right-hand sides in a workspace that holds the samples of two at once: the groups of
+    two and one run on one plan, so repeated products neither wait nor copy, and a capture of one
+    holds."""
+    host_runtime.run(so, """
+s = solver(*spheres(400, 160.0, 1, 9), use_fmm=True, leaf_size=32, workspace_mb=64)
+x, b = (ctypes.create_string_buffer(16 * 3 * s.n) for _ in range(2))
+x, b = ctypes.addressof(x), ctypes.addressof(b)
+s.calculate_vector_b_batch_device(x, b, 3)
+fake.calls()
+s.calculate_vector_b_batch_device(x, b, 3)
+seen = fake.calls()
+assert len(launches(seen, "k_pw_unpack")) == 4  # leaf samples and box translations of two groups
+assert not [c for c in seen if c[0] != "launch"], [c for c in seen if c[0] != "launch"]
+stream, graph = ctypes.c_void_p(), ctypes.c_void_p()
+fake.hipStreamCreate(ctypes.byref(stream))
+s.set_stream(stream.value)
+assert fake.hipStreamBeginCapture(stream, 1) == 0
+s.calculate_vector_b_batch_device(x, b, 3)
+assert fake.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+""")
