@@ -753,7 +753,7 @@ static void remember_rows(const std::array<int, 7> &k, int st, int r) {
     g_rows[k][st] = r;
 }
 
-int class_batch_run(ifs_ctx *c, ClassBatch &B, const double2 *src_pool, double2 *dst_pool, int nrhs, int prec) {
+int class_batch_prepare(ifs_ctx *c, ClassBatch &B, int nrhs) {
     if (B.gen.empty() || nrhs <= 0) return IFS_OK;
     if (B.plan_nrhs != nrhs) {
         // the kernels of an earlier product read the lists that a new cut replaces
@@ -761,7 +761,12 @@ int class_batch_run(ifs_ctx *c, ClassBatch &B, const double2 *src_pool, double2 
         int rc = class_batch_plan(c, B, nrhs);
         if (rc) return rc;
     }
-    if (int rc = ws_reserve(c, B.ws)) return rc;
+    return ws_reserve(c, B.ws);
+}
+
+int class_batch_run(ifs_ctx *c, ClassBatch &B, const double2 *src_pool, double2 *dst_pool, int nrhs, int prec) {
+    if (B.gen.empty() || nrhs <= 0) return IFS_OK;
+    if (int rc = class_batch_prepare(c, B, nrhs)) return rc;
     const GroupDesc *dd = B.d_desc.as<GroupDesc>();
     const Task *dg = B.d_gen.as<Task>();
     const Task *dk = B.d_dkeys.as<Task>();
@@ -1198,6 +1203,16 @@ int ifs_set_precision(ifs_ctx *c, int32_t precision) {
 }  // extern "C"
 
 namespace ifs {
+// Everything a product of nrhs right-hand sides needs beyond its launches: vectors, plans cut
+// for that many, workspaces.  Afterwards it only enqueues, until a product of another number.
+static int matvec_prepare(ifs_ctx *c, int nrhs) {
+    const int64_t nc = c->ncompact;
+    int rc;
+    if ((rc = c->d_xh.alloc(16ull * nc * nrhs)) || (rc = c->d_acc.alloc(16ull * nc * nrhs))) return rc;
+    if (c->fmm) return fmm::prepare(c, c->fmm, nrhs);
+    return c->pair ? pair_prepare(c, *c->pair, nrhs) : ws_reserve(c, c->direct.ws);
+}
+
 // b = M x in the reference basis, or b_hat = S M S^-1 x_hat in the normalised
 // basis (normalised = 1), both in the flat layout.
 int matvec_impl(ifs_ctx *c, const double2 *x, double2 *b, int normalised, int nrhs, int64_t ld, int64_t ldb,
@@ -1208,7 +1223,7 @@ int matvec_impl(ifs_ctx *c, const double2 *x, double2 *b, int normalised, int nr
     const double *snm = normalised ? nullptr : c->d_snm.as<double>();
     const int64_t nc = c->ncompact;
     int rc;
-    if ((rc = c->d_xh.alloc(16ull * nc * nrhs)) || (rc = c->d_acc.alloc(16ull * nc * nrhs))) return rc;
+    if ((rc = matvec_prepare(c, nrhs))) return rc;
     {
         Scope s(c, "pack_in");
         launch_pack_in(c->ns, c->N, c->d_Leff.as<int32_t>(), c->d_off.as<int64_t>(), snm, x, c->d_xh.as<double2>(),
@@ -1267,6 +1282,9 @@ int matvec_graph(ifs_ctx *c, const double2 *x, double2 *b, int normalised, int n
         if (e.x == x && e.b == b && e.normalised == normalised && e.nrhs == nrhs && e.ld == ld && e.ldb == ldb &&
             e.prec == prec)
             g = &e;
+    // outside the capture, which waits, copies and allocations break; plans cut for another number
+    // of right-hand sides since the capture come back as they were
+    if (int rc = matvec_prepare(c, nrhs)) return rc;
     const uint64_t sig = matvec_sig(c);
     if (g && g->exec && g->sig == sig)
         return hipGraphLaunch(g->exec, c->stream) == hipSuccess ? IFS_OK : IFS_E_HIP;

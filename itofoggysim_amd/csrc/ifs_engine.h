@@ -259,6 +259,9 @@ void gauss_legendre(int Q, std::vector<double> &x, std::vector<double> &w);
 // Device Gauss-Legendre rule of Q nodes (cached per context): mu, then w.
 int gq_rule(ifs_ctx *c, int Q, const double **mu, const double **w);
 int class_batch_plan(ifs_ctx *c, ClassBatch &B, int nrhs);
+// The plan for nrhs right-hand sides (waits for the stream where it is cut anew) and its workspaces;
+// class_batch_run asks for both itself.
+int class_batch_prepare(ifs_ctx *c, ClassBatch &B, int nrhs);
 // After every class batch is finalized: decides which tables persist, then plans each.
 int class_batches_prepare(ifs_ctx *c, const std::vector<ClassBatch *> &bs);
 int class_batch_run(ifs_ctx *c, ClassBatch &B, const double2 *src_pool, double2 *dst_pool, int nrhs, int prec = 0);

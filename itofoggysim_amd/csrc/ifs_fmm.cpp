@@ -419,10 +419,28 @@ fail:
 
 void destroy(Fmm *f) { delete f; }
 
-int run(ifs_ctx *c, Fmm *f, const double2 *xh, double2 *acc, int nrhs, int64_t ld, int prec) {
+int prepare(ifs_ctx *c, Fmm *f, int nrhs) {
     int rc;
     // multipole / local pools hold nrhs copies at stride nC
     if ((rc = f->C.alloc(16ull * f->nC * nrhs)) || (rc = f->D.alloc(16ull * f->nC * nrhs))) return rc;
+    if (f->leaf.active() && (rc = leaf_prepare(c, f->leaf, nrhs))) return rc;
+    for (auto &P : f->pw)
+        if (P.active() && (rc = pw_prepare(c, P, nrhs))) return rc;
+    for (auto *v : {&f->m2m, &f->m2l, &f->l2l})
+        for (auto &B : *v)
+            if ((rc = class_batch_prepare(c, B, nrhs))) return rc;
+    for (auto &v : f->rem)
+        for (auto &B : v)
+            if ((rc = class_batch_prepare(c, B, nrhs))) return rc;
+    if (f->pair.active() && (rc = pair_prepare(c, f->pair, nrhs))) return rc;
+    for (const Batch *B : {&f->p2m, &f->l2p, &f->p2p})
+        if ((rc = ws_reserve(c, B->ws))) return rc;
+    return IFS_OK;
+}
+
+int run(ifs_ctx *c, Fmm *f, const double2 *xh, double2 *acc, int nrhs, int64_t ld, int prec) {
+    int rc;
+    if ((rc = prepare(c, f, nrhs))) return rc;
     double2 *C = f->C.as<double2>(), *D = f->D.as<double2>();
     const int64_t st = f->nC;
     launch_zero(C, f->nC * nrhs, c->stream);

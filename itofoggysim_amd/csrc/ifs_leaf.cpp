@@ -63,21 +63,6 @@ void box_matrices(ifs_ctx *c, Leaf &F, LeafArg &a, const PwLevel::Chunk &ch, siz
     }
 }
 
-// The plan for nrhs right-hand sides and its workspaces.
-int replan(ifs_ctx *c, Leaf &F, int nrhs) {
-    if (F.g.plan_nrhs != nrhs) {
-        if (hipStreamSynchronize(c->stream) != hipSuccess) return IFS_E_HIP;
-        // row coefficients of the spheres: an eighth of the workspace, at least one sphere
-        const int64_t per = row_coefs(F) * nrhs;
-        F.gcap = std::max<int64_t>(1, std::min<int64_t>((int64_t)std::max(F.up.size(), F.down.size()),
-                                                        (int64_t)(c->ws_budget / 8 / 16) / per));
-        F.g.ws.s = 16 * (size_t)(F.gcap * per);
-        int rc = pw_plan(c, F.g, nrhs);
-        if (rc) return rc;
-    }
-    return ws_reserve(c, F.g.ws);
-}
-
 }  // namespace
 
 // The synthesis and analysis of a box cost about what one sphere of order 20 does one by one
@@ -86,6 +71,21 @@ int replan(ifs_ctx *c, Leaf &F, int nrhs) {
 bool leaf_worth(ifs_ctx *c, int L, int nb, int ns) {
     // up to order 850 a quarter of a row's azimuths fits LDS (about 2 L + 250 azimuths)
     return L >= 32 && L <= 850 && 2 * ns >= 3 * nb && pw_fits(c, L, nb, 1);
+}
+
+int leaf_prepare(ifs_ctx *c, Leaf &F, int nrhs) {
+    const int g = pw_group(c, F.g, nrhs);
+    if (F.g.plan_nrhs != g) {
+        if (hipStreamSynchronize(c->stream) != hipSuccess) return IFS_E_HIP;
+        // row coefficients of the spheres: an eighth of the workspace, at least one sphere
+        const int64_t per = row_coefs(F) * g;
+        F.gcap = std::max<int64_t>(1, std::min<int64_t>((int64_t)std::max(F.up.size(), F.down.size()),
+                                                        (int64_t)(c->ws_budget / 8 / 16) / per));
+        F.g.ws.s = 16 * (size_t)(F.gcap * per);
+        int rc = pw_plan(c, F.g, g);
+        if (rc) return rc;
+    }
+    return ws_reserve(c, F.g.ws);
 }
 
 int leaf_build(ifs_ctx *c, Leaf &F, const std::vector<Task> &p2m, const std::vector<Task> &l2p, int L, int nb,
@@ -133,12 +133,12 @@ int leaf_build(ifs_ctx *c, Leaf &F, const std::vector<Task> &p2m, const std::vec
     else
         (void)hipGetLastError();
     if (hipPeekAtLastError() != hipSuccess) return IFS_E_HIP;
-    return replan(c, F, 1);
+    return leaf_prepare(c, F, 1);
 }
 
 int leaf_p2m(ifs_ctx *c, Leaf &F, const double2 *xh, double2 *C, int nrhs, int64_t ldx, int64_t ldC) {
     const int g = pw_group(c, F.g, nrhs);
-    if (int rc = replan(c, F, g)) return rc;
+    if (int rc = leaf_prepare(c, F, nrhs)) return rc;
     for (int r0 = 0; r0 < nrhs; r0 += g) {
         const int nr = std::min(g, nrhs - r0);
         LeafArg a = leaf_arg(c, F, nr);
@@ -166,7 +166,7 @@ int leaf_p2m(ifs_ctx *c, Leaf &F, const double2 *xh, double2 *C, int nrhs, int64
 
 int leaf_l2p(ifs_ctx *c, Leaf &F, const double2 *D, double2 *acc, int nrhs, int64_t ldD, int64_t ldacc) {
     const int g = pw_group(c, F.g, nrhs);
-    if (int rc = replan(c, F, g)) return rc;
+    if (int rc = leaf_prepare(c, F, nrhs)) return rc;
     for (int r0 = 0; r0 < nrhs; r0 += g) {
         const int nr = std::min(g, nrhs - r0);
         LeafArg a = leaf_arg(c, F, nr);

@@ -32,6 +32,8 @@ bool leaf_worth(ifs_ctx *c, int L, int nb, int ns);
 // p2m, l2p: the translations; off: pool offset of the first leaf box
 int leaf_build(ifs_ctx *c, Leaf &F, const std::vector<Task> &p2m, const std::vector<Task> &l2p, int L, int nb,
                int64_t off);
+// As pw_prepare.
+int leaf_prepare(ifs_ctx *c, Leaf &F, int nrhs);
 int leaf_p2m(ifs_ctx *c, Leaf &F, const double2 *xh, double2 *C, int nrhs, int64_t ldx, int64_t ldC);
 int leaf_l2p(ifs_ctx *c, Leaf &F, const double2 *D, double2 *acc, int nrhs, int64_t ldD, int64_t ldacc);
 uint64_t leaf_sig(const Leaf &F);

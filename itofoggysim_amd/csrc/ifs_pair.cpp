@@ -333,11 +333,15 @@ bool pair_parts(const ifs_ctx *c, const PairBatch &B, int nrhs) {
     return B.d_parts.p && pair_group(c, B, nrhs) == nrhs;
 }
 
+int pair_prepare(ifs_ctx *c, const PairBatch &B, int nrhs) {
+    return ws_reserve(c, pair_need(B, pair_group(c, B, nrhs)));
+}
+
 int pair_run(ifs_ctx *c, PairBatch &B, const double2 *src_pool, double2 *dst_pool, int nrhs, int64_t src_stride,
              int64_t dst_stride) {
     const int group = pair_group(c, B, nrhs);
     const bool parts = pair_parts(c, B, nrhs);
-    if (int rc = ws_reserve(c, pair_need(B, group))) return rc;
+    if (int rc = pair_prepare(c, B, nrhs)) return rc;
     const PairTile *tiles = B.d_tiles.as<PairTile>();
     const PairSlot *slots = B.d_slots.as<PairSlot>();
     const PairSeg *segs = B.d_segs.as<PairSeg>();

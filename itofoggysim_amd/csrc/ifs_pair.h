@@ -86,6 +86,8 @@ bool pair_takes(const std::vector<Task> &tasks);
 int pair_finalize(ifs_ctx *c, PairBatch &B, std::vector<Task> &tasks, const char *name);
 // Whether a product leaves partial sums in ws_s to its caller (d_parts) and adds nothing to dst_pool.
 bool pair_parts(const ifs_ctx *c, const PairBatch &B, int nrhs);
+// The workspaces of a product of nrhs right-hand sides; pair_run asks for them itself.
+int pair_prepare(ifs_ctx *c, const PairBatch &B, int nrhs);
 int pair_run(ifs_ctx *c, PairBatch &B, const double2 *src_pool, double2 *dst_pool, int nrhs, int64_t src_stride,
              int64_t dst_stride);
 uint64_t pair_sig(const PairBatch &B);

@@ -291,14 +291,19 @@ PwArg pw_arg(ifs_ctx *c, const PwLevel &P, int nrhs) {
     return a;
 }
 
-int pw_run(ifs_ctx *c, PwLevel &P, const double2 *C, double2 *D, int nrhs, int64_t stride, int prec) {
+int pw_prepare(ifs_ctx *c, PwLevel &P, int nrhs) {
     const int g = pw_group(c, P, nrhs);
     if (P.plan_nrhs != g) {
         if (hipStreamSynchronize(c->stream) != hipSuccess) return IFS_E_HIP;
         int rc = pw_plan(c, P, g);
         if (rc) return rc;
     }
-    if (int rc = ws_reserve(c, P.ws)) return rc;
+    return ws_reserve(c, P.ws);
+}
+
+int pw_run(ifs_ctx *c, PwLevel &P, const double2 *C, double2 *D, int nrhs, int64_t stride, int prec) {
+    const int g = pw_group(c, P, nrhs);
+    if (int rc = pw_prepare(c, P, nrhs)) return rc;
     for (int r0 = 0; r0 < nrhs; r0 += g) {
         const int nr = std::min(g, nrhs - r0);
         hipStream_t s = c->stream;

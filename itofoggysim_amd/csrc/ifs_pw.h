@@ -94,6 +94,9 @@ int pw_plan(ifs_ctx *c, PwLevel &P, int nrhs);  // leaves ws.s as it is
 // Right-hand sides whose samples the workspace holds at once.  A level is planned for that many;
 // the last, smaller group of a product runs on the same plan.
 int pw_group(ifs_ctx *c, const PwLevel &P, int nrhs);
+// The plan for nrhs right-hand sides (waits for the stream where it is cut anew) and its workspaces;
+// pw_run asks for both itself.
+int pw_prepare(ifs_ctx *c, PwLevel &P, int nrhs);
 int pw_run(ifs_ctx *c, PwLevel &P, const double2 *C, double2 *D, int nrhs, int64_t stride, int prec);
 bool pw_fits(ifs_ctx *c, int L, int nb, int nrhs);
 // Algorithmic flops of one product: the two GEMMs (8 Q degrees^2 each way per box), the

@@ -162,7 +162,7 @@ int hipStreamBeginCapture(void *s, int) {
 }
 int hipStreamEndCapture(void *s, void **g) {
     const int was = capturing[s];
-    capturing[s] = 0;
+    if (was == 1) capturing[s] = 0;  // a broken capture leaves the stream unusable, as the GPU's runtime does
     *g = was == 1 ? (void *)16 : nullptr;
     say(was == 1 ? "captured" : "capture broken");
     return was == 1 ? kOk : fail(kCapture);
@@ -216,6 +216,7 @@ int hipLaunchKernel(const void *f, Dim3 grid, Dim3 block, void **args, size_t sh
     const std::string k = kernels.count(f) ? kernels[f] : "?";
     const bool ok = grid.x && grid.y && grid.z && grid.y <= 65535 && grid.z <= 65535 &&
                     block.x * block.y * block.z <= 1024 && shm <= 65536;
+    if (capturing[stream] == 2) return fail(kCapture);
     say((ok ? "launch " : "refused ") + k + " " + name_of(stream) + " " + std::to_string(shm));
     for (auto &w : watched) {
         if (k.find(w.kernel) == std::string::npos) continue;

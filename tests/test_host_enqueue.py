@@ -166,3 +166,33 @@ assert fake.hipStreamBeginCapture(stream, 1) == 0
 s.calculate_vector_b_batch_device(x, b, 3)
 assert fake.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
 """)
+
+
+def test_graph_products_between_batched_ones_of_a_tree(so):
+    """An MLFMM context cuts its lists anew when the number of right-hand sides changes: not inside
+    the capture of a graph product, where waiting and copying break the capture, and a graph whose
+    lists are the ones it was captured with is replayed."""
+    host_runtime.run(so, """
+for kw in ({}, dict(workspace_mb=4)):
+    s = solver(*spheres(400, 160.0, 1, 9), use_fmm=True, leaf_size=32, **kw)
+    x, b = (ctypes.create_string_buffer(16 * 3 * s.n) for _ in range(2))
+    x, b = ctypes.addressof(x), ctypes.addressof(b)
+    s.calculate_vector_b_batch_device(x, b, 3)
+    fake.calls()
+    for _ in range(2):
+        for _ in range(3):
+            s.calculate_vector_b_graph_device(x, b)
+        s.calculate_vector_b_batch_device(x, b, 3)
+    s.calculate_vector_b_graph_device(x, b)
+    seen = fake.calls()
+    inside = False
+    for c in seen:
+        if c[0] == "capture":
+            inside = True
+        elif c[0] == "captured":
+            inside = False
+        assert not inside or c[0] in ("capture", "launch"), c
+    assert len([c for c in seen if c[0] == "captured"]) == 1, seen
+    assert len([c for c in seen if c[0] == "graph"]) == 6
+    s.close()
+""")
