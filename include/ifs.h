@@ -77,7 +77,9 @@ typedef struct {
  *   IFS_PREC_FP64   FP64 throughout;
  *   IFS_PREC_MIXED  the MLFMM's dense box products (M2M, L2L, the class products of M2L) run
  *                   as FP32 matrix-core products with FP32 accumulation on the FP64 tables, and
- *                   the plane-wave M2L reads its tables in FP32 (samples and sums FP64);
+ *                   the plane-wave M2L reads its tables in FP32 (samples and sums FP64; kept
+ *                   tables get their FP32 copy with the first mixed product, and stay FP64 where
+ *                   cache_mb has no room for it or that product is being captured);
  *                   sphere-level translations, T-apply, vectors and solver state stay FP64. */
 #define IFS_PREC_FP64 0
 #define IFS_PREC_MIXED 1

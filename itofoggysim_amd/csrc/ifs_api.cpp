@@ -1205,11 +1205,11 @@ int ifs_set_precision(ifs_ctx *c, int32_t precision) {
 namespace ifs {
 // Everything a product of nrhs right-hand sides needs beyond its launches: vectors, plans cut
 // for that many, workspaces.  Afterwards it only enqueues, until a product of another number.
-static int matvec_prepare(ifs_ctx *c, int nrhs) {
+static int matvec_prepare(ifs_ctx *c, int nrhs, int prec) {
     const int64_t nc = c->ncompact;
     int rc;
     if ((rc = c->d_xh.alloc(16ull * nc * nrhs)) || (rc = c->d_acc.alloc(16ull * nc * nrhs))) return rc;
-    if (c->fmm) return fmm::prepare(c, c->fmm, nrhs);
+    if (c->fmm) return fmm::prepare(c, c->fmm, nrhs, prec);
     return c->pair ? pair_prepare(c, *c->pair, nrhs) : ws_reserve(c, c->direct.ws);
 }
 
@@ -1223,7 +1223,7 @@ int matvec_impl(ifs_ctx *c, const double2 *x, double2 *b, int normalised, int nr
     const double *snm = normalised ? nullptr : c->d_snm.as<double>();
     const int64_t nc = c->ncompact;
     int rc;
-    if ((rc = matvec_prepare(c, nrhs))) return rc;
+    if ((rc = matvec_prepare(c, nrhs, prec))) return rc;
     {
         Scope s(c, "pack_in");
         launch_pack_in(c->ns, c->N, c->d_Leff.as<int32_t>(), c->d_off.as<int64_t>(), snm, x, c->d_xh.as<double2>(),
@@ -1284,7 +1284,7 @@ int matvec_graph(ifs_ctx *c, const double2 *x, double2 *b, int normalised, int n
             g = &e;
     // outside the capture, which waits, copies and allocations break; plans cut for another number
     // of right-hand sides since the capture come back as they were
-    if (int rc = matvec_prepare(c, nrhs)) return rc;
+    if (int rc = matvec_prepare(c, nrhs, prec)) return rc;
     const uint64_t sig = matvec_sig(c);
     if (g && g->exec && g->sig == sig)
         return hipGraphLaunch(g->exec, c->stream) == hipSuccess ? IFS_OK : IFS_E_HIP;

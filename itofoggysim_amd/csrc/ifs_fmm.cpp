@@ -419,13 +419,13 @@ fail:
 
 void destroy(Fmm *f) { delete f; }
 
-int prepare(ifs_ctx *c, Fmm *f, int nrhs) {
+int prepare(ifs_ctx *c, Fmm *f, int nrhs, int prec) {
     int rc;
     // multipole / local pools hold nrhs copies at stride nC
     if ((rc = f->C.alloc(16ull * f->nC * nrhs)) || (rc = f->D.alloc(16ull * f->nC * nrhs))) return rc;
     if (f->leaf.active() && (rc = leaf_prepare(c, f->leaf, nrhs))) return rc;
     for (auto &P : f->pw)
-        if (P.active() && (rc = pw_prepare(c, P, nrhs))) return rc;
+        if (P.active() && (rc = pw_prepare(c, P, nrhs, prec))) return rc;
     for (auto *v : {&f->m2m, &f->m2l, &f->l2l})
         for (auto &B : *v)
             if ((rc = class_batch_prepare(c, B, nrhs))) return rc;
@@ -440,7 +440,7 @@ int prepare(ifs_ctx *c, Fmm *f, int nrhs) {
 
 int run(ifs_ctx *c, Fmm *f, const double2 *xh, double2 *acc, int nrhs, int64_t ld, int prec) {
     int rc;
-    if ((rc = prepare(c, f, nrhs))) return rc;
+    if ((rc = prepare(c, f, nrhs, prec))) return rc;
     double2 *C = f->C.as<double2>(), *D = f->D.as<double2>();
     const int64_t st = f->nC;
     launch_zero(C, f->nC * nrhs, c->stream);

@@ -17,7 +17,7 @@ struct Fmm;
 int build(ifs_ctx *c, Fmm **out);
 void destroy(Fmm *f);
 // Pools, plans and workspaces of a product of nrhs right-hand sides.
-int prepare(ifs_ctx *c, Fmm *f, int nrhs);
+int prepare(ifs_ctx *c, Fmm *f, int nrhs, int prec);
 // acc += (far field via P2M, M2M, M2L, L2L, L2P) + (near field P2P) of xh
 // (libmlfmm/src/lib/lib_ml_fmm.f90:231-262).
 // prec: precision of the class products (see launch_class).

@@ -205,11 +205,10 @@ int pw_build(ifs_ctx *c, PwLevel &P, int isg) {
         return IFS_E_HIP;
     launch_pw_hankel(nc, 2 * L, dt, (const int32_t *)(dt + nc), P.d_hank.as<double2>(), c->stream);
     const size_t ub = 8 * (size_t)pw_ucnt(L + 1, L) * 2 * P.Q2, tb = 16 * (size_t)nc * P.SN;
-    P.kept = ub + tb + tb / 2 + c->ws_cached <= c->cache_budget;
+    P.kept = ub + tb + c->ws_cached <= c->cache_budget;
     if (P.kept) {
-        if (P.own_U.alloc(ub) || P.own_T.alloc(tb) || P.own_T32.alloc(tb / 2)) {
-            (void)hipGetLastError();
-            for (DevBuf *d : {&P.own_U, &P.own_T, &P.own_T32})
+        if (P.own_U.alloc(ub) || P.own_T.alloc(tb)) {
+            for (DevBuf *d : {&P.own_U, &P.own_T})
                 if (d->p) {
                     (void)hipFree(d->p);
                     d->p = nullptr;
@@ -217,11 +216,11 @@ int pw_build(ifs_ctx *c, PwLevel &P, int isg) {
                 }
             P.kept = false;
         } else {
-            c->ws_cached += ub + tb + tb / 2;
+            c->ws_cached += ub + tb;
         }
     }
     if (hipPeekAtLastError() != hipSuccess) return IFS_E_HIP;
-    return pw_plan(c, P, 1);
+    return pw_prepare(c, P, 1, c->prm.precision);
 }
 
 int pw_plan(ifs_ctx *c, PwLevel &P, int nrhs) {
@@ -291,7 +290,16 @@ PwArg pw_arg(ifs_ctx *c, const PwLevel &P, int nrhs) {
     return a;
 }
 
-int pw_prepare(ifs_ctx *c, PwLevel &P, int nrhs) {
+int pw_prepare(ifs_ctx *c, PwLevel &P, int nrhs, int prec) {
+    if (prec == 1 && P.kept && !P.own_T32.p && !P.no_t32) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        (void)hipStreamIsCapturing(c->stream, &cap);
+        if (cap == hipStreamCaptureStatusNone) {
+            const size_t b = 8 * P.canon.size() * (size_t)P.SN;
+            P.no_t32 = b + c->ws_cached > c->cache_budget || P.own_T32.alloc(b) != IFS_OK;
+            if (!P.no_t32) c->ws_cached += b;
+        }
+    }
     const int g = pw_group(c, P, nrhs);
     if (P.plan_nrhs != g) {
         if (hipStreamSynchronize(c->stream) != hipSuccess) return IFS_E_HIP;
@@ -303,7 +311,7 @@ int pw_prepare(ifs_ctx *c, PwLevel &P, int nrhs) {
 
 int pw_run(ifs_ctx *c, PwLevel &P, const double2 *C, double2 *D, int nrhs, int64_t stride, int prec) {
     const int g = pw_group(c, P, nrhs);
-    if (int rc = pw_prepare(c, P, nrhs)) return rc;
+    if (int rc = pw_prepare(c, P, nrhs, prec)) return rc;
     for (int r0 = 0; r0 < nrhs; r0 += g) {
         const int nr = std::min(g, nrhs - r0);
         hipStream_t s = c->stream;
@@ -327,11 +335,12 @@ int pw_run(ifs_ctx *c, PwLevel &P, const double2 *C, double2 *D, int nrhs, int64
             a.tpre = P.d_gpre.as<int64_t>();
             a.tsn = P.SN;
             a.ustr = 2 * P.Q2;
-            if (!P.ready || !P.t_ready[prec & 1]) {
+            const int t = T32 ? 1 : 0;
+            if (!P.ready || !P.t_ready[t]) {
                 a.a0 = 0;
                 a.a1 = P.Q2;
-                tables(0, P.Q2, *std::max_element(P.N.begin(), P.N.end()), !P.ready, !P.t_ready[prec & 1]);
-                P.ready = P.t_ready[prec & 1] = true;
+                tables(0, P.Q2, *std::max_element(P.N.begin(), P.N.end()), !P.ready, !P.t_ready[t]);
+                P.ready = P.t_ready[t] = true;
             }
         }
         {

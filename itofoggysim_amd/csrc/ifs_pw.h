@@ -59,6 +59,7 @@ struct PwLevel {
     DevBuf own_U, own_T, own_T32;  // T in FP64, and in FP32 for mixed products
     bool kept = false, ready = false;
     bool t_ready[2] = {false, false};
+    bool no_t32 = false;      // the budget or the device has no room for the FP32 copy: mixed products read T
     int64_t SN = 0;           // azimuths of all positions
     struct Chunk {
         int j0, R2;           // nodes [j0, j0 + R2) and their mirrors
@@ -94,9 +95,9 @@ int pw_plan(ifs_ctx *c, PwLevel &P, int nrhs);  // leaves ws.s as it is
 // Right-hand sides whose samples the workspace holds at once.  A level is planned for that many;
 // the last, smaller group of a product runs on the same plan.
 int pw_group(ifs_ctx *c, const PwLevel &P, int nrhs);
-// The plan for nrhs right-hand sides (waits for the stream where it is cut anew) and its workspaces;
-// pw_run asks for both itself.
-int pw_prepare(ifs_ctx *c, PwLevel &P, int nrhs);
+// The plan for nrhs right-hand sides (waits for the stream where it is cut anew), its workspaces and,
+// for the first mixed product, the FP32 tables' room; pw_run asks for them itself.
+int pw_prepare(ifs_ctx *c, PwLevel &P, int nrhs, int prec);
 int pw_run(ifs_ctx *c, PwLevel &P, const double2 *C, double2 *D, int nrhs, int64_t stride, int prec);
 bool pw_fits(ifs_ctx *c, int L, int nb, int nrhs);
 // Algorithmic flops of one product: the two GEMMs (8 Q degrees^2 each way per box), the

@@ -196,3 +196,63 @@ for kw in ({}, dict(workspace_mb=4)):
     assert len([c for c in seen if c[0] == "graph"]) == 6
     s.close()
 """)
+
+
+def test_tables_in_fp32_only_for_contexts_that_run_mixed(so):
+    """FP64 contexts hold no FP32 copy of the plane-wave tables; the first mixed product brings one,
+    once, where the cache budget has room, and a captured one that comes first runs on the FP64 tables."""
+    host_runtime.run(so, """
+make = lambda **kw: solver(*spheres(400, 160.0, 1, 9), use_fmm=True, leaf_size=32, **kw)
+x, b = (ctypes.create_string_buffer(16 << 20) for _ in range(2))
+x, b = ctypes.addressof(x), ctypes.addressof(b)
+def held(s):
+    for _ in range(2):
+        s.calculate_vector_b_device(x, b)
+    return fake.fake_live_bytes()
+s = make()
+fp64 = held(s)
+s.set_precision("mixed")
+late = held(s) - fp64
+s.calculate_vector_b_device(x, b)
+fake.calls()
+s.calculate_vector_b_device(x, b)
+seen = fake.calls()
+assert len(launches(seen)) == len(seen) and not launches(seen, "k_pw_ttable"), seen
+s.close()
+s = make(precision="mixed")
+assert held(s) - fp64 == late > 0
+s.close()
+s = make()
+stream, graph = ctypes.c_void_p(), ctypes.c_void_p()
+fake.hipStreamCreate(ctypes.byref(stream))
+s.set_stream(stream.value)
+s.set_class_tiles(64, 64, False)
+s.calculate_vector_b_device(x, b)
+s.set_precision("mixed")
+fake.calls()
+assert fake.hipStreamBeginCapture(stream, 1) == 0
+s.calculate_vector_b_device(x, b)
+assert fake.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+assert launches(fake.calls(), "k_pw_m2lI15HIP_vector_typeIdLj2EE")
+s.close()
+# the smallest budget that holds every table of FP64 products: they stay when mixed ones follow
+def warm(s):
+    held(s)
+    fake.calls()
+    s.calculate_vector_b_device(x, b)
+    return len(launches(fake.calls()))
+s = make()
+all_kept = warm(s)
+mb = 1
+while True:
+    s = make(cache_mb=mb)
+    if warm(s) == all_kept:
+        break
+    mb += 1
+    s.close()
+assert mb < fp64 >> 20
+s.set_precision("mixed")
+assert warm(s) == all_kept
+s.set_precision("fp64")
+assert warm(s) == all_kept
+""")
