@@ -28,7 +28,7 @@ struct Leaf {
 };
 
 // Whether the leaf level's spheres go this way (rule and figures at the definition).
-bool leaf_worth(ifs_ctx *c, int L, int nb, int ns);
+bool leaf_worth(ifs_ctx *c, const std::vector<Task> &p2m, const std::vector<Task> &l2p, int L, int nb, int ns);
 // p2m, l2p: the translations; off: pool offset of the first leaf box
 int leaf_build(ifs_ctx *c, Leaf &F, const std::vector<Task> &p2m, const std::vector<Task> &l2p, int L, int nb,
                int64_t off);
@@ -37,6 +37,11 @@ int leaf_prepare(ifs_ctx *c, Leaf &F, int nrhs);
 int leaf_p2m(ifs_ctx *c, Leaf &F, const double2 *xh, double2 *C, int nrhs, int64_t ldx, int64_t ldC);
 int leaf_l2p(ifs_ctx *c, Leaf &F, const double2 *D, double2 *acc, int nrhs, int64_t ldD, int64_t ldacc);
 uint64_t leaf_sig(const Leaf &F);
+
+// Dynamic LDS of a block: the row sums of two spheres (P2M); a quarter of a row's azimuths in four
+// classes and both helicities, and partial sums (L2P).
+inline size_t leaf_p2m_lds(int Nmax) { return 16 * 4 * (size_t)(2 * Nmax + 1); }
+inline size_t leaf_l2p_lds(int maxN) { return 16 * (8 * (size_t)(maxN / 4) + 128); }
 
 // -- kernels --------------------------------------------------------------------
 struct LeafArg {

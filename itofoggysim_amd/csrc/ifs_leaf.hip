@@ -381,13 +381,13 @@ void launch_leaf_p2m(const LeafArg &a, const LeafSphere *sph, const int32_t *fir
                            xh, ldx, g);
     const int tiles = (maxN / 4 + 63) / 64;
     hipLaunchKernelGGL(k_leaf_p2m, dim3(a.nb, 2 * a.p.R2, tiles * nrhs), dim3(64),
-                       sizeof(double2) * 4 * (size_t)(2 * a.Nmax + 1), s, a, sph, first, s0, s0 + ns, g, accumulate);
+                       leaf_p2m_lds(a.Nmax), s, a, sph, first, s0, s0 + ns, g, accumulate);
 }
 void launch_leaf_l2p(const LeafArg &a, const LeafSphere *sph, int s0, int ns, int nrhs, int maxN, double2 *g,
                      hipStream_t s) {
     if (ns <= 0) return;
     const int n4 = maxN / 4;
-    hipLaunchKernelGGL(k_leaf_l2p, dim3(ns * nrhs, 2 * a.p.R2), dim3(128), sizeof(double2) * (8 * (size_t)n4 + 128), s,
+    hipLaunchKernelGGL(k_leaf_l2p, dim3(ns * nrhs, 2 * a.p.R2), dim3(128), leaf_l2p_lds(maxN), s,
                        a, sph, s0, n4, g);
 }
 void launch_leaf_sum(const LeafArg &a, const LeafSphere *sph, int s0, int ns, int nrhs, const double2 *g, double2 *acc,

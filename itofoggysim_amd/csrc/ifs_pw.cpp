@@ -90,6 +90,18 @@ int pw_group(ifs_ctx *c, const PwLevel &P, int nrhs) {
     return nrhs;
 }
 
+namespace {
+// Azimuths of a row at polar angle asin(s) whose transform keeps the orders up to mF.
+int azimuths(int mF, double s, double tdeg, int tcap, int order) {
+    const int N = fft_length(mF + m_reach(order + 0.5, s, order) + m_reach(tdeg, s, tcap) + 1);
+    return N < 2 * mF + 1 ? fft_length(2 * mF + 1) : N;  // the transform reads every order up to mF
+}
+}  // namespace
+
+int pw_max_azimuths(int L, double tdeg, int tcap, int order) {
+    return azimuths(m_reach(L + 0.5, 1.0, L), 1.0, tdeg, tcap, order);
+}
+
 int pw_grid(ifs_ctx *c, PwLevel &P, int Q2, double tdeg, int tcap, int order) {
     const int L = P.L;
     P.Q2 = Q2;
@@ -107,9 +119,7 @@ int pw_grid(ifs_ctx *c, PwLevel &P, int Q2, double tdeg, int tcap, int order) {
         mu[P.Q2 + j] = w[j];
         const double s = std::sqrt((1.0 - mu[j]) * (1.0 + mu[j]));
         P.mF[j] = m_reach(L + 0.5, s, L);
-        P.N[j] = fft_length(P.mF[j] + m_reach(order + 0.5, s, order) + m_reach(tdeg, s, tcap) + 1);
-        // the transform reads every order up to mF
-        if (P.N[j] < 2 * P.mF[j] + 1) P.N[j] = fft_length(2 * P.mF[j] + 1);
+        P.N[j] = azimuths(P.mF[j], s, tdeg, tcap, order);
         auto it = lens.find(P.N[j]);
         if (it == lens.end()) {
             it = lens.emplace(P.N[j], (int)P.fft.size()).first;

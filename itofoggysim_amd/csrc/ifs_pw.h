@@ -89,6 +89,8 @@ bool pw_worth(int L, int nb, int64_t cols);
 // The grid of a level: 2 Q2 nodes, azimuths for fields of order L and `order` under factors
 // whose azimuthal orders fall like J_m(tdeg sin(theta)), at most tcap.
 int pw_grid(ifs_ctx *c, PwLevel &P, int Q2, double tdeg, int tcap, int order);
+// The longest azimuthal transform of such a grid (that of a row at the equator).
+int pw_max_azimuths(int L, double tdeg, int tcap, int order);
 // parents: for every parent box its children and sources; called once per level.
 int pw_build(ifs_ctx *c, PwLevel &P, int isg);
 int pw_plan(ifs_ctx *c, PwLevel &P, int nrhs);  // leaves ws.s as it is

@@ -60,3 +60,40 @@ def test_leaf_samples_vs_translations(name):
         eb = np.linalg.norm(both[r] - b[r]) / den
         print(name, f"vs translations {e:.2e}, batched vs single {eb:.2e}, sample launches", ran["l2p_samples"][1])
         assert e < 1e-11 and eb < 1e-13
+
+
+def test_leaf_samples_of_larger_spheres():
+    """Orders 31, 32 and 40 among small spheres: up to 31 one pass of a block covers an order's sums
+    over the azimuths, beyond it two do; against all pairs.  The large spheres stand alone near the
+    middle of their boxes: one that reaches beyond its box reads back degrees at which |h1| has grown
+    to 1e12, where the one-by-one translations differ from themselves by 5e-9 to 4e-7 (kept against
+    regenerated tables).  Inside, no sphere reaches beyond degree 85 of the box's 139, so the
+    truncation vanishes and the bound of the translations holds for the direct product too."""
+    edge, rng = 110.0, np.random.default_rng(41)
+    pos, lmax = [], []
+    for b in range(64):
+        mid = (np.array([b // 16, b // 4 % 4, b % 4]) + 0.5) * edge
+        big = {0: 31, 22: 32, 63: 40}.get(b)
+        for k in range(1 if big else 2):  # two small spheres on different sides of the middle
+            off = rng.uniform(-5.0, 5.0, 3) if big else (2 * k - 1) * rng.uniform(10.0, 35.0, 3)
+            pos.append(mid + off)
+            lmax.append(big or rng.integers(1, 10))
+    pos += [np.zeros(3), np.full(3, 4 * edge)]  # corners of the tree
+    pos, lmax = np.array(pos), np.array(lmax + [1, 1], np.int32)
+    n = len(pos)
+    args = (pos, 0.8 * lmax, 1.4 + 0.01j, 1.0)
+    f = MultiSphereSolver(*args, lmax=lmax, use_fmm=True, leaf_size=32)
+    d = MultiSphereSolver(*args, lmax=lmax)
+    S, mask = snm_flat(f.n_global, lmax)
+    x = (rng.standard_normal(f.n) + 1j * rng.standard_normal(f.n)) * mask
+    f.profile(True)
+    got, ref = f.calculate_vector_b(x / S) * S, d.calculate_vector_b(x / S) * S
+    ran = f.profile_read()
+    f.close(), d.close()
+    assert "l2p_samples" in ran
+    got, ref, x = (v.reshape(n, -1) for v in (got, ref, x))
+    for j in np.concatenate([np.flatnonzero(lmax > 30), [1, 50]]):
+        e = np.linalg.norm(got[j] - ref[j]) / np.linalg.norm(ref[j] - x[j])
+        print(f"order {lmax[j]}: {e:.2e}")
+        assert e < 1e-11
+    assert np.linalg.norm(got - ref) / np.linalg.norm(ref - x) < 1e-11

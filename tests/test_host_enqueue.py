@@ -256,3 +256,23 @@ assert warm(s) == all_kept
 s.set_precision("fp64")
 assert warm(s) == all_kept
 """)
+
+
+@pytest.mark.parametrize("big,side", [(520, 200.0), (420, 3140.0)])
+def test_samples_of_leaf_boxes_only_where_local_memory_holds_them(so, big, side):
+    """One sphere of a very high order (row sums of 64 KiB a pair of spheres), and high box and sphere
+    orders together (a quarter of a row's azimuths): no launch beyond the 64 KiB of a block."""
+    host_runtime.run(so, f"""
+import numpy as np
+pos, lmax = spheres(12, {side}, 1, 4)
+pos *= 0.3
+pos[-1] = {side}
+lmax[3] = {big}
+s = solver(pos, lmax, use_fmm=True, leaf_size=12)
+x, b = (ctypes.create_string_buffer(16 * s.n) for _ in range(2))
+s.calculate_vector_b_device(ctypes.addressof(x), ctypes.addressof(b))
+seen = fake.calls()
+assert not [c for c in seen if c[0] == "refused"], [c for c in seen if c[0] == "refused"]
+assert not launches(seen, "k_leaf")
+print(s.fmm_stats())
+""")
