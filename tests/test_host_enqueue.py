@@ -276,3 +276,22 @@ assert not [c for c in seen if c[0] == "refused"], [c for c in seen if c[0] == "
 assert not launches(seen, "k_leaf")
 print(s.fmm_stats())
 """)
+
+
+@pytest.mark.parametrize("side,d0,blocks", [(180.0, 5.2, False), (190.0, 5.4, True)])
+def test_last_degrees_by_the_thread_kernel_up_to_32(so, side, d0, blocks):
+    """What the plane waves leave of near offsets is shifted by one thread a translation up to 32 degrees
+    (offsets of two boxes: 32 and 33 in these trees) and by 64-row blocks beyond."""
+    host_runtime.run(so, f"""
+import numpy as np
+rng = np.random.default_rng(int({side}))
+pos = rng.uniform(0.0, {side}, (260, 3))
+lmax = rng.integers(1, 5, 260).astype(np.int32)
+s = solver(pos, lmax, use_fmm=True, leaf_size=32, fmm_d0={d0})
+x, b = (ctypes.create_string_buffer(16 * s.n) for _ in range(2))
+fake.calls()
+s.calculate_vector_b_device(ctypes.addressof(x), ctypes.addressof(b))
+seen = fake.calls()
+assert launches(seen, "k_class_axial_remI") and launches(seen, "k_pw_m2l")
+assert bool(launches(seen, "k_class_axialI")) == {blocks}, [c[1] for c in launches(seen, "k_class")]
+""")
