@@ -199,7 +199,7 @@ int build(ifs_ctx *c, Fmm **out) {
     f->rem.resize(lmax + 1);
     for (int l = lmin; l <= lmax; ++l) {
         const Level &V = f->lv[l];
-        const bool pw_ok = c->prm.z_selector == IFS_ZSEL_HANKEL1 && pw_fits(c, V.L, (int)V.boxes.size(), 1);
+        const bool pw_ok = c->prm.z_selector == IFS_ZSEL_HANKEL1 && pw_fits(c->ws_budget, V.L, (int)V.boxes.size(), 1);
         int64_t pw_cols = 0;
         std::map<std::array<int, 3>, std::vector<std::pair<int64_t, int64_t>>> cls;
         for (size_t q = 0; q < V.boxes.size(); ++q) {
@@ -394,7 +394,7 @@ int build(ifs_ctx *c, Fmm **out) {
         }
         if ((rc = class_batches_prepare(c, cls))) goto fail;
     }
-    if (!f->l2p.tasks.empty() && leaf_worth(c, f->p2m.tasks, f->l2p.tasks, LL.L, (int)LL.boxes.size(), ns)) {
+    if (!f->l2p.tasks.empty() && leaf_worth(c->ws_budget, leaf_reach(f->p2m.tasks, f->l2p.tasks), LL.L, (int)LL.boxes.size(), ns)) {
         batch_cost(f->p2m, c->flops_mv, c->bytes_mv);
         batch_cost(f->l2p, c->flops_mv, c->bytes_mv);
         if ((rc = leaf_build(c, f->leaf, f->p2m.tasks, f->l2p.tasks, LL.L, (int)LL.boxes.size(), LL.off))) goto fail;

@@ -23,26 +23,6 @@ void exponent(const Task &T, double v[3]) {
     v[2] = T.t * T.cth;
 }
 
-// Largest sphere order and exponent of the translations, and the degree where (2p+1) j_p of that
-// exponent vanishes.
-struct Reach {
-    int order = 0, deg = 0;
-    double t = 0.0;
-};
-Reach reach(const std::vector<Task> &p2m, const std::vector<Task> &l2p) {
-    Reach R;
-    for (auto &T : p2m) {
-        R.order = std::max(R.order, T.Ls);
-        R.t = std::max(R.t, T.t);
-    }
-    for (auto &T : l2p) {
-        R.order = std::max(R.order, T.Lt);
-        R.t = std::max(R.t, T.t);
-    }
-    R.deg = (int)std::ceil(R.t + 8.0 * std::cbrt(R.t) + 30.0);
-    return R;
-}
-
 // Coefficients of all rows of one sphere and right-hand side (complex).
 int64_t row_coefs(const Leaf &F) { return 2LL * F.g.Q2 * 2 * (2 * F.Nmax + 1); }
 
@@ -88,13 +68,23 @@ void box_matrices(ifs_ctx *c, Leaf &F, LeafArg &a, const PwLevel::Chunk &ch, siz
 // The synthesis and analysis of a box cost about what one sphere of order 20 does one by one
 // (order 410: 50 us against 55 us), so from 1.5 spheres a box on; below order 32 both are
 // launches.
-bool leaf_worth(ifs_ctx *c, const std::vector<Task> &p2m, const std::vector<Task> &l2p, int L, int nb, int ns) {
-    if (L < 32 || L > 850 || 2 * ns < 3 * nb || !pw_fits(c, L, nb, 1)) return false;
+bool leaf_worth(size_t ws_budget, const LeafReach &R, int L, int nb, int ns) {
+    if (L < 32 || L > 850 || 2 * ns < 3 * nb || !pw_fits(ws_budget, L, nb, 1)) return false;
     // what the blocks hold in LDS: sphere orders up to 511, and rows of up to 1984 azimuths (box order,
     // sphere order and the factor's degree together; 2 L + 250 where the spheres are small)
-    const Reach R = reach(p2m, l2p);
-    const int maxN = pw_max_azimuths(L, R.t, R.deg, R.order);
+    const int maxN = pw_max_azimuths(L, R.t, R.deg(), R.order);
     return leaf_p2m_lds(R.order) <= 65536 && leaf_l2p_lds(maxN) <= 65536 && maxN <= kPwMaxN;
+}
+
+int LeafReach::deg() const { return (int)std::ceil(t + 8.0 * std::cbrt(t) + 30.0); }
+
+int LeafReach::nodes(int L) const { return (L + order + deg()) / 4 + 1; }
+
+LeafReach leaf_reach(const std::vector<Task> &p2m, const std::vector<Task> &l2p) {
+    LeafReach R;
+    for (auto &T : p2m) R.add(T.Ls, T.t);
+    for (auto &T : l2p) R.add(T.Lt, T.t);
+    return R;
 }
 
 int leaf_prepare(ifs_ctx *c, Leaf &F, int nrhs) {
@@ -119,7 +109,7 @@ int leaf_build(ifs_ctx *c, Leaf &F, const std::vector<Task> &p2m, const std::vec
     P.nb = nb;
     P.off = off;
     const int64_t per_box = 2LL * L * (L + 2);
-    const Reach R = reach(p2m, l2p);
+    const LeafReach R = leaf_reach(p2m, l2p);
     F.Nmax = R.order;
     F.first.assign(nb + 1, 0);
     for (auto &T : p2m) {
@@ -136,8 +126,7 @@ int leaf_build(ifs_ctx *c, Leaf &F, const std::vector<Task> &p2m, const std::vec
     }
     std::stable_sort(F.up.begin(), F.up.end(), [](auto &a, auto &b) { return a.box < b.box; });
     std::stable_sort(F.down.begin(), F.down.end(), [](auto &a, auto &b) { return a.box < b.box; });
-    // 2 Q nodes integrate degree 4 Q - 1 >= L + N + the factor's degree
-    int rc = pw_grid(c, P, (L + F.Nmax + R.deg) / 4 + 1, R.t, R.deg, F.Nmax);
+    int rc = pw_grid(c, P, R.nodes(L), R.t, R.deg(), F.Nmax);
     if (rc) return rc;
     const int ucols = (F.Nmax + 1) * (F.Nmax + 2) / 2;
     if ((rc = upload(F.d_up, F.up.data(), sizeof(LeafSphere) * F.up.size())) ||

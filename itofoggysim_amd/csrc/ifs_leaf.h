@@ -27,8 +27,20 @@ struct Leaf {
     bool active() const { return g.nb > 0; }
 };
 
+// Largest sphere order and exponent of the translations.
+struct LeafReach {
+    int order = 0;
+    double t = 0.0;
+    void add(int N, double exponent) {
+        order = N > order ? N : order;
+        t = exponent > t ? exponent : t;
+    }
+    int deg() const;          // degree of the factor: (2p+1) j_p(t) vanishes beyond
+    int nodes(int L) const;   // Q: 2 Q nodes integrate degree 4 Q - 1 >= L + order + deg
+};
+LeafReach leaf_reach(const std::vector<Task> &p2m, const std::vector<Task> &l2p);
 // Whether the leaf level's spheres go this way (rule and figures at the definition).
-bool leaf_worth(ifs_ctx *c, const std::vector<Task> &p2m, const std::vector<Task> &l2p, int L, int nb, int ns);
+bool leaf_worth(size_t ws_budget, const LeafReach &R, int L, int nb, int ns);
 // p2m, l2p: the translations; off: pool offset of the first leaf box
 int leaf_build(ifs_ctx *c, Leaf &F, const std::vector<Task> &p2m, const std::vector<Task> &l2p, int L, int nb,
                int64_t off);

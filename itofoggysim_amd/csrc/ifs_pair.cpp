@@ -276,6 +276,45 @@ bool pair_takes(const std::vector<Task> &tasks) {
     return !tasks.empty();
 }
 
+double pair_work_cap() { return (double)kPairChunk; }
+
+void pair_size(const std::vector<Task> &of_target, double weight, PairSize &S) {
+    if (of_target.empty()) return;
+    PairBatch B;
+    B.tasks = of_target;
+    std::map<int, int64_t> quads;
+    build_tiles(B, quads);
+    for (size_t t = 0; t < B.tiles.size(); ++t) {
+        const PairTile &T = B.tiles[t];
+        S.tables += weight * 64.0 * T.tabw;
+        S.work += weight * 128.0 * (double)(rows_size(T.Ls, T.K) + rows_size(T.Lt, T.K));
+        for (int s = 0; s < 4 && !T.Q; ++s) {
+            const PairSlot &P = B.slots[4 * t + s];
+            if (P.src < 0) continue;
+            S.tables += weight * 16.0 * (double)ax_size(T.Lt, P.Ls, P.K);
+            S.sect += weight * 16.0 * (double)sect_size(P.K, T.Lt + P.Ls + 2);
+            S.lists += weight * sizeof(Task);
+        }
+    }
+    // at most eight partial sums a target
+    const double nt = (double)B.tiles.size(), L = of_target[0].Lt;
+    S.work += weight * 32.0 * L * (L + 2.0) * std::min(8.0, nt);
+    S.lists += weight * (nt * (sizeof(PairTile) + 4 * sizeof(PairSlot) + sizeof(PairGroup) / 4 + 4) +
+                         8.0 * sizeof(PairSeg) + sizeof(PairTarget) + sizeof(SphereParts));
+    for (auto &T : of_target) {
+        const double m = std::max(T.Ls, T.Lt);
+        S.flops += weight * 21.0 * m * m * m;
+        S.NL = std::max(S.NL, std::max(T.Ls, T.Lt));
+    }
+    for (auto &q : quads) S.nodes.insert(q.first);
+}
+
+double PairSize::shared() const {
+    double b = 8.0 * (double)pair_delta_off_host(NL + 1);
+    for (int q : nodes) b += 8.0 * (double)quad_size(NL, q) + 16.0 * q;
+    return b;
+}
+
 int pair_finalize(ifs_ctx *c, PairBatch &B, std::vector<Task> &tasks, const char *name) {
     static const char *p2p[4] = {"p2p_gen_tables", "p2p_rot_fwd", "p2p_axial", "p2p_rot_back"};
     if (std::string(name) == "p2p")

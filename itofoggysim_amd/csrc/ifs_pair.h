@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <set>
 #include <vector>
 
 #include "ifs_engine.h"
@@ -86,6 +87,20 @@ bool pair_takes(const std::vector<Task> &tasks);
 int pair_finalize(ifs_ctx *c, PairBatch &B, std::vector<Task> &tasks, const char *name);
 // Whether a product leaves partial sums in ws_s to its caller (d_parts) and adds nothing to dst_pool.
 bool pair_parts(const ifs_ctx *c, const PairBatch &B, int nrhs);
+// Device bytes and algorithmic flops of a plan, counted target by target without planning it
+// (admission of served requests).
+struct PairSize {
+    double tables = 0.0, work = 0.0;  // kept tables; Y, Z and partial sums of one right-hand side
+    double sect = 0.0, lists = 0.0;   // workspace of the close pairs' tables; tiles, slots and the rest
+    double flops = 0.0;               // 21 L^3 a pair, L the larger order
+    int NL = 0;
+    std::set<int> nodes;
+    double shared() const;            // d(pi/2) and the node sets
+};
+// Adds one target's translations `weight` times.
+void pair_size(const std::vector<Task> &of_target, double weight, PairSize &S);
+// Largest workspace of the rotated and shifted columns, whatever the budget.
+double pair_work_cap();
 // The workspaces of a product of nrhs right-hand sides; pair_run asks for them itself.
 int pair_prepare(ifs_ctx *c, const PairBatch &B, int nrhs);
 int pair_run(ifs_ctx *c, PairBatch &B, const double2 *src_pool, double2 *dst_pool, int nrhs, int64_t src_stride,

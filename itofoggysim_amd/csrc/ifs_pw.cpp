@@ -81,12 +81,12 @@ int pw_terms(double k, double edge, int o2, int L) {
 // dozen spheres) or order 32 both are launches, and the class products stay.
 bool pw_worth(int L, int nb, int64_t cols) { return L >= 32 && cols >= 16LL * nb; }
 
-bool pw_fits(ifs_ctx *c, int L, int nb, int nrhs) {
-    return 4 * L + 1 <= kPwMaxN - 96 && 64.0 * (double)x_size(L) * nb * nrhs <= (double)c->ws_budget;
+bool pw_fits(size_t ws_budget, int L, int nb, int nrhs) {
+    return 4 * L + 1 <= kPwMaxN - 96 && 64.0 * (double)x_size(L) * nb * nrhs <= (double)ws_budget;
 }
 
 int pw_group(ifs_ctx *c, const PwLevel &P, int nrhs) {
-    while (nrhs > 1 && !pw_fits(c, P.L, P.nb, nrhs)) --nrhs;
+    while (nrhs > 1 && !pw_fits(c->ws_budget, P.L, P.nb, nrhs)) --nrhs;
     return nrhs;
 }
 
@@ -100,6 +100,23 @@ int azimuths(int mF, double s, double tdeg, int tcap, int order) {
 
 int pw_max_azimuths(int L, double tdeg, int tcap, int order) {
     return azimuths(m_reach(L + 0.5, 1.0, L), 1.0, tdeg, tcap, order);
+}
+
+PwSize pw_size(int L, int nbr, int Q2, double tdeg, int tcap, int order) {
+    PwSize S;
+    for (int j = 0; j < Q2; ++j) {
+        // the j-th node of the rule of 2 Q2 nodes, to about 1 / (8 Q2)^2
+        const double s = std::sin(3.14159265358979323846 * (4.0 * j + 3.0) / (8.0 * Q2 + 2.0));
+        const int mF = m_reach(L + 0.5, s, L), N = azimuths(mF, s, tdeg, tcap, order);
+        S.samples += 2.0 * N;
+        for (int m = -mF; m <= mF; ++m) S.box_flops += 2.0 * 2.0 * 8.0 * pw_cn(m, L);
+        S.box_flops += 2.0 * 2.0 * 2.0 * 5.0 * N * std::log2((double)N);
+    }
+    S.U = 8.0 * (double)pw_ucnt(L + 1, L) * 2.0 * Q2;
+    S.T = 16.0 * S.samples;
+    S.y = 16.0 * (2.0 * (double)x_size(L) + 4.0 * (2.0 * L + 1.0) * Q2) * nbr;
+    S.z = 64.0 * S.samples * nbr;
+    return S;
 }
 
 int pw_grid(ifs_ctx *c, PwLevel &P, int Q2, double tdeg, int tcap, int order) {

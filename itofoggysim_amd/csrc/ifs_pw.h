@@ -101,7 +101,14 @@ int pw_group(ifs_ctx *c, const PwLevel &P, int nrhs);
 // for the first mixed product, the FP32 tables' room; pw_run asks for them itself.
 int pw_prepare(ifs_ctx *c, PwLevel &P, int nrhs, int prec);
 int pw_run(ifs_ctx *c, PwLevel &P, const double2 *C, double2 *D, int nrhs, int64_t stride, int prec);
-bool pw_fits(ifs_ctx *c, int L, int nb, int nrhs);
+bool pw_fits(size_t ws_budget, int L, int nb, int nrhs);
+// Device bytes of a level on such a grid (pw_grid), counted without planning it: U, T of one canonical
+// offset, and the workspaces of all rows in one chunk.
+struct PwSize {
+    double U = 0.0, T = 0.0, y = 0.0, z = 0.0;
+    double samples = 0.0, box_flops = 0.0;  // of one box: azimuths of all rows; synthesis, analysis, transforms
+};
+PwSize pw_size(int L, int nbr, int Q2, double tdeg, int tcap, int order);
 // Algorithmic flops of one product: the two GEMMs (8 Q degrees^2 each way per box), the
 // azimuthal transforms (5 N log2 N), 16 per sample and translation.
 double pw_flops(const PwLevel &P);

@@ -12,17 +12,25 @@
 // Per request: right-hand sides T p for every direction, lock-step GMRES over the
 // directions (one batched matvec per Arnoldi step), then the cross sections.
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <cmath>
 #include <condition_variable>
+#include <cstdio>
 #include <deque>
 #include <map>
-#include <cstdio>
 #include <mutex>
+#include <set>
 #include <thread>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/ifs.h"
+#include "ifs_engine.h"
+#include "ifs_leaf.h"
+#include "ifs_pair.h"
+#include "ifs_pw.h"
+#include "ifs_tree.h"
 
 namespace {
 
@@ -74,13 +82,14 @@ namespace {
 //              host with the library's own functions: scaling, Morton keys, l_max);
 //   workspace  the translation workspace (ifs_params.workspace_mb), at most a quarter
 //              of a slot's share of the budget and at most 8 GiB;
-//   tables     translation tables kept across matvecs (ifs_params.cache_mb): the
-//              direct path's tables or the MLFMM's M2L coaxial tables, when they fit
-//              the rest of the slot's share; otherwise regenerated in every matvec;
-//   fixed      per-context buffers and the quadrature workspaces.
+//   tables     translation tables kept across matvecs (ifs_params.cache_mb) of the paths
+//              that ifs_create will choose, when they fit the rest of the slot's share;
+//              otherwise regenerated in every matvec;
+//   fixed      per-context buffers, matrices shared by all pairs, and the workspaces beside
+//              the translation workspace (generators, partial sums, row coefficients).
 struct Plan {
     size_t vectors = 0, pools = 0, workspace = 0, tables = 0, fixed = 0;
-    double flops = 0.0;  // translation flops of one matvec per right-hand side (about 21 L^3 each)
+    double seconds = 0.0;  // device time of one product, per right-hand side
     size_t total() const { return vectors + pools + workspace + tables + fixed; }
 };
 
@@ -92,11 +101,247 @@ int box_L(double k, double edge, double d0, int cap) {
     return L;
 }
 
-// sum_{q=1..K} 2 (L+1-q)^2 + (L)^2 complex per coaxial table of orders (L, L), both P and Q
-double coax_table_bytes(int L) {
-    double e = (double)L * L;
-    for (int q = 1; q <= L; ++q) e += 2.0 * (L + 1.0 - q) * (L + 1.0 - q);
-    return 2.0 * 16.0 * e;
+// What the translations of a request need: tables to keep, the workspaces of all right-hand
+// sides (y, z: the translation workspace, each the largest of the stages that share it), the
+// buffers beside it, and the time of a product.
+struct Need {
+    double tables = 0.0, y = 0.0, z = 0.0, s = 0.0, gen = 0.0, fixed = 0.0, seconds = 0.0;
+    void work(double a, double b) {
+        y = std::max(y, a);
+        z = std::max(z, b);
+    }
+};
+
+// Rates of the stages in the flops counted here (per pair or class translation 21 L^3, L the larger
+// order): 22650 sphere pairs of orders 10 to 18 in 0.45 ms; 56046 sampled translations of orders 97
+// and 174 in 5.2 ms; P2M and L2P of 2500 spheres in 4 ms; class products of orders 400 to 800.
+constexpr double kPairRate = 4e12, kPwRate = 1e13, kLeafRate = 1e13, kClassRate = 4e13;
+
+void need_pairs(const ifs::PairSize &S, int nd, Need &N) {
+    const double work = std::min(S.work * nd, ifs::pair_work_cap());
+    N.tables += S.tables;
+    N.work(work, 0.0);
+    N.s = std::max(N.s, S.sect);
+    N.fixed += S.shared() + S.lists;
+    N.seconds += S.flops / kPairRate;
+}
+
+// One-by-one translations of orders Ls -> Lt, K their smaller: tables, and what they take in all.
+double one_by_one(double Ls, double Lt) {
+    const double K = std::min(Ls, Lt), Lm = std::max(Ls, Lt);
+    return 8.0 * 2.0 * (K + 1) * (Lm + 1) * (Lm + 2) / 2.0 + 16.0 * 2.0 * (2 * K + 1) * Ls * Lt +
+           16.0 * 2.0 * (2 * K + 1) * (Ls + Lt);
+}
+
+// A batch of class products: `cols` translations of degrees n0..L (n0 = 1: orders Ls -> Lt) with
+// so many coaxial and Wigner tables.
+void need_class(int Ls, int Lt, int n0, double cols, double ax, double d, int nd, Need &N) {
+    const int K = std::min(Ls, Lt);
+    const double rb = (double)ifs::rows_off(n0, K), e0 = (double)n0 * n0 - 1.0;
+    const double nax = 16.0 * (double)(n0 > 1 ? ifs::ax0_size(Lt, n0) : ifs::ax_size(Lt, Ls, K));
+    N.tables += nax * ax + 8.0 * (double)ifs::fold_size(std::max(Ls, Lt), K) * d;
+    N.work(32.0 * std::max((double)ifs::rows_size(Ls, K) - rb, (double)Lt * (Lt + 2.0) - e0) * cols * nd,
+           32.0 * ((double)ifs::rows_size(Lt, K) - rb) * cols * nd);
+    N.fixed += 400.0 * cols;  // lists
+    const double part = n0 > 1 ? 1.0 - std::pow((double)n0 / Lt, 3.0) : 1.0, Lm = std::max(Ls, Lt);
+    N.seconds += 21.0 * Lm * Lm * Lm * part * cols / kClassRate;
+}
+
+void need_tree(const Req &r, const std::vector<int> &L, size_t ws_cap, Plan &P, Need &N) {
+    using namespace ifs;
+    const int ns = (int)L.size(), nd = (int)r.alpha.size();
+    const double k = r.prm.k, d0 = r.prm.fmm_d0 > 0.0 ? r.prm.fmm_d0 : 6.0;
+    std::vector<double> scaled;
+    const tree::Scaling S = tree::scale_points(r.centres.data(), ns, scaled);
+    std::vector<int64_t> u(ns), us;
+    for (int i = 0; i < ns; ++i) u[i] = tree::universal_index(&scaled[3 * i], tree::kThresholdLevel);
+    us = u;
+    std::sort(us.begin(), us.end());
+    const int s = r.prm.leaf_size > 0 ? r.prm.leaf_size : 10;
+    const int lmin = 2, lmax = std::max(lmin, tree::level_max(us, s));
+    const bool outgoing = r.prm.z_selector != IFS_ZSEL_BESSEL_J;
+    const size_t gq_cap = (size_t)1 << 30;
+    auto generator = [&](int kind, double t, int Lt, int Ls) {  // boxes that no GPU holds are not worth the count
+        if (std::max(Lt, Ls) > 4096) return (double)gq_cap;
+        return (double)gq_plan(kind, t, Lt, Ls, std::min(Lt, Ls), gq_cap).ws_bytes;
+    };
+    std::unordered_map<int64_t, std::vector<int>> members;  // of the leaf boxes
+    double pools = 0.0;
+    int Lup = 0;
+    for (int l = lmin; l <= lmax; ++l) {
+        std::vector<int64_t> b(us);
+        for (auto &v : b) v >>= 3 * (tree::kThresholdLevel - l);
+        b.erase(std::unique(b.begin(), b.end()), b.end());
+        const int nb = (int)b.size();
+        const double edge = S.D / std::ldexp(1.0, l);
+        const int Lb = box_L(k, edge, d0, r.prm.fmm_lmax_cap);
+        pools += 2.0 * nb * 2.0 * Lb * (Lb + 2.0) * 16.0 * nd;
+        if (l > lmin) {  // M2M and L2L with the level above: eight offsets of one length and polar angle
+            const double t = k * edge * std::sqrt(0.75);
+            need_class(Lb, Lup, 1, nb, 1, 1, nd, N);
+            need_class(Lup, Lb, 1, nb, 1, 1, nd, N);
+            N.gen = std::max({N.gen, generator(1, t, Lup, Lb), generator(1, t, Lb, Lup)});
+        }
+        Lup = Lb;
+        // M2L offsets and how many boxes have each
+        std::map<std::array<int, 3>, double> off;
+        {
+            std::unordered_map<int64_t, char> have;
+            for (int64_t v : b) have[v] = 1;
+            auto coords = [l](int64_t n, int v[3]) {
+                v[0] = v[1] = v[2] = 0;
+                for (int i = l - 1; i >= 0; --i)
+                    for (int d = 0; d < 3; ++d) v[d] = (v[d] << 1) | (int)((n >> (3 * i + 2 - d)) & 1);
+            };
+            for (int64_t q : b) {
+                int vt[3], vs[3];
+                coords(q, vt);
+                for (int64_t p : tree::domain_i4(q, l, 1)) {
+                    if (!have.count(p)) continue;
+                    coords(p, vs);
+                    off[{vs[0] - vt[0], vs[1] - vt[1], vs[2] - vt[2]}] += 1.0;
+                }
+            }
+        }
+        auto o2_of = [](const std::array<int, 3> &o) { return o[0] * o[0] + o[1] * o[1] + o[2] * o[2]; };
+        auto waves = [&](int o2) { return pw_takes(pw_terms(k, edge, o2, Lb), Lb); };
+        double cols = 0.0;
+        std::set<std::array<int, 3>> canon;
+        for (auto &o : off)
+            if (waves(o2_of(o.first))) {
+                cols += o.second;
+                const int x = std::abs(o.first[0]), y = std::abs(o.first[1]);
+                canon.insert({std::max(x, y), std::min(x, y), std::abs(o.first[2])});
+            }
+        const bool pw = outgoing && pw_fits(ws_cap, Lb, nb, 1) && pw_worth(Lb, nb, (int64_t)cols);
+        if (pw) {
+            const PwSize Z = pw_size(Lb, nb * nd, Lb + 1, 2 * Lb + 0.5, 2 * Lb, Lb);
+            const double nc = (double)canon.size();
+            N.tables += Z.U + Z.T * nc * (r.prm.precision == IFS_PREC_MIXED ? 1.5 : 1.0);
+            N.work(std::max(Z.y, 0.5 * 64.0 * 4.0 * Lb * (Lb + 2.0) * nb * nd), Z.z);
+            N.fixed += 16.0 * nc * (2.0 * Lb + 1.0) + 16.0 * cols;
+            N.seconds += (Z.box_flops * nb + 16.0 * Z.samples * cols) / kPwRate;
+        }
+        // class products: whole offsets, and the last degrees of near ones, one batch a length
+        std::map<int, std::pair<double, std::set<double>>> rem;
+        std::set<int> ax;
+        std::set<double> d;
+        double whole = 0.0;
+        for (auto &o : off) {
+            const int o2 = o2_of(o.first);
+            const int terms = pw_terms(k, edge, o2, Lb);
+            const double cth = std::fabs(o.first[2] / std::sqrt((double)o2));
+            if (pw && waves(o2)) {
+                if (terms >= 2 * Lb) continue;
+                rem[o2].first += o.second;
+                rem[o2].second.insert(cth);
+            } else {
+                whole += o.second;
+                ax.insert(o2);
+                d.insert(cth);
+            }
+        }
+        for (auto &q : rem) {
+            const int lo = pw_terms(k, edge, q.first, Lb) + 1;
+            need_class(Lb, Lb, lo - Lb, q.second.first, 1, (double)q.second.second.size(), nd, N);
+            N.gen = std::max(N.gen, (double)gq_plan_rem(k * edge * std::sqrt((double)q.first), Lb, lo, gq_cap).ws_bytes);
+        }
+        if (whole > 0.0) {
+            need_class(Lb, Lb, 1, whole, (double)ax.size(), (double)d.size(), nd, N);
+            N.gen = std::max(N.gen, generator(outgoing ? IFS_ZSEL_HANKEL1 : IFS_ZSEL_BESSEL_J, k * edge * std::sqrt((double)*ax.rbegin()), Lb, Lb));
+        }
+        if (l < lmax) continue;
+        // spheres and their leaf boxes
+        LeafReach R;
+        double batch = 0.0;
+        for (int i = 0; i < ns; ++i) {
+            const int64_t q = u[i] >> (3 * (tree::kThresholdLevel - l));
+            members[q].push_back(i);
+            double c[3], t2 = 0.0;
+            tree::centre(q, l, c);
+            for (int e = 0; e < 3; ++e) {
+                const double v = r.centres[3 * i + e] - (c[e] * S.D + S.x_min[e]);
+                t2 += v * v;
+            }
+            R.add(L[i], k * std::sqrt(t2));
+            batch += 2.0 * (one_by_one(L[i], Lb) + 64.0 * Lb * (2.0 * L[i] + 1.0));
+        }
+        if (leaf_worth(ws_cap, R, Lb, nb, ns)) {
+            const PwSize Z = pw_size(Lb, nb * nd, R.nodes(Lb), R.t, R.deg(), R.order);
+            N.tables += Z.U;
+            N.work(Z.y, Z.z);
+            N.fixed += 16.0 * R.nodes(Lb) * (R.order + 1.0) * (R.order + 2.0) / 2.0 + 200.0 * ns;
+            N.s = std::max(N.s, std::min((double)ws_cap / 8.0, 64.0 * R.nodes(Lb) * (2.0 * R.order + 1.0) * ns * nd));
+            N.seconds += Z.box_flops * nb / kPwRate;
+            for (int i = 0; i < ns; ++i) N.seconds += 2.0 * (8.0 * L[i] + 150.0) * Z.samples / kLeafRate;
+        } else {
+            N.s = std::max(N.s, std::min(batch, (double)ws_cap));  // in buffers of its own
+            N.gen = std::max(N.gen, (R.order + 1.0) * (Lb + 2.0) * (Lb + R.order + R.deg()) * 4.0);
+            for (int i = 0; i < ns; ++i) N.seconds += 2.0 * 21.0 * L[i] * (double)Lb * Lb / kPairRate;
+        }
+    }
+    P.pools = (size_t)pools;
+    // near field; of many spheres every so-manieth stands for the others
+    PairSize Q;
+    double generic = 0.0;
+    const int step = std::max(1, ns / 2048);
+    bool takes = outgoing && *std::max_element(L.begin(), L.end()) <= kPairMaxL;
+    std::vector<Task> tasks;
+    for (int j = 0; j < ns; j += step) {
+        tasks.clear();
+        for (int64_t b : tree::domain_i2(u[j] >> (3 * (tree::kThresholdLevel - lmax)), lmax, 1)) {
+            auto it = members.find(b);
+            if (it == members.end()) continue;
+            for (int i : it->second) {
+                if (i == j) continue;
+                double dv[3];
+                for (int d = 0; d < 3; ++d) dv[d] = r.centres[3 * j + d] - r.centres[3 * i + d];
+                tasks.push_back(make_task(dv, k, IFS_ZSEL_HANKEL1, L[i], L[j], 0, 0));
+                generic += step * one_by_one(L[i], L[j]);
+                takes = takes && tasks.back().t > 0.0;
+            }
+        }
+        if (takes) pair_size(tasks, step, Q);
+    }
+    if (takes) {
+        need_pairs(Q, nd, N);
+    } else {
+        N.tables += generic;
+        N.s = std::max(N.s, std::min(generic, (double)ws_cap));
+        N.seconds += generic / 1e12;
+    }
+}
+
+void need_direct(const Req &r, const std::vector<int> &L, Need &N) {
+    using namespace ifs;
+    const int ns = (int)L.size(), nd = (int)r.alpha.size();
+    bool takes = r.prm.z_selector != IFS_ZSEL_BESSEL_J && *std::max_element(L.begin(), L.end()) <= kPairMaxL;
+    PairSize Q;
+    std::vector<Task> tasks;
+    // of many spheres every so-manieth stands for the others
+    const int step = std::max(1, ns / 512);
+    for (int j = 0; j < ns && takes; j += step) {
+        tasks.clear();
+        for (int i = 0; i < ns; ++i) {
+            if (i == j) continue;
+            double dv[3];
+            for (int d = 0; d < 3; ++d) dv[d] = r.centres[3 * j + d] - r.centres[3 * i + d];
+            tasks.push_back(make_task(dv, r.prm.k, IFS_ZSEL_HANKEL1, L[i], L[j], 0, 0));
+            takes = takes && tasks.back().t > 0.0;
+        }
+        pair_size(tasks, (double)step, Q);
+    }
+    if (takes) {
+        need_pairs(Q, nd, N);
+        return;
+    }
+    double t = 0.0;
+    for (int a = 0; a < ns; ++a)
+        for (int b = 0; b < ns; ++b)
+            if (a != b) t += one_by_one(L[a], L[b]);
+    N.tables += t;
+    N.work(t * nd, 0.0);
+    N.seconds += t / 1e12;
 }
 
 Plan plan_request(Req &r, size_t budget, int slots) {
@@ -107,7 +352,7 @@ Plan plan_request(Req &r, size_t budget, int slots) {
     std::vector<int> L(ns);
     for (int j = 0; j < ns; ++j) {
         int lj = r.lmax.empty() ? (int)std::ceil(k * r.radii[j] + 4.05 * std::cbrt(k * r.radii[j]) + 2.0) : r.lmax[j];
-        L[j] = N > 0 ? std::min(lj, N) : lj;
+        L[j] = std::max(1, N > 0 ? std::min(lj, N) : lj);
     }
     if (N <= 0) N = *std::max_element(L.begin(), L.end());
     const double n = 2.0 * ns * N * (N + 2);
@@ -115,52 +360,23 @@ Plan plan_request(Req &r, size_t budget, int slots) {
     P.vectors = (size_t)(16.0 * n * ((r.restart + 1) * nd + 6.0 * nd + 4.0));
     const size_t share = budget / (size_t)std::max(slots, 1);
     const size_t ws_cap = std::min<size_t>(std::max<size_t>(share / 4, (size_t)256 << 20), (size_t)8 << 30);
-    double table_need = 0.0, ws_need = 0.0;
-    if (r.prm.use_fmm) {
-        std::vector<double> scaled(3 * ns), xmd(4);
-        std::vector<int64_t> u(ns);
-        ifs_tree_scale(r.centres.data(), ns, scaled.data(), xmd.data());
-        ifs_tree_universal_index(scaled.data(), ns, 21, u.data());
-        std::sort(u.begin(), u.end());
-        const int s = r.prm.leaf_size > 0 ? r.prm.leaf_size : 10;
-        const int lmax = std::max(2, ifs_tree_level_max(u.data(), ns, s));
-        const double d0 = r.prm.fmm_d0 > 0.0 ? r.prm.fmm_d0 : 6.0;
-        double pools = 0.0;
-        for (int l = 2; l <= lmax; ++l) {
-            std::vector<int64_t> b(u.size());
-            for (int i = 0; i < ns; ++i) b[i] = u[i] >> (3 * (21 - l));
-            b.erase(std::unique(b.begin(), b.end()), b.end());
-            const int Lb = box_L(k, xmd[3] / std::ldexp(1.0, l), d0, r.prm.fmm_lmax_cap);
-            pools += 2.0 * (double)b.size() * 2.0 * Lb * (Lb + 2.0) * 16.0 * nd;
-            P.flops += (double)b.size() * 100.0 * 21.0 * Lb * Lb * (double)Lb;  // ~100 M2L per box
-            // M2L: at most 15 distinct offset lengths per level, one coaxial table each
-            table_need += 15.0 * coax_table_bytes(Lb);
-            // class columns: up to 189 M2L per box, Y/W and Z of 4 L(L+2) doubles each
-            ws_need += (double)b.size() * 189.0 * 2.0 * 4.0 * Lb * (Lb + 2.0) * 8.0 * nd;
-            // sphere <-> box quadrature tables of one chunk
-            ws_need = std::max(ws_need, (double)ns * 2.0 * 16.0 * Lb * 51.0 * 51.0);
-        }
-        P.pools = (size_t)pools;
-        double l3 = 0.0;
-        for (int j = 0; j < ns; ++j) l3 += (double)L[j] * L[j] * L[j];
-        P.flops += 27.0 * std::min(ns, 2 * s) * 21.0 * l3;  // near field: about 27 leaves of up to 2 s spheres
-        P.fixed = ((size_t)1 << 30) + ((size_t)256 << 20);  // quadrature workspaces and tables of the box levels
-    } else {
-        for (int a = 0; a < ns; ++a)
-            for (int b = 0; b < ns; ++b) {
-                if (a == b) continue;
-                double Ls = L[a], Lt = L[b], K = std::min(Ls, Lt), Lm = std::max(Ls, Lt);
-                table_need += 8.0 * 2.0 * (K + 1) * (Lm + 1) * (Lm + 2) / 2.0 + 16.0 * 2.0 * (2 * K + 1) * Ls * Lt +
-                              16.0 * 2.0 * (2 * K + 1) * (Ls + Lt);
-                P.flops += 21.0 * Lm * Lm * Lm;
-            }
-        ws_need = table_need * nd;
-        P.fixed = (size_t)64 << 20;
-    }
-    P.workspace = (size_t)std::min<double>((double)ws_cap, ws_need + (64 << 20));
+    Need D;
+    if (r.prm.use_fmm)
+        need_tree(r, L, ws_cap, P, D);
+    else
+        need_direct(r, L, D);
+    P.seconds = D.seconds;
+    P.workspace = (size_t)std::min<double>((double)ws_cap, D.y + D.z + (64 << 20));
+    // counted rather than planned: a tenth more, and the per-context buffers.  Wigner tables
+    // regenerated in a product take at most a quarter of the workspace.
+    P.fixed = (size_t)(1.1 * (D.s + D.gen + D.fixed)) + ((size_t)96 << 20);
+    const double table_need = 1.1 * D.tables;
     // tables kept only when they fit what the slot's share leaves
     const size_t used = P.vectors + P.pools + P.workspace + P.fixed;
-    if (table_need > 0.0 && used + (size_t)table_need <= share) P.tables = (size_t)table_need;
+    if (table_need > 0.0 && (double)used + table_need <= (double)share)
+        P.tables = (size_t)table_need;
+    else if (r.prm.use_fmm)
+        P.fixed += P.workspace / 4;
     r.prm.workspace_mb = (int32_t)std::max<size_t>(1, P.workspace >> 20);
     r.prm.cache_mb = P.tables > 0 ? (int32_t)((P.tables >> 20) + 1) : -1;
     if (P.tables > 0) P.tables = (size_t)r.prm.cache_mb << 20;
@@ -299,8 +515,7 @@ int ifs_server_submit(ifs_server *s, const ifs_cluster *cl, const ifs_params *pr
     {
         const Plan P = plan_request(r, s->budget, s->slots);
         r.footprint = P.total();
-        // ~20 matvecs per solve at ~10 TFLOP/s effective, per right-hand side
-        r.est_s = 20.0 * P.flops * (double)r.alpha.size() / 1e13;
+        r.est_s = 20.0 * P.seconds * (double)r.alpha.size();  // about 20 products a solve
     }
     std::lock_guard<std::mutex> lk(s->mu);
     if (s->stop) return IFS_E_ARG;

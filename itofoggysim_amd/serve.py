@@ -7,6 +7,7 @@ import numpy as np
 
 from . import _lib
 from ._lib import check, lib
+from .solver import _prec
 
 
 class Server:
@@ -35,9 +36,7 @@ class Server:
         pr.use_fmm = int(ns > 200 if use_fmm is None else bool(use_fmm))
         pr.leaf_size = int(leaf_size)
         pr.fmm_d0 = float(fmm_d0)
-        if precision not in ("fp64", "mixed"):
-            raise ValueError("precision must be 'fp64' or 'mixed'")
-        pr.precision = 0 if precision == "fp64" else 1
+        pr.precision = _prec(precision)
         d = np.asarray(directions, dtype=np.float64).reshape(-1, 2)
         al = np.ascontiguousarray(d[:, 0])
         be = np.ascontiguousarray(d[:, 1])
@@ -83,7 +82,7 @@ class Server:
 
 
 def plan_request(centres, radii, k, ndir, lmax=None, restart=30, n_global=None, use_fmm=None, leaf_size=32,
-                 fmm_d0=6.0, hbm_budget_gb=200.0, slots=4):
+                 fmm_d0=6.0, hbm_budget_gb=200.0, slots=4, z_selector=3, precision="fp64"):
     """The server's admission plan of one request, on the host (ifs_server_plan): bytes of
     vectors, MLFMM pools, workspace, kept tables, fixed buffers and their total, and the
     workspace_mb / cache_mb its context would get (cache_mb -1: no tables kept)."""
@@ -102,6 +101,8 @@ def plan_request(centres, radii, k, ndir, lmax=None, restart=30, n_global=None, 
     pr.use_fmm = int(ns > 200 if use_fmm is None else bool(use_fmm))
     pr.leaf_size = int(leaf_size)
     pr.fmm_d0 = float(fmm_d0)
+    pr.z_selector = int(z_selector)
+    pr.precision = _prec(precision)
     out = np.zeros(8)
     check(lib().ifs_server_plan(ctypes.byref(cl), ctypes.byref(pr), int(ndir), int(restart), float(hbm_budget_gb),
                                 int(slots), out.ctypes.data), "ifs_server_plan")

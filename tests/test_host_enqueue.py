@@ -274,7 +274,6 @@ s.calculate_vector_b_device(ctypes.addressof(x), ctypes.addressof(b))
 seen = fake.calls()
 assert not [c for c in seen if c[0] == "refused"], [c for c in seen if c[0] == "refused"]
 assert not launches(seen, "k_leaf")
-print(s.fmm_stats())
 """)
 
 
@@ -294,4 +293,36 @@ s.calculate_vector_b_device(ctypes.addressof(x), ctypes.addressof(b))
 seen = fake.calls()
 assert launches(seen, "k_class_axial_remI") and launches(seen, "k_pw_m2l")
 assert bool(launches(seen, "k_class_axialI")) == {blocks}, [c[1] for c in launches(seen, "k_class")]
+""")
+
+
+@pytest.mark.parametrize("gen,n,ndir,fmm,precision,budget", [
+    ("uniform", 20, 1, False, "fp64", 200.0), ("uniform", 180, 2, False, "fp64", 8.0),
+    ("uniform", 250, 1, True, "fp64", 200.0), ("uniform", 500, 8, True, "fp64", 200.0),
+    ("uniform", 2500, 1, True, "mixed", 200.0), ("lognormal", 200, 2, True, "mixed", 200.0)])
+def test_a_served_request_stays_in_its_plan_and_keeps_its_tables(so, gen, n, ndir, fmm, precision, budget):
+    """A context made with the limits that the server's plan gives it: what it allocates for products
+    of all directions is what the plan holds beside the Krylov basis, which in turn is no more than
+    twice that (and 256 MiB), and the second product generates no table.  180 spheres in a share of 2
+    GiB: the tables of all pairs are 75 MiB."""
+    host_runtime.run(so, f"""
+import numpy as np
+from itofoggysim_amd import MultiSphereSolver, config_cluster, make_cluster, plan_request
+c = make_cluster({n}, ("uniform", 0.3, 1.0), side=10.0 * ({n} / 20.0) ** (1.0 / 3.0), seed={n}) \
+    if {gen!r} == "uniform" else config_cluster(2, n={n})
+p = plan_request(c["centres"], c["radii"], c["k"], {ndir}, lmax=c["lmax"], use_fmm={fmm}, precision={precision!r},
+                 hbm_budget_gb={budget}, slots=4)
+fake.fake_set_free(250 << 30)
+s = MultiSphereSolver(c["centres"], c["radii"], 1.33, c["k"], lmax=c["lmax"], use_fmm={fmm}, leaf_size=32,
+                      precision={precision!r}, workspace_mb=p["workspace_mb"], cache_mb=p["cache_mb"])
+x = ctypes.create_string_buffer(64)
+for _ in range(2):
+    fake.calls()
+    s.calculate_vector_b_batch_device(ctypes.addressof(x), ctypes.addressof(x), {ndir})
+made = [k[1] for k in launches(fake.calls()) if any(t in k[1] for t in ("table", "k_gen", "k_gq"))]
+live = fake.fake_live_bytes()
+basis = 16.0 * s.n * 31 * {ndir}
+print({n}, {ndir}, "live", live / 2 ** 20, "MiB, plan", (p["total"] - basis) / 2 ** 20, made)
+assert not made and live <= p["total"] - basis
+assert p["total"] - p["vectors"] <= 2.0 * live + (256 << 20)
 """)
