@@ -26,6 +26,7 @@ sys.path.insert(0, ROOT)
 
 FP64_PEAK_TFLOPS = 78.6
 FP32_PEAK_TFLOPS = 157.3
+HBM_PEAK_TBS = 8.0
 METRIC = "MLFMM matvecs/s & solves/s at rel. residual 1e-6; p50/p99 solve latency"
 
 
@@ -35,6 +36,25 @@ def snm_flat(N, ns):
     s = np.array([np.exp(0.5 * (np.log(n * (n + 1) * (2 * n + 1)) + lgamma(n - m + 1) - lgamma(n + m + 1)))
                   for n in range(1, N + 1) for m in range(-n, n + 1)])
     return np.tile(np.concatenate([s, s]), ns)
+
+
+def roofline(kern, traffic, suffix):
+    """The kernel group that takes longest against what bounds it: the matrix cores (FP64; FP32 for
+    the groups named so) or, where its HBM bytes are known and take longer at their peak, HBM.
+    kern: {name: (total ms, launches, algorithmic flops)}; traffic: bytes per launch by name and suffix."""
+    dom = max(kern, key=lambda k: kern[k][0])
+    tot_ms, launches, fl = kern[dom]
+    t = traffic.get(dom + suffix)
+    per_launch = t["read"] + t["write"] if t else None
+    peak = FP32_PEAK_TFLOPS if dom.endswith("_f32") else FP64_PEAK_TFLOPS
+    tflops = fl / (tot_ms * 1e-3) / 1e12
+    tbs = per_launch * launches / (tot_ms * 1e-3) / 1e12 if t else 0.0
+    hbm = tbs / HBM_PEAK_TBS > tflops / peak
+    got, top = (tbs, HBM_PEAK_TBS) if hbm else (tflops, peak)
+    return {"bound": "hbm" if hbm else "mfma", "kernel": dom, "achieved": round(got, 3), "peak": top,
+            "unit": "TB/s" if hbm else "TFLOP/s", "frac": round(got / top, 4), "tflops": round(tflops, 3),
+            "traffic": per_launch, "traffic_unit": "bytes/launch", "launches": launches,
+            "avg_launch_ms": round(tot_ms / launches, 4), "algorithmic_flops_per_launch": fl / launches}
 
 
 def cpu_model():
@@ -393,31 +413,21 @@ def main():
     # mixed vs FP64 matvec, relative in the normalised basis
     mixed_err = float(torch.linalg.norm((be32 - be64) * snm) / torch.linalg.norm((be64 - xe) * snm))
 
+    # the scopes that report algorithmic flops; HBM bytes per launch of the largest kernels:
+    # measured offline with FETCH_SIZE / WRITE_SIZE counter runs of this same workload, calibrated
+    # on a plain copy (profiles/)
     kern = {k: v for k, v in prof.items() if v[2] > 0}
-    dom = max(kern, key=lambda k: kern[k][0])
-    tot_ms, launches, fl = kern[dom]
-    achieved = fl / (tot_ms * 1e-3) / 1e12
-    # FP64 dense products; MI355X's FP64 matrix and vector peaks are both 78.6 TFLOP/s
-    # HBM bytes per launch of the dominant kernel: measured offline with FETCH_SIZE / WRITE_SIZE
-    # counter runs of this same workload, calibrated on a plain copy (profiles/)
-    traffic, traffic_src = None, None
-    tfile = os.path.join(ROOT, "profiles", "mlfmm_2000_spheres_traffic.json")
-    if os.path.exists(tfile) and args.n == 2000 and args.config == 2:
-        tj = json.load(open(tfile))
-        t = tj["bytes_per_dispatch"].get(dom)
-        if t:
-            traffic, traffic_src = t["read"] + t["write"], "profiles/mlfmm_2000_spheres_traffic.json"
+    traffic_file = "profiles/mlfmm_2000_spheres_traffic.json"
+    traffic = {}
+    if os.path.exists(os.path.join(ROOT, traffic_file)) and args.n == 2000 and args.config == 2:
+        traffic = json.load(open(os.path.join(ROOT, traffic_file)))["bytes_per_dispatch"]
+    roof = roofline(kern, traffic, "")
+    roof["traffic_source"] = traffic_file if roof["traffic"] else None
     # the same launches counted in the per-translation unit of the reference's formulation
     # (unfolded rotations, coaxial operator [A B; B A] not decoupled): the coaxial shift
-    # performs exactly half of that count, so its reference-unit rate is twice `achieved`
-    ref_unit = 2.0 if dom == "class_axial" else None
-    roofline = {"bound": "mfma", "kernel": dom, "achieved": round(achieved, 3),
-                "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": round(achieved / FP64_PEAK_TFLOPS, 4),
-                "traffic": traffic, "traffic_unit": "bytes/launch", "traffic_source": traffic_src,
-                "launches": launches, "avg_launch_ms": round(tot_ms / launches, 4),
-                "algorithmic_flops_per_launch": fl / launches,
-                "achieved_reference_unit": round(achieved * ref_unit, 3) if ref_unit else None,
-                "matvec_algorithmic_tflops": round(flops_mv / (ms * 1e-3) / 1e12, 3)}
+    # performs exactly half of that count, so its reference-unit rate is twice its own
+    roof["achieved_reference_unit"] = round(2.0 * roof["tflops"], 3) if roof["kernel"] == "class_axial" else None
+    roof["matvec_algorithmic_tflops"] = round(flops_mv / (ms * 1e-3) / 1e12, 3)
 
     out = {
         "metric": METRIC,
@@ -436,24 +446,19 @@ def main():
             "workload": workload,
             "n_spheres": s.n_spheres, "unknowns_flat": s.n, "box_L_per_level": levels, "translations": counts,
             "matvec_algorithmic_flop": flops_mv, "build_s": round(build_s, 3)},
-        "roofline": roofline,
+        "roofline": roof,
         "kernels_ms": {k: round(v[0], 2) for k, v in prof.items()},
         "kernels_tflops": {k: round(v[2] / (v[0] * 1e-3) / 1e12, 2) for k, v in kern.items() if v[0] > 0},
         "finite": finite,
     }
     kern32 = {k: v for k, v in prof32.items() if v[2] > 0 and v[0] > 0}
-    dom32 = max(kern32, key=lambda k: kern32[k][0])
-    a32 = kern32[dom32][2] / (kern32[dom32][0] * 1e-3) / 1e12
-    peak32 = FP32_PEAK_TFLOPS if dom32.endswith("_f32") else FP64_PEAK_TFLOPS
     out["mixed"] = {
-        "roofline": {"bound": "mfma", "kernel": dom32, "achieved": round(a32, 3), "peak": peak32,
-                     "unit": "TFLOP/s", "frac": round(a32 / peak32, 4), "launches": kern32[dom32][1],
-                     "avg_launch_ms": round(kern32[dom32][0] / kern32[dom32][1], 4)},
+        "roofline": roofline(kern32, traffic, "_mixed"),
         "value": round(1000.0 / ms32, 6), "unit": "matvecs/s", "ms_per_step": round(ms32, 3),
         "speedup_vs_fp64": round(ms / ms32, 3),
         "rel_error_vs_fp64_normalised": mixed_err,
         "kernels_ms": {k: round(v[0], 2) for k, v in prof32.items()},
-        "kernels_tflops": {k: round(v[2] / (v[0] * 1e-3) / 1e12, 2) for k, v in prof32.items() if v[2] > 0 and v[0] > 0},
+        "kernels_tflops": {k: round(v[2] / (v[0] * 1e-3) / 1e12, 2) for k, v in kern32.items()},
         "note": "M2M, L2L and M2L's class products as FP32 matrix-core products (FP32 accumulation) on the FP64 "
                 "tables, plane-wave M2L tables in FP32; samples, sphere-level translations, T-apply and vectors "
                 "FP64; FP32 peak 157.3 TFLOP/s"}

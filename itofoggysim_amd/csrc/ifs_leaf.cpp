@@ -26,6 +26,20 @@ void exponent(const Task &T, double v[3]) {
 // Coefficients of all rows of one sphere and right-hand side (complex).
 int64_t row_coefs(const Leaf &F) { return 2LL * F.g.Q2 * 2 * (2 * F.Nmax + 1); }
 
+// Algorithmic flops of spheres s0 .. s0 + n - 1 and one right-hand side: on a chunk's samples
+// (8 N + 150 a sample) with their row sums (P2M), and of the sums over all rows (L2P).
+double sample_flops(const std::vector<LeafSphere> &v, int s0, int n, const PwLevel::Chunk &ch, bool rows) {
+    double f = 0.0;
+    for (int i = s0; i < s0 + n; ++i)
+        f += (8.0 * v[i].N + 150.0) * (double)ch.sn + (rows ? 16.0 * ch.R2 * v[i].N * (v[i].N + 2.0) : 0.0);
+    return f;
+}
+double sum_flops(const std::vector<LeafSphere> &v, int s0, int n, int Q2) {
+    double f = 0.0;
+    for (int i = s0; i < s0 + n; ++i) f += 16.0 * Q2 * v[i].N * (v[i].N + 2.0);
+    return f;
+}
+
 LeafArg leaf_arg(ifs_ctx *c, Leaf &F, int nrhs) {
     LeafArg a{};
     a.p = pw_arg(c, F.g, nrhs);
@@ -157,13 +171,13 @@ int leaf_p2m(ifs_ctx *c, Leaf &F, const double2 *xh, double2 *C, int nrhs, int64
             const auto &ch = F.g.chunks[i];
             box_matrices(c, F, a, ch, i);
             {
-                Scope s(c, "p2m_samples");
+                Scope s(c, "p2m_samples", sample_flops(F.up, 0, ns, ch, true) * nr);
                 for (int s0 = 0; s0 == 0 || s0 < ns; s0 += (int)F.gcap)
                     launch_leaf_p2m(a, F.d_up.as<LeafSphere>(), F.d_first.as<int32_t>(), s0,
                                     std::min<int>((int)F.gcap, ns - s0), xh + r0 * ldx, ldx, nr, ch.maxN, rows, s0 > 0,
                                     c->stream);
             }
-            Scope s(c, "p2m_box");
+            Scope s(c, "p2m_box", (ch.f_fft + ch.f_gemm) * F.g.nb * nr);
             launch_pw_fft(a.p, 1, ch.maxN, c->stream);
             launch_pw_anal(a.p, i > 0, c->stream);
         }
@@ -193,14 +207,14 @@ int leaf_l2p(ifs_ctx *c, Leaf &F, const double2 *D, double2 *acc, int nrhs, int6
                 const auto &ch = F.g.chunks[i];
                 box_matrices(c, F, a, ch, i);
                 if (!made) {
-                    Scope s(c, "l2p_box");
+                    Scope s(c, "l2p_box", (ch.f_fft + ch.f_gemm) * F.g.nb * nr);
                     launch_pw_synth(a.p, c->stream);
                     launch_pw_fft(a.p, 0, ch.maxN, c->stream);
                 }
-                Scope s(c, "l2p_samples");
+                Scope s(c, "l2p_samples", sample_flops(F.down, s0, n, ch, false) * nr);
                 launch_leaf_l2p(a, F.d_down.as<LeafSphere>(), s0, n, nr, ch.maxN, rows, c->stream);
             }
-            Scope s(c, "l2p_sum");
+            Scope s(c, "l2p_sum", sum_flops(F.down, s0, n, F.g.Q2) * nr);
             launch_leaf_sum(a, F.d_down.as<LeafSphere>(), s0, n, nr, rows, acc + r0 * ldacc, ldacc, c->stream);
         }
     }

@@ -109,8 +109,9 @@ PwSize pw_size(int L, int nbr, int Q2, double tdeg, int tcap, int order) {
         const double s = std::sin(3.14159265358979323846 * (4.0 * j + 3.0) / (8.0 * Q2 + 2.0));
         const int mF = m_reach(L + 0.5, s, L), N = azimuths(mF, s, tdeg, tcap, order);
         S.samples += 2.0 * N;
-        for (int m = -mF; m <= mF; ++m) S.box_flops += 2.0 * 2.0 * 8.0 * pw_cn(m, L);
-        S.box_flops += 2.0 * 2.0 * 2.0 * 5.0 * N * std::log2((double)N);
+        double gemm, fft;
+        pw_row_flops(L, mF, N, gemm, fft);
+        S.box_flops += 2.0 * (gemm + fft);
     }
     S.U = 8.0 * (double)pw_ucnt(L + 1, L) * 2.0 * Q2;
     S.T = 16.0 * S.samples;
@@ -261,7 +262,7 @@ int pw_plan(ifs_ctx *c, PwLevel &P, int nrhs) {
     P.cpre_at.clear();
     P.n_g = P.n_f = P.n_u = P.n_t = 0;
     for (int j = 0; j < P.Q2;) {
-        PwLevel::Chunk ch{j, 0, 0, 0};
+        PwLevel::Chunk ch{j, 0, 0, 0, 0.0, 0.0};
         double bytes = 0.0;
         while (j + ch.R2 < P.Q2) {
             const int n = P.N[j + ch.R2];
@@ -271,6 +272,10 @@ int pw_plan(ifs_ctx *c, PwLevel &P, int nrhs) {
             bytes += b;
             ch.sn += 2 * n;
             ch.maxN = std::max(ch.maxN, n);
+            double gemm, fft;
+            pw_row_flops(L, P.mF[j + ch.R2], n, gemm, fft);
+            ch.f_gemm += gemm;
+            ch.f_fft += fft;
             ++ch.R2;
         }
         P.cpre_at.push_back((int64_t)cpre.size());
@@ -390,25 +395,26 @@ int pw_run(ifs_ctx *c, PwLevel &P, const double2 *C, double2 *D, int nrhs, int64
                 a.tsn = ch.sn;
                 tables(ch.j0, ch.R2, ch.maxN, true, true);
             }
+            const double nbr = (double)P.nb * nr;
             {
-                Scope sc(c, "m2l_synth");
+                Scope sc(c, "m2l_synth", ch.f_gemm * nbr);
                 launch_pw_synth(a, s);
             }
             {
-                Scope sc(c, "m2l_fft");
+                Scope sc(c, "m2l_fft", ch.f_fft * nbr);
                 launch_pw_fft(a, 0, ch.maxN, s);
             }
             {
-                Scope sc(c, "m2l_product");
+                Scope sc(c, "m2l_product", 16.0 * (double)ch.sn * (double)P.ncols * nr);
                 launch_pw_m2l(a, P.d_par.as<PwParent>(), (int)P.par.size(), P.d_src.as<PwSource>(), P.d_map.as<PwMaps>(),
                               P.nb, nr, ch.maxN, s);
             }
             {
-                Scope sc(c, "m2l_fft");
+                Scope sc(c, "m2l_fft", ch.f_fft * nbr);
                 launch_pw_fft(a, 1, ch.maxN, s);
             }
             {
-                Scope sc(c, "m2l_anal");
+                Scope sc(c, "m2l_anal", ch.f_gemm * nbr);
                 launch_pw_anal(a, i > 0, s);
             }
         }
@@ -420,13 +426,19 @@ int pw_run(ifs_ctx *c, PwLevel &P, const double2 *C, double2 *D, int nrhs, int64
     return hipPeekAtLastError() == hipSuccess ? IFS_OK : IFS_E_HIP;
 }
 
+void pw_row_flops(int L, int mF, int N, double &gemm, double &fft) {
+    gemm = 16.0 * (double)(pw_xcnt(mF, L) + pw_cn(mF, L) - pw_xcnt(-mF, L));
+    fft = 20.0 * N * std::log2((double)N);
+}
+
 double pw_flops(const PwLevel &P) {
-    double gemm = 0.0, fft = 0.0;
+    double box = 0.0;
     for (int j = 0; j < P.Q2; ++j) {
-        for (int m = -P.mF[j]; m <= P.mF[j]; ++m) gemm += 2.0 * 2.0 * 8.0 * pw_cn(m, P.L);
-        fft += 2.0 * 2.0 * 2.0 * 5.0 * P.N[j] * std::log2((double)P.N[j]);
+        double gemm, fft;
+        pw_row_flops(P.L, P.mF[j], P.N[j], gemm, fft);
+        box += 2.0 * (gemm + fft);
     }
-    return (gemm + fft) * P.nb + 16.0 * (double)P.SN * (double)P.ncols;
+    return box * P.nb + 16.0 * (double)P.SN * (double)P.ncols;
 }
 
 uint64_t pw_sig(const PwLevel &P) {

@@ -65,6 +65,7 @@ struct PwLevel {
         int j0, R2;           // nodes [j0, j0 + R2) and their mirrors
         int64_t sn;           // azimuths of the chunk's rows
         int maxN;
+        double f_gemm, f_fft; // algorithmic flops of one direction, per box (pw_row_flops)
     };
     std::vector<Chunk> chunks;
     DevBuf d_cpre;            // per chunk: prefix of N over its 2 R2 rows, chunk after chunk
@@ -112,6 +113,9 @@ PwSize pw_size(int L, int nbr, int Q2, double tdeg, int tcap, int order);
 // Algorithmic flops of one product: the two GEMMs (8 Q degrees^2 each way per box), the
 // azimuthal transforms (5 N log2 N), 16 per sample and translation.
 double pw_flops(const PwLevel &P);
+// One direction of one node and its mirror, per box: the products with U (complex by real, two
+// helicities), and the azimuthal transforms.
+void pw_row_flops(int L, int mF, int N, double &gemm, double &fft);
 uint64_t pw_sig(const PwLevel &P);
 
 // -- kernels --------------------------------------------------------------------

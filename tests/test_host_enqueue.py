@@ -326,3 +326,34 @@ print({n}, {ndir}, "live", live / 2 ** 20, "MiB, plan", (p["total"] - basis) / 2
 assert not made and live <= p["total"] - basis
 assert p["total"] - p["vectors"] <= 2.0 * live + (256 << 20)
 """)
+
+
+def test_profile_counts_the_flops_of_every_product(so):
+    """Each kernel group of an MLFMM product that multiplies reports its algorithmic flops, in proportion to
+    the right-hand sides and whatever the chunks; the sampled translations 16 flops per sample of the
+    grid and translation."""
+    host_runtime.run(so, """
+import numpy as np
+def flops(nrhs, **kw):
+    s = solver(*spheres(400, 160.0, 1, 9), use_fmm=True, leaf_size=32, **kw)
+    x = ctypes.create_string_buffer(64)
+    s.profile(True)
+    s.calculate_vector_b_batch_device(ctypes.addressof(x), ctypes.addressof(x), nrhs)
+    f = {k: v[2] for k, v in s.profile_read().items()}
+    (L,), m2l = s.fmm_stats()[1].values(), s.fmm_stats()[0]["M2L"]
+    total = s.matvec_cost()[0]
+    s.close()
+    return f, L, m2l, total
+f, L, m2l, total = flops(1)
+names = ["m2l_synth", "m2l_fft", "m2l_product", "m2l_anal", "p2m_samples", "p2m_box", "l2p_box", "l2p_samples",
+         "l2p_sum", "p2p_rot_fwd", "p2p_axial", "p2p_rot_back", "class_rot_fwd", "class_axial", "class_rot_back"]
+assert all(f[k] > 0.0 for k in names), f
+samples = f["m2l_product"] / (16.0 * m2l)  # few offsets are class products as a whole
+assert 2 * (L + 1) * L < samples < 2 * (L + 1) * (4 * L + 100), (samples, L)
+assert f["m2l_synth"] == f["m2l_anal"] and f["m2l_synth"] + f["m2l_fft"] + f["m2l_anal"] + f["m2l_product"] < total
+for kw in ({}, dict(workspace_mb=64)):
+    g = flops(3, **kw)[0]
+    for k in names:
+        if not (kw and k.startswith("l2p_box")):  # boxes are sampled again for each group of spheres
+            assert abs(g[k] - 3.0 * f[k]) < 1e-12 * g[k], (k, kw, f[k], g[k])
+""")
