@@ -822,6 +822,7 @@ int class_batch_run(ifs_ctx *c, ClassBatch &B, const double2 *src_pool, double2 
     };
     const char *pn_fwd = prec == 1 ? "class_rot_fwd_f32" : "class_rot_fwd";
     const char *pn_ax = prec == 1 ? "class_axial_f32" : "class_axial";
+    if (rem_by_threads(T0.Lt, B.n0)) pn_ax = prec == 1 ? "class_axial_rem_f32" : "class_axial_rem";
     const char *pn_back = prec == 1 ? "class_rot_back_f32" : "class_rot_back";
     // Rotation block heights (64 or 32 rows of each folded product).  64 halves the
     // column-panel re-reads; 32 wastes less padding where the degrees hold few rows

@@ -646,7 +646,7 @@ __global__ __launch_bounds__(256) void k_class_axial(const GroupDesc *__restrict
 // the scalar loads of P and Q.  Box translations of 2500 spheres (24 and 9 last degrees of 97):
 // 1302 -> 768 us, of 3000 small-order spheres (1 to 23 of 45): 1100 -> 508 us.  With 41 and
 // 50 degrees the 64-row blocks are the faster (474 against 591 us).
-constexpr int kRemDegrees = 32, RR = 8;
+constexpr int RR = 8;
 template <typename TC>
 __global__ __launch_bounds__(256) void k_class_axial_rem(const GroupDesc *__restrict__ desc,
                                                          const double2 *__restrict__ wax, const TC *__restrict__ wy,
@@ -738,7 +738,7 @@ static void launch_class_t(const GroupDesc &h, const GroupDesc *d_desc, const in
         else
             hipLaunchKernelGGL((k_class_rot_fwd<TC, TW, FMF, 3>), grid, dim3(256), 0, s, d_desc, src_off, pidx, phase,
                                src_pool, wd, wy);
-    } else if (stage == 1 && h.n0 > 1 && h.Lt - h.n0 < kRemDegrees) {
+    } else if (stage == 1 && rem_by_threads(h.Lt, h.n0)) {
         hipLaunchKernelGGL(k_class_axial_rem<TC>,
                            dim3((h.ncols * h.nrhs + 255) / 256, (h.Lt - h.n0 + RR) / RR, 2 * K + 1), dim3(256), 0, s,
                            d_desc, wax, (const TC *)wy, wz);

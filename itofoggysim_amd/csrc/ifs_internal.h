@@ -144,6 +144,9 @@ __host__ __device__ inline int64_t ax0_off(int k, int L, int n0) {
     if (k <= n0) return neg + (int64_t)(k - 1 + n0) * b;
     return neg + (int64_t)(2 * n0) * b + 2 * ax_sum(n0 + 1, k - 1, L, L);
 }
+// Whether the coaxial shift of degrees n0..Lt is a thread per translation (figures at the kernel).
+constexpr int kRemDegrees = 32;
+inline bool rem_by_threads(int Lt, int n0) { return n0 > 1 && Lt - n0 < kRemDegrees; }
 __host__ __device__ inline int64_t ax0_size(int L, int n0) { return ax0_off(L, L, n0) + 2 * ax0_block(L, L, n0); }
 __host__ __device__ inline int64_t sect_size(int K, int nmax) { return (int64_t)(K + 1) * (nmax + 2); }
 

@@ -53,7 +53,7 @@ struct PairBatch {
         int t0 = 0, t1 = 0, s0 = 0, s1 = 0, g0 = 0, g1 = 0, c0 = 0, c1 = 0;  // tiles, segments, targets, close tasks
         int a0 = 0, a1 = 0, waves = 4;  // groups, tiles of a group
         int64_t n_y = 0, n_z = 0, n_w = 0, n_tab = 0, n_ax = 0, n_s = 0;
-        int max_Ls = 0, max_Lt = 0, max_K = 0, maxK_close = 0, max_nmax = 0, max_tabw = 0, max_P = 0;
+        int max_Ls = 0, max_Lt = 0, max_K = 0, maxK_close = 0, max_nmax = 0, max_P = 0;
         double f_fwd = 0.0, f_ax = 0.0, f_back = 0.0;
     };
     std::vector<PairTile> tiles;
@@ -76,7 +76,6 @@ struct PairBatch {
     WsNeed ws;                // tables that are not kept
     int NL = 0;               // orders of the shared matrices
     std::vector<Task> tasks;  // the translations, sorted by target
-    double cost_flops = 0.0, cost_bytes = 0.0;
     const char *pn[4] = {"gen_tables", "rot_fwd", "axial_apply", "rot_back"};
     bool active() const { return !tasks.empty(); }
 };

@@ -289,8 +289,11 @@ lmax = rng.integers(1, 5, 260).astype(np.int32)
 s = solver(pos, lmax, use_fmm=True, leaf_size=32, fmm_d0={d0})
 x, b = (ctypes.create_string_buffer(16 * s.n) for _ in range(2))
 fake.calls()
+s.profile(True)
 s.calculate_vector_b_device(ctypes.addressof(x), ctypes.addressof(b))
 seen = fake.calls()
+ran = s.profile_read()  # one level, no whole offset: only 33 degrees run as class products by blocks
+assert "class_axial_rem" in ran and ("class_axial" in ran) == {blocks}
 assert launches(seen, "k_class_axial_remI") and launches(seen, "k_pw_m2l")
 assert bool(launches(seen, "k_class_axialI")) == {blocks}, [c[1] for c in launches(seen, "k_class")]
 """)
@@ -346,7 +349,8 @@ def flops(nrhs, **kw):
     return f, L, m2l, total
 f, L, m2l, total = flops(1)
 names = ["m2l_synth", "m2l_fft", "m2l_product", "m2l_anal", "p2m_samples", "p2m_box", "l2p_box", "l2p_samples",
-         "l2p_sum", "p2p_rot_fwd", "p2p_axial", "p2p_rot_back", "class_rot_fwd", "class_axial", "class_rot_back"]
+         "l2p_sum", "p2p_rot_fwd", "p2p_axial", "p2p_rot_back", "class_rot_fwd", "class_axial", "class_axial_rem",
+         "class_rot_back"]
 assert all(f[k] > 0.0 for k in names), f
 samples = f["m2l_product"] / (16.0 * m2l)  # few offsets are class products as a whole
 assert 2 * (L + 1) * L < samples < 2 * (L + 1) * (4 * L + 100), (samples, L)
