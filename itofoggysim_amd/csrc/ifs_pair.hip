@@ -23,11 +23,12 @@
 // t/2-growth allows (PairTile::Q = 0, rule in ifs_pair.cpp) take coaxial tables from
 // the degree recurrence instead; their rotations run here all the same.
 //
-// Bound by the matrix cores and their operand reads from L1/L2 (tiles are 50-75% full at
-// orders 10 to 25).  Against per-pair tables: 22650 pairs of orders 9-18 (151 spheres at
-// 800 nm) 3.57 -> 0.53 ms per product, the near field of 2500 spheres at 550 nm (248818
-// pairs, orders 9-23) 40.1 -> 8.8 ms, with four right-hand sides (114758 pairs) 81.9 ->
-// 15.3 ms; error against 64-bit sums unchanged (3e-13, 1.1e-13).
+// Bound by the latency of operand loads: the matrix cores are busy 28 to 35% of the time, with
+// 3.4 to 6.2 waves resident on a SIMD that wait 33 to 63% of theirs (tiles are 50-75% full at orders
+// 10 to 25).  Against per-pair tables: 22650 pairs of orders 10-18 (151 spheres at
+// 800 nm) 3.57 -> 0.47 ms per product, the near field of 2500 spheres at 550 nm (248818
+// pairs, orders 9-23) 40.1 -> 7.3 ms, with four right-hand sides (114758 pairs) 81.9 ->
+// 13.0 ms; error against 64-bit sums unchanged (3e-13, 1.1e-13).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -397,7 +398,7 @@ __global__ __launch_bounds__(256) void k_pair_fwd(const PairTile *__restrict__ t
 // P_m, z_+(-m) and z_-(m) take Q_m, so each of the two products has 16 columns.  The tiles
 // of a block share one node set: its matrices pass through LDS one node tile at a time (read
 // per wave from L1 they took 8 cache accesses per 64-cycle product and bounded the kernel:
-// 5740 tiles of orders 9-18 in 343 us; through LDS, rows read whole, 238 us).  A wave fetches
+// 5740 tiles of orders 10-18 in 343 us; through LDS, rows read whole, 238 us).  A wave fetches
 // its rows of the next node tile while the block works on this one, and a block's tiles have
 // similar orders (few waves without work at high m): 48 clusters 588 -> 522 us, 5740 tiles 234.
 // Node-set matrices at off_q: for [m][P, Q]: A1[Q/16][S1][64] (rows

@@ -17,12 +17,12 @@
 // Launches per chunk of rows: GEMM (X -> G, orders x rows x boxes), FFT along the
 // azimuth in LDS (G -> F), products (F -> H), FFT back (H -> G), GEMM (G -> Xd).
 //
-// Bound by the products' reads of T (16 bytes per 16 flops, from L1/L2) and by the
-// transforms' passes over G and F.  M2L against class products of rotations and shifts:
+// Bound by the products' reads of T and of samples (16 bytes of T per 16 flops, 16 TB/s from
+// L2) and by the transforms' passes over G and F.  M2L against class products of rotations and shifts:
 // 64 boxes of order 410 (3004 translations) 120 -> 16.5 ms, 512 + 64 boxes of orders 97
 // and 174 (56046) 64 -> 17 ms, orders 45 and 77 (56448) 13.7 -> 5.7 ms (with what the class
 // products keep of near offsets).  Against the direct product of 200 / 600 spheres the
-// MLFMM is off by 1.2e-13 / 3.0e-13 (class products 3.7e-10 / 5.7e-9).
+// MLFMM is off by 4.4e-14 / 1.0e-13 (class products 3.7e-10 / 5.7e-9).
 #include <hip/hip_runtime.h>
 #include <math.h>
 
@@ -364,8 +364,8 @@ __device__ __forceinline__ int div_small(int a, float inv) { return (int)(((floa
 // Azimuthal transforms of NB boxes of one (row, helicity), in place in LDS: decimation in
 // frequency with radices 2, 3, 4, 5 (natural order in, digit-reversed out).  Forward: orders
 // -mF..mF of G to azimuths, e^{+i m phi}; inverse: azimuths to orders, e^{-i m phi}.
-// Bound by LDS passes and barriers (64 boxes of order 410: 2.75 GB of samples, 1.09 ms a
-// direction, 0.95 at the copy rate).  Index divisions go through FP32 and the radices are read
+// Bound by LDS passes, barriers and short pieces of G (waves wait 70% of the time; 64 boxes of order
+// 410: 1.09 ms a direction).  Index divisions go through FP32 and the radices are read
 // from memory: as integer divisions and a local copy in scratch they took 1.60 ms.
 template <bool INV>
 __global__ __launch_bounds__(512) void k_pw_fft(PwArg a, int NBmax) {
@@ -471,13 +471,15 @@ __global__ __launch_bounds__(512) void k_pw_fft(PwArg a, int NBmax) {
 // children's sums of both helicities in registers; a source's samples are read once per
 // parent, the tables by neighbouring waves of the same azimuths from one L2 (mixed precision
 // reads them rounded to FP32, half of the bytes; samples and sums stay FP64).
-// Bound by the tables' reads: 16 bytes per 16 flops, through L1 from L2.  The loads of a
+// Bound by the reads of tables and samples, through L1 from L2 (16 bytes of table per 16 flops): 16.4
+// TB/s of L2 reads at orders 97 and 174, 16.1 at order 410, where HBM delivers 6.3 of them (25 GB
+// a launch for 2.1 GB of samples and 0.6 GB of tables: the dies fetch both several times).  The loads of a
 // source and all eight children are in flight while the previous source's products run, also
 // for children that the source does not reach (they read some entry of the first table): with
 // a branch around each load every product waited for its own load.  56046 translations of
 // orders 97 and 174: 9.5 ms with loads behind branches, 7.2 with a source's loads first and
 // the next source's beside the products, 5.2 as here with 32-bit offsets from scalar row
-// addresses (12 TB/s of tables).
+// addresses.
 template <typename TT>
 __global__ __launch_bounds__(256) void k_pw_m2l(const TT *__restrict__ T, PwArg a, const PwParent *__restrict__ par, int npar,
                                                 const PwSource *__restrict__ src, const PwMaps *__restrict__ map,
