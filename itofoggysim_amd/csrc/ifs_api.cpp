@@ -113,6 +113,12 @@ int ws_reserve(ifs_ctx *c, const WsNeed &need) {
     return IFS_OK;
 }
 
+bool capturing(const ifs_ctx *c) {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    (void)hipStreamIsCapturing(c->stream, &s);
+    return s != hipStreamCaptureStatusNone;
+}
+
 // Split a target-sorted task list into segments and workspace chunks and upload it.
 // The tables are kept across matvecs when they fit the context's cache budget.
 int batch_finalize(ifs_ctx *c, Batch &B, size_t budget_bytes, bool allow_cache) {
@@ -348,7 +354,7 @@ int batch_run(ifs_ctx *c, Batch &B, const double2 *src_pool, double2 *dst_pool, 
         }
         if (hipPeekAtLastError() != hipSuccess) return IFS_E_HIP;
     }
-    if (B.cached) B.tables_ready = true;
+    if (B.cached && !B.tables_ready) B.tables_ready = !capturing(c);
     return IFS_OK;
 }
 
@@ -787,11 +793,12 @@ int class_batch_run(ifs_ctx *c, ClassBatch &B, const double2 *src_pool, double2 
     const int ftab = prec == 1 && !B.d_persist ? 1 : 0;
     int cur_ax = -1;                                        // coaxial key in the shared workspace
     std::vector<int> owner(std::max(B.n_dslots, 1), -1);    // Wigner key in each shared slot
+    std::vector<char> made_d(B.dkeys.size(), 0), made_ax(B.axkey_cls.size(), 0);  // kept tables made in this call
     auto need_d = [&](const ClassBatch::Piece &P) {
         const int key = B.dkey[P.gen];
         if (B.d_persist) {
-            if (B.d_ready[key]) return;
-            B.d_ready[key] = 1;
+            if (B.d_ready[key] || made_d[key]) return;
+            made_d[key] = 1;
         } else {
             int slot = (int)(P.g.off_d / std::max<int64_t>(B.n_d, 1));
             if (owner[slot] == key) return;
@@ -808,8 +815,8 @@ int class_batch_run(ifs_ctx *c, ClassBatch &B, const double2 *src_pool, double2 
     auto need_ax = [&](const ClassBatch::Piece &P) {
         const int key = B.axkey[P.gen];
         if (B.ax_persist) {
-            if (B.ax_ready[key]) return;
-            B.ax_ready[key] = 1;
+            if (B.ax_ready[key] || made_ax[key]) return;
+            made_ax[key] = 1;
         } else {
             if (cur_ax == key) return;
             cur_ax = key;
@@ -831,9 +838,8 @@ int class_batch_run(ifs_ctx *c, ClassBatch &B, const double2 *src_pool, double2 
     // product, and remembers the choice per shape for later contexts.
     int rows[2];
     bool tune[2] = {false, false};
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    (void)hipStreamIsCapturing(c->stream, &cap);
-    const bool can_tune = c->autotune && !c->prof.on && cap == hipStreamCaptureStatusNone;
+    const bool recorded = capturing(c);
+    const bool can_tune = c->autotune && !c->prof.on && !recorded;
     const std::array<int, 7> tkey = {T0.Ls, T0.Lt, T0.K, B.n0, prec, nrhs, ilog2((int64_t)B.src.size())};
     for (int st = 0; st < 2; ++st) {
         int r = c->force_rows[st] ? c->force_rows[st] : B.rot_rows[prec & 1][st];
@@ -890,6 +896,12 @@ int class_batch_run(ifs_ctx *c, ClassBatch &B, const double2 *src_pool, double2 
         }
     }
     if (hipPeekAtLastError() != hipSuccess) return IFS_E_HIP;
+    if (!recorded) {
+        for (size_t k = 0; k < made_d.size(); ++k)
+            if (made_d[k]) B.d_ready[k] = 1;
+        for (size_t k = 0; k < made_ax.size(); ++k)
+            if (made_ax[k]) B.ax_ready[k] = 1;
+    }
     for (int st = 0; st < 2; ++st) {
         if (!tune[st]) continue;
         double t64 = 0.0, t32 = 0.0;

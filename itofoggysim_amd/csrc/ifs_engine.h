@@ -189,6 +189,9 @@ namespace ifs {
 // addresses.  One that cannot grow gets its old size back for the plans that fit it, and
 // where even that fails the next run that needs it asks again.
 int ws_reserve(ifs_ctx *c, const WsNeed &need);
+// Whether the context's stream is being captured: what is enqueued then has not run when the call
+// returns, so kept tables stay to be made by a product that does run.
+bool capturing(const ifs_ctx *c);
 // Device address of the far-field scratch array on the current device (looked up
 // once per device); ifs_create calls it with the context's device current.
 int far_field_scratch(int device, void **out);

@@ -64,7 +64,7 @@ void box_matrices(ifs_ctx *c, Leaf &F, LeafArg &a, const PwLevel::Chunk &ch, siz
         if (!P.ready) {
             Scope s(c, "leaf_gen_tables");
             launch_pw_utable(P.L, P.Q2, 0, P.Q2, 0, P.Q2, a.p.ustr, a.mu, U, c->stream);
-            P.ready = true;
+            P.ready = !capturing(c);
         }
         a.p.a0 = ch.j0;
         a.p.a1 = P.Q2 + ch.j0;

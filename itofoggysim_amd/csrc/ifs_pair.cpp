@@ -429,7 +429,7 @@ int pair_run(ifs_ctx *c, PairBatch &B, const double2 *src_pool, double2 *dst_poo
         }
     }
     if (hipPeekAtLastError() != hipSuccess) return IFS_E_HIP;
-    if (B.kept) B.ready = true;
+    if (B.kept && !B.ready) B.ready = !capturing(c);
     return IFS_OK;
 }
 

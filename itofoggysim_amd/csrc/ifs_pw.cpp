@@ -324,9 +324,7 @@ PwArg pw_arg(ifs_ctx *c, const PwLevel &P, int nrhs) {
 
 int pw_prepare(ifs_ctx *c, PwLevel &P, int nrhs, int prec) {
     if (prec == 1 && P.kept && !P.own_T32.p && !P.no_t32) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        (void)hipStreamIsCapturing(c->stream, &cap);
-        if (cap == hipStreamCaptureStatusNone) {
+        if (!capturing(c)) {
             const size_t b = 8 * P.canon.size() * (size_t)P.SN;
             P.no_t32 = b + c->ws_cached > c->cache_budget || P.own_T32.alloc(b) != IFS_OK;
             if (!P.no_t32) c->ws_cached += b;
@@ -372,7 +370,7 @@ int pw_run(ifs_ctx *c, PwLevel &P, const double2 *C, double2 *D, int nrhs, int64
                 a.a0 = 0;
                 a.a1 = P.Q2;
                 tables(0, P.Q2, *std::max_element(P.N.begin(), P.N.end()), !P.ready, !P.t_ready[t]);
-                P.ready = P.t_ready[t] = true;
+                if (!capturing(c)) P.ready = P.t_ready[t] = true;
             }
         }
         {

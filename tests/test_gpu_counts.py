@@ -4,7 +4,8 @@
     direct plans of the pair kernels, a direct plan whose largest sphere (order 66) is beyond
     them, and an MLFMM whose workspace holds two right-hand sides at once, so that three run in
     groups of two and one;
-  * the first product of a context on a caller's own stream.
+  * the first product of a context on a caller's own stream;
+  * a context's first product inside a caller's capture, then an eager one, then the captured one.
 
 A replay runs the captured launches on the same buffers: equal bits.  Direct batched products
 take the same sums per right-hand side: equal bits.  In the MLFMM the number of right-hand sides
@@ -100,3 +101,38 @@ def test_first_product_on_a_stream_set_after_creation(name):
     hip.free_all()
     assert hip.rt.hipStreamDestroy(stream) == 0
     assert np.array_equal(out[0], out[1]) and np.isfinite(out[0]).all()
+
+
+@pytest.mark.parametrize("name", ["direct", "order 66", "MLFMM"])
+def test_first_product_in_a_callers_capture(name):
+    hip = Hip()
+    rt, stream = hip.rt, ctypes.c_void_p()
+    assert rt.hipStreamCreateWithFlags(ctypes.byref(stream), 1) == 0
+    _, lmax, s = _make(name)
+    S, mask = snm_flat(s.n_global, lmax)
+    rng = np.random.default_rng(10)
+    v = (rng.standard_normal(s.n) + 1j * rng.standard_normal(s.n)) * mask / S
+    s.set_class_tiles(64, 64, False)
+    want = s.calculate_vector_b(v)
+    s.close()
+    _, _, s = _make(name)
+    s.set_class_tiles(64, 64, False)
+    s.set_stream(stream.value)
+    x, b, g = hip.upload(v), hip.upload(np.zeros_like(v)), hip.upload(np.zeros_like(v))
+    graph, run = ctypes.c_void_p(), ctypes.c_void_p()
+    assert rt.hipStreamBeginCapture(stream, 1) == 0
+    s.calculate_vector_b_device(x.value, g.value)
+    assert rt.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    s.calculate_vector_b_device(x.value, b.value)
+    hip.sync(stream)
+    assert np.array_equal(hip.download(b, v), want)
+    assert rt.hipGraphInstantiate(ctypes.byref(run), graph, None, None, 0) == 0
+    for _ in range(2):
+        assert rt.hipGraphLaunch(run, stream) == 0
+        s.calculate_vector_b_device(x.value, b.value)
+        hip.sync(stream)
+        assert np.array_equal(hip.download(g, v), want) and np.array_equal(hip.download(b, v), want)
+    rt.hipGraphExecDestroy(run), rt.hipGraphDestroy(graph)
+    s.close()
+    hip.free_all()
+    assert rt.hipStreamDestroy(stream) == 0

@@ -361,3 +361,28 @@ for kw in ({}, dict(workspace_mb=64)):
         if not (kw and k.startswith("l2p_box")):  # boxes are sampled again for each group of spheres
             assert abs(g[k] - 3.0 * f[k]) < 1e-12 * g[k], (k, kw, f[k], g[k])
 """)
+
+
+@pytest.mark.parametrize("args", ["12, 40.0, 1, 9", "400, 160.0, 1, 9, use_fmm=True, leaf_size=32",
+                                  "400, 160.0, 1, 9, use_fmm=True, leaf_size=32, workspace_mb=4",
+                                  "3, 200.0, 60, 66"])
+def test_tables_of_a_captured_first_product_stay_to_be_made(so, args):
+    """A caller's capture may hold a context's first product: its table kernels are recorded, not run, so an
+    eager product beside the graph makes the tables itself; those after it find them."""
+    n, side, lo, hi, *kw = args.split(", ")
+    host_runtime.run(so, f"""
+s = solver(*spheres({n}, {side}, {lo}, {hi}), {", ".join(kw)})
+x = ctypes.create_string_buffer(64)
+stream, graph = ctypes.c_void_p(), ctypes.c_void_p()
+fake.hipStreamCreate(ctypes.byref(stream))
+s.set_stream(stream.value)
+def tables():
+    fake.calls()
+    s.calculate_vector_b_device(ctypes.addressof(x), ctypes.addressof(x))
+    return [c[1] for c in launches(fake.calls()) if any(t in c[1] for t in ("table", "k_gen", "k_gq"))]
+assert fake.hipStreamBeginCapture(stream, 1) == 0
+captured = tables()
+assert fake.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+assert captured and set(tables()) == set(captured)
+assert not tables()
+""")
