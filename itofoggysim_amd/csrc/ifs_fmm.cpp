@@ -394,7 +394,8 @@ int build(ifs_ctx *c, Fmm **out) {
         }
         if ((rc = class_batches_prepare(c, cls))) goto fail;
     }
-    if (!f->l2p.tasks.empty() && leaf_worth(c->ws_budget, leaf_reach(f->p2m.tasks, f->l2p.tasks), LL.L, (int)LL.boxes.size(), ns)) {
+    if (!f->l2p.tasks.empty() &&
+        leaf_worth(c->ws_budget, leaf_reach(f->p2m.tasks, f->l2p.tasks), LL.L, (int)LL.boxes.size(), ns)) {
         batch_cost(f->p2m, c->flops_mv, c->bytes_mv);
         batch_cost(f->l2p, c->flops_mv, c->bytes_mv);
         if ((rc = leaf_build(c, f->leaf, f->p2m.tasks, f->l2p.tasks, LL.L, (int)LL.boxes.size(), LL.off))) goto fail;

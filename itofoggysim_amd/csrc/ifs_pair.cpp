@@ -435,8 +435,8 @@ int pair_run(ifs_ctx *c, PairBatch &B, const double2 *src_pool, double2 *dst_poo
 
 uint64_t pair_sig(const PairBatch &B) {
     uint64_t h = 0;
-    for (const DevBuf *d : {&B.d_tiles, &B.d_slots, &B.d_segs, &B.d_targets, &B.d_parts, &B.d_close, &B.d_groups, &B.d_order, &B.d_delta, &B.d_quad,
-                            &B.own_tab, &B.own_ax})
+    for (const DevBuf *d : {&B.d_tiles, &B.d_slots, &B.d_segs, &B.d_targets, &B.d_parts, &B.d_close, &B.d_groups,
+                            &B.d_order, &B.d_delta, &B.d_quad, &B.own_tab, &B.own_ax})
         h ^= (uint64_t)(uintptr_t)d->p + 0x9e3779b97f4a7c15ull + (h << 6) + (h >> 2);
     return h;
 }

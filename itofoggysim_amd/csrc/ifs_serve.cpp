@@ -248,7 +248,8 @@ void need_tree(const Req &r, const std::vector<int> &L, size_t ws_cap, Plan &P, 
         }
         if (whole > 0.0) {
             need_class(Lb, Lb, 1, whole, (double)ax.size(), (double)d.size(), nd, N);
-            N.gen = std::max(N.gen, generator(outgoing ? IFS_ZSEL_HANKEL1 : IFS_ZSEL_BESSEL_J, k * edge * std::sqrt((double)*ax.rbegin()), Lb, Lb));
+            N.gen = std::max(N.gen, generator(outgoing ? IFS_ZSEL_HANKEL1 : IFS_ZSEL_BESSEL_J,
+                                              k * edge * std::sqrt((double)*ax.rbegin()), Lb, Lb));
         }
         if (l < lmax) continue;
         // spheres and their leaf boxes
